@@ -2,12 +2,12 @@
 // (crates/core/src/models/cfm.rs), the itts_cfm_* entry points of include/itts_hip.h.
 //
 // CfmDit::from_weights -> itts_cfm_create (tensors by checkpoint name, checked by element
-// count), forward_merged -> itts_cfm_forward, solve_euler -> itts_cfm_solve_euler.  The
-// estimator keeps fp32 activations: its linears (and WaveNet's kernel-5 convolution, as one
-// GEMM over a zero-padded buffer whose operand rows overlap) run on the split-fp16 MFMA GEMM
-// of kernels_cfm.hip on the estimator's stream, products under 64 rows on its few-row fp32
-// product; the other kernels in kernels_cfm.hip do the rest.  Layout: activations [B][T][C] row-major, the CFG
-// pair as batch rows 0 (conditioned) and 1 (unconditioned).
+// count), forward_merged -> itts_cfm_forward, solve_euler -> itts_cfm_solve_euler.  Forwards of
+// 64 rows and more keep the residual stream in fp32 and hand every product its operands as
+// fp16 hi/lo planes in MFMA fragment order (kernels_cfm_mm.hip); smaller ones, and operands
+// whose widths are not multiples of 4, run the linears as fp32 FMA products
+// (kernels_cfm.hip).  Layout: activations [B][T][C] row-major, the CFG pair as batch rows 0
+// (conditioned) and 1 (unconditioned).
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -16,7 +16,7 @@
 #include <cstring>
 #include <map>
 #include <string>
-#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/itts_hip.h"
@@ -71,9 +71,6 @@ struct Buf {
   }
 };
 
-hipError_t gemm(itts_cfm *m, int M, int N, int K, const float *A, int lda, const float *W, int ldw, float *y,
-                int ldy, float beta, const float *bias = nullptr, const float *yr = nullptr);
-
 struct Block {
   const float *wqkv, *wo, *w13, *w2, *skip_w, *skip_b, *an_w, *fn_w;
 };
@@ -95,19 +92,23 @@ struct itts_cfm {
   std::vector<WnLayer> wn;
   // per-forward workspace (sized for R = B*T rows)
   Buf emb, th, t1, t2, st, mods, wng, fmod, tdev;
-  Buf hA, hB, n, qkv, att, gu, act, xres, hpad, acts, rs, oacc, v, rope, apo, aml, kvs;
-  int rope_T = 0;  // sequence length the rope table holds
-  int n_cu = 0;    // compute units of the device (the attention's split planner)
-  std::vector<Buf> skips;
+  Buf hA, hB, n, qkv, att, gu, act, xres, hw, acts, rs, oacc, v, rope;
+  // fragment planes (16-byte pieces): norm / attention / FFN outputs, the block output a
+  // long skip joins, the skips, merged and x_t inputs, x_res, WaveNet's padded input, Q, K / V
+  Buf nP, attP, actP, curP, mP, xtP, xresP, hpP, qF, kvF;
+  std::vector<Buf> skipP, skips;
+  int rope_T = 0;           // sequence length the rope table holds
+  int hp_B = 0, hp_T = 0;   // shape whose padding rows hpP holds as zeros
+  int n_cu = 0;             // compute units of the device (the launch rules' parameter)
   // solve / API staging
   Buf x, xt, merged, catc, refm, sty, io_a, io_b;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   float last_ms = -1.0f;
-  // the weights' fp16 hi/lo quads for the MFMA GEMM, split on first use: (W, ldw, N, K,
-  // interleave) -> cfm_split_weights output
-  std::map<std::tuple<const float *, int, int, int, int>, uint4 *> wsplit;
+  // the weights' fragment planes, laid out at their first use, by (first row, halves
+  // interleaved)
+  std::map<std::pair<const float *, int>, uint4 *> wfrag;
   ~itts_cfm() {
-    for (auto &kv : wsplit) (void)hipFree(kv.second);
+    for (auto &kv : wfrag) (void)hipFree(kv.second);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (arena) (void)hipFree(arena);
@@ -117,36 +118,51 @@ struct itts_cfm {
 
 namespace {
 
-// The split quads of the weight view (W, ldw, N, K; rows interleaved when ilv > 0), made on
-// the estimator's stream at its first use (the weights are constant while the estimator
-// lives); nullptr on failure.
-uint4 *split_weights(itts_cfm *m, const float *W, int ldw, int N, int K, int ilv = 0) {
-  const auto key = std::make_tuple(W, ldw, N, K, ilv);
-  auto it = m->wsplit.find(key);
-  if (it != m->wsplit.end()) return it->second;
+constexpr int kMfmaRows = 64;  // forwards of fewer rows run their linears as fp32 FMA products
+
+int steps16(int K) { return (K + 15) / 16; }
+int round32(int n) { return (n + 31) / 32 * 32; }
+uint4 *pieces(const Buf &b) { return reinterpret_cast<uint4 *>(b.p); }
+size_t piece_floats(size_t n) { return 4 * n; }
+
+// The fragment planes of weight W [N][ldw] (K values, plus K2 more at W + off2 as further K
+// steps; halves interleaved when ilv > 0), made on the estimator's stream at their first use
+// (the weights are constant while the estimator lives); nullptr on failure.
+const uint4 *weight_frag(itts_cfm *m, const float *W, int ldw, int N, int K, int ilv = 0, int off2 = 0, int K2 = 0) {
+  const auto key = std::make_pair(W, ilv);
+  auto it = m->wfrag.find(key);
+  if (it != m->wfrag.end()) return it->second;
+  const int nk = steps16(K) + (K2 ? steps16(K2) : 0);
+  const size_t bytes = cfm_frag_pieces(ilv ? 64L * ((ilv + 31) / 32) : N, nk) * sizeof(uint4);
   uint4 *p = nullptr;
-  if (hipMalloc(&p, itts::cfm_split_weights_quads(N, K) * sizeof(uint4)) != hipSuccess) return nullptr;
-  if (itts::cfm_split_weights(W, ldw, N, K, p, m->s, ilv) != hipSuccess) {
+  if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
+  if (hipMemsetAsync(p, 0, bytes, m->s) != hipSuccess ||
+      cfm_weight_frag(W, ldw, N, K, 0, nk, ilv, p, m->s) != hipSuccess ||
+      (K2 && cfm_weight_frag(W + off2, ldw, N, K2, steps16(K), nk, ilv, p, m->s) != hipSuccess)) {
     (void)hipFree(p);
     return nullptr;
   }
-  m->wsplit.emplace(key, p);
+  m->wfrag.emplace(key, p);
   return p;
 }
 
-// y[M][N] = A[M][K] W[N][K]^T (+ bias[n]) + beta y (row-major; W rows ldw apart) on the
-// estimator's stream: row blocks of 64 and more on the split-fp16 MFMA GEMM over the weight's split
-// quads, fewer rows (the per-batch timestep, AdaLN and WaveNet-conditioning projections,
-// forwards of under 64 frames) and operands the MFMA GEMM cannot take on the few-row fp32
-// product.
+// y[M][N] = A[M][K] W[N][K]^T (+ bias[n]) + beta y (row-major; W rows ldw apart) in fp32 FMAs
+// on the estimator's stream: the per-batch timestep, AdaLN and WaveNet-conditioning
+// projections, forwards of under kMfmaRows rows, and widths that are not multiples of 4.
 hipError_t gemm(itts_cfm *m, int M, int N, int K, const float *A, int lda, const float *W, int ldw, float *y,
-                int ldy, float beta, const float *bias, const float *yr) {
-  if (M >= 64 && itts::cfm_gemm_fits(A, lda, W, ldw, K)) {
-    const uint4 *wp = split_weights(m, W, ldw, N, K);
-    if (!wp) return hipErrorOutOfMemory;
-    return itts::cfm_gemm_split_w(1, M, N, K, A, lda, 0, wp, y, ldy, 0, beta, m->s, bias, yr);
-  }
-  return itts::cfm_rows_gemm(1, M, N, K, A, lda, 0, W, ldw, 0, y, ldy, 0, beta, m->s, bias, yr);
+                int ldy, float beta, const float *bias = nullptr) {
+  return itts::cfm_rows_gemm(1, M, N, K, A, lda, 0, W, ldw, 0, y, ldy, 0, beta, m->s, bias);
+}
+
+// A product over fragment planes: M rows of `a` (K values, ka K steps) by the planes w.
+CfmMm mm_args(const uint4 *a, int K, const uint4 *w, int M, int N) {
+  CfmMm g{};
+  g.a = a;
+  g.kt_a = g.nk = steps16(K);
+  g.w = w;
+  g.M = M;
+  g.N = N;
+  return g;
 }
 
 itts_status check_config(const itts_cfm_config &c) {
@@ -156,9 +172,17 @@ itts_status check_config(const itts_cfm_config &c) {
   return ITTS_OK;
 }
 
+// Pieces of one batch entry of WaveNet's padded input: the rows whole tiles of T read at every tap.
+size_t hp_pieces(const itts_cfm_config &c, int T) {
+  return cfm_frag_pieces((T + 127) / 128 * 128 + c.wn_kernel, c.dim / 16);
+}
+// The skip / merge products whose fp32 rows are not 16-byte aligned stay fp32 FMA products.
+bool unaligned_skip(const itts_cfm_config &c) { return c.in_ch % 4 != 0 || (c.dim + c.in_ch) % 4 != 0; }
+bool unaligned_merge(const itts_cfm_config &c) { return (2 * c.in_ch + c.dim + c.style_dim) % 4 != 0; }
+
 itts_status ensure_rows(itts_cfm *m, int B, int T) {
   const itts_cfm_config &c = m->c;
-  const size_t R = (size_t)B * T, d = c.dim, F = c.inter, NL = c.wn_layers, pad = c.wn_kernel / 2;
+  const size_t R = (size_t)B * T, d = c.dim, F = c.inter, NL = c.wn_layers;
   const size_t na = 2 * (size_t)c.n_layers + 1;
   CK(m->emb.ensure(B * kFreqDim));
   CK(m->th.ensure(B * d));
@@ -171,23 +195,41 @@ itts_status ensure_rows(itts_cfm *m, int B, int T) {
   CK(m->tdev.ensure(B));
   CK(m->hA.ensure(R * d));
   CK(m->hB.ensure(R * d));
-  CK(m->n.ensure(R * d));
-  CK(m->qkv.ensure(R * 3 * d));
-  CK(m->att.ensure(R * d));
-  CK(m->gu.ensure(R * 2 * F));
-  CK(m->act.ensure(R * (F > d ? F : d)));
-  CK(m->xres.ensure(R * d));
-  CK(m->hpad.ensure((size_t)B * (T + 2 * pad) * d));
-  CK(m->acts.ensure(R * 2 * d));
-  CK(m->rs.ensure(R * 2 * d));
+  CK(m->hw.ensure(R * d));
   CK(m->oacc.ensure(R * d));
   CK(m->v.ensure(R * c.in_ch));
-  for (auto &b : m->skips) CK(b.ensure(R * d));
-  CK(m->kvs.ensure(((size_t)cfm_kv_split_halves(B, T, c.n_heads) + 1) / 2));  // 16-bit values, float units
-  const size_t S = (size_t)cfm_attn_splits(B, T, c.n_heads, m->n_cu);
-  if (S > 1) {
-    CK(m->apo.ensure(S * R * d));
-    CK(m->aml.ensure(S * R * c.n_heads * 2));
+  const int dk = (int)d / 16;
+  CK(m->actP.ensure(piece_floats(cfm_frag_pieces(R, round32(F > d ? F : d) / 16))));
+  CK(m->qF.ensure(piece_floats(cfm_q_pieces(B, T, c.n_heads))));
+  CK(m->kvF.ensure(piece_floats(cfm_kv_pieces(B, T, c.n_heads))));
+  const size_t hp = hp_pieces(c, T);
+  CK(m->hpP.ensure(piece_floats(B * hp)));
+  if (m->hp_B != B || m->hp_T != T) {  // the convolution's padding rows, zero from here on
+    CK(hipMemsetAsync(m->hpP.p, 0, sizeof(uint4) * B * hp, m->s));
+    m->hp_B = B;
+    m->hp_T = T;
+  }
+  const bool few = R < kMfmaRows;
+  if (few || unaligned_skip(c)) {
+    CK(m->n.ensure(R * d));
+    CK(m->xres.ensure(R * d));
+  }
+  if (few) {
+    CK(m->qkv.ensure(R * 3 * d));
+    CK(m->att.ensure(R * d));
+    CK(m->gu.ensure(R * 2 * F));
+    CK(m->act.ensure(R * (F > d ? F : d)));
+    CK(m->acts.ensure(R * 2 * d));
+    CK(m->rs.ensure(R * 2 * d));
+    for (auto &b : m->skips) CK(b.ensure(R * d));
+  } else {
+    const size_t rows = piece_floats(cfm_frag_pieces(R, dk));
+    // (a tile over one batch entry's rows reads up to 127 rows past them)
+    CK(m->nP.ensure(piece_floats(cfm_frag_pieces(R + 128, dk))));
+    for (Buf *b : {&m->attP, &m->curP, &m->xresP}) CK(b->ensure(rows));
+    for (auto &b : m->skipP) CK(b.ensure(rows));
+    CK(m->mP.ensure(piece_floats(cfm_frag_pieces(R, steps16(2 * c.in_ch + c.dim + c.style_dim)))));
+    CK(m->xtP.ensure(piece_floats(cfm_frag_pieces(R, steps16(c.in_ch)))));
   }
   if (m->rope_T != T) {
     CK(m->rope.ensure((size_t)T * 64));
@@ -208,13 +250,166 @@ itts_status timestep(itts_cfm *m, int e, int B, float *out) {
   return ITTS_OK;
 }
 
+// The U-ViT blocks, skip_linear and conv1 (cfm.rs:553-585) of at least kMfmaRows rows: residual
+// stream fp32 in hA / hB, every product's operand as fragment planes; leaves x_res in xresP,
+// WaveNet's input in hw (fp32) and hpP.
+itts_status blocks_mfma(itts_cfm *m, const float *x_t, const float *merged, int B, int T) {
+  const itts_cfm_config &c = m->c;
+  const int d = c.dim, C = c.in_ch, MD = 2 * C + d + c.style_dim, R = B * T, Lc = c.n_layers, split = Lc / 2;
+  const int na2 = (2 * Lc + 1) * 2 * d, dk = d / 16, F32 = round32(c.inter), pad = c.wn_kernel / 2;
+  hipStream_t s = m->s;
+#define WF(var, ...)                                                                                  \
+  const uint4 *var = weight_frag(m, __VA_ARGS__);                                                     \
+  if (!var) return cerr(ITTS_E_DEVICE, "out of device memory for the weights' operand planes")
+  auto mm = [&](const CfmMm &g, int epi, int batch) { return cfm_mm(g, epi, batch, m->n_cu, s); };
+  float *cur = m->hA.p, *oth = m->hB.p;
+  if (unaligned_merge(c)) {
+    CK(gemm(m, R, d, MD, merged, MD, m->merge_w, MD, cur, d, 0.0f, m->merge_b));
+  } else {
+    WF(w, m->merge_w, MD, d, MD);
+    CK(cfm_rows_frag(merged, MD, R, MD, steps16(MD), 0, pieces(m->mP), s));
+    CfmMm g = mm_args(pieces(m->mP), MD, w, R, d);
+    g.bias = m->merge_b;
+    g.y = cur;
+    g.ldy = d;
+    CK(mm(g, kMmPlain, 1));
+  }
+  int nsk = 0;
+  for (int i = 0; i < Lc; i++) {
+    const Block &b = m->L[i];
+    if (i > split && nsk > 0) {  // skip_in_linear([h, skip]): two operands along K
+      WF(w, b.skip_w, 2 * d, d, 2 * d);
+      CfmMm g = mm_args(pieces(m->curP), d, w, R, d);
+      g.a2 = pieces(m->skipP[--nsk]);
+      g.kt_a2 = g.nk1 = dk;
+      g.nk = 2 * dk;
+      g.bias = b.skip_b;
+      g.y = oth;
+      g.ldy = d;
+      CK(mm(g, kMmPlain, 1));
+      std::swap(cur, oth);
+    }
+    const float *mod_a = m->mods.p + (size_t)(2 * i) * 2 * d, *mod_f = m->mods.p + (size_t)(2 * i + 1) * 2 * d;
+    CK(cfm_norm_frag(cur, R, T, d, mod_a, na2, b.an_w, false, pieces(m->nP), s));
+    {
+      WF(w, b.wqkv, d, 3 * d, d);
+      CfmMm g = mm_args(pieces(m->nP), d, w, T, 3 * d);
+      g.zr = T;
+      g.o = pieces(m->qF);
+      g.o2 = pieces(m->kvF);
+      g.g = m->rope.p;
+      CK(mm(g, kMmQkv, B));
+    }
+    CK(cfm_attn_frag(pieces(m->qF), pieces(m->kvF), B, T, c.n_heads, pieces(m->attP), nullptr, m->n_cu, s));
+    {
+      WF(w, b.wo, d, d, d);
+      CfmMm g = mm_args(pieces(m->attP), d, w, R, d);
+      g.y = cur;
+      g.yr = cur;
+      g.ldy = d;
+      CK(mm(g, kMmPlain, 1));
+    }
+    CK(cfm_norm_frag(cur, R, T, d, mod_f, na2, b.fn_w, false, pieces(m->nP), s));
+    {
+      WF(w, b.w13, d, 2 * c.inter, d, c.inter);
+      CfmMm g = mm_args(pieces(m->nP), d, w, R, F32);
+      g.o = pieces(m->actP);
+      g.kt_o = F32 / 16;
+      CK(mm(g, kMmSwiglu, 1));
+    }
+    {  // hidden + ffn; the output's planes where a skip_in_linear reads them
+      WF(w, b.w2, c.inter, d, c.inter);
+      CfmMm g = mm_args(pieces(m->actP), c.inter, w, R, d);
+      g.kt_a = F32 / 16;
+      g.y = cur;
+      g.yr = cur;
+      g.ldy = d;
+      if (i < split) g.o = pieces(m->skipP[nsk++]);
+      else if (i + 1 < Lc && nsk > 0) g.o = pieces(m->curP);
+      g.kt_o = dk;
+      CK(mm(g, kMmPlain, 1));
+    }
+  }
+  // transformer.norm, x_res = skip_linear([h, x_t]), h = conv1(x_res)
+  const float *mod_n = m->mods.p + (size_t)(2 * Lc) * 2 * d;
+  if (unaligned_skip(c)) {
+    CK(cfm_adaln(cur, m->n.p, R, T, d, mod_n, na2, m->tn_w, s));
+    CK(gemm(m, R, d, d, m->n.p, d, m->skl_w, d + C, m->xres.p, d, 0.0f, m->skl_b));
+    CK(gemm(m, R, d, C, x_t, C, m->skl_w + d, d + C, m->xres.p, d, 1.0f));
+    CK(cfm_rows_frag(m->xres.p, d, R, d, dk, 0, pieces(m->xresP), s));
+  } else {
+    CK(cfm_norm_frag(cur, R, T, d, mod_n, na2, m->tn_w, false, pieces(m->nP), s));
+    CK(cfm_rows_frag(x_t, C, R, C, steps16(C), 0, pieces(m->xtP), s));
+    WF(w, m->skl_w, d + C, d, d, 0, d, C);
+    CfmMm g = mm_args(pieces(m->nP), d, w, R, d);
+    g.a2 = pieces(m->xtP);
+    g.kt_a2 = steps16(C);
+    g.nk1 = dk;
+    g.nk = dk + g.kt_a2;
+    g.bias = m->skl_b;
+    g.o = pieces(m->xresP);
+    g.kt_o = dk;
+    CK(mm(g, kMmPlain, 1));
+  }
+  WF(w, m->c1_w, d, d, d);
+  CfmMm g = mm_args(pieces(m->xresP), d, w, R, d);
+  g.bias = m->c1_b;
+  g.y = m->hw.p;
+  g.ldy = d;
+  g.T = T;
+  g.o = pieces(m->hpP);
+  g.so = (long)hp_pieces(c, T);
+  g.o_row0 = pad;
+  g.kt_o = dk;
+  CK(mm(g, kMmPlain, 1));
+  return ITTS_OK;
+}
+
+// The same of fewer rows: fp32 activations, fp32 FMA linears; x_res in xres, WaveNet's input in hw.
+itts_status blocks_few(itts_cfm *m, const float *x_t, const float *merged, int B, int T) {
+  const itts_cfm_config &c = m->c;
+  const int d = c.dim, F = c.inter, C = c.in_ch, MD = 2 * C + d + c.style_dim, R = B * T, Lc = c.n_layers;
+  const int split = Lc / 2, na2 = (2 * Lc + 1) * 2 * d;
+  hipStream_t s = m->s;
+  float *cur = m->hA.p, *oth = m->hB.p;
+  CK(gemm(m, R, d, MD, merged, MD, m->merge_w, MD, cur, d, 0.0f, m->merge_b));
+  int nsk = 0;
+  for (int i = 0; i < Lc; i++) {
+    const Block &b = m->L[i];
+    if (i > split && nsk > 0) {  // skip_in_linear([h, skip]) as two accumulating products
+      const float *sk = m->skips[--nsk].p;
+      CK(gemm(m, R, d, d, cur, d, b.skip_w, 2 * d, oth, d, 0.0f, b.skip_b));
+      CK(gemm(m, R, d, d, sk, d, b.skip_w + d, 2 * d, oth, d, 1.0f));
+      std::swap(cur, oth);
+    }
+    const float *mod_a = m->mods.p + (size_t)(2 * i) * 2 * d, *mod_f = m->mods.p + (size_t)(2 * i + 1) * 2 * d;
+    CK(cfm_adaln(cur, m->n.p, R, T, d, mod_a, na2, b.an_w, s));
+    CK(gemm(m, R, 3 * d, d, m->n.p, d, b.wqkv, d, m->qkv.p, 3 * d, 0.0f));
+    CK(cfm_qkv_frag(m->qkv.p, m->rope.p, B, T, c.n_heads, pieces(m->qF), pieces(m->kvF), s));
+    CK(cfm_attn_frag(pieces(m->qF), pieces(m->kvF), B, T, c.n_heads, nullptr, m->att.p, m->n_cu, s));
+    CK(gemm(m, R, d, d, m->att.p, d, b.wo, d, cur, d, 1.0f));
+    CK(cfm_adaln(cur, m->n.p, R, T, d, mod_f, na2, b.fn_w, s));
+    CK(gemm(m, R, 2 * F, d, m->n.p, d, b.w13, d, m->gu.p, 2 * F, 0.0f));
+    CK(cfm_swiglu(m->gu.p, R, F, m->act.p, s));
+    CK(gemm(m, R, d, F, m->act.p, F, b.w2, F, cur, d, 1.0f));  // hidden + ffn
+    if (i < split) {
+      CK(hipMemcpyAsync(m->skips[nsk++].p, cur, sizeof(float) * R * d, hipMemcpyDeviceToDevice, s));
+    }
+  }
+  CK(cfm_adaln(cur, m->n.p, R, T, d, m->mods.p + (size_t)(2 * Lc) * 2 * d, na2, m->tn_w, s));
+  CK(gemm(m, R, d, d, m->n.p, d, m->skl_w, d + C, m->xres.p, d, 0.0f, m->skl_b));
+  CK(gemm(m, R, d, C, x_t, C, m->skl_w + d, d + C, m->xres.p, d, 1.0f));
+  CK(gemm(m, R, d, d, m->xres.p, d, m->c1_w, d, m->hw.p, d, 0.0f, m->c1_b));
+  return ITTS_OK;
+}
+
 // forward_merged (cfm.rs:545-617) on device inputs x_t [B][T][C], merged [B][T][MD] and the
 // timesteps already in m->tdev; the velocity lands in m->v as [B][T][C].
 itts_status forward(itts_cfm *m, const float *x_t, const float *merged, int B, int T) {
   const itts_cfm_config &c = m->c;
-  const int d = c.dim, F = c.inter, C = c.in_ch, NL = c.wn_layers, K = c.wn_kernel, pad = K / 2;
-  const int MD = 2 * C + d + c.style_dim, R = B * T, Lc = c.n_layers, split = Lc / 2;
-  const int na2 = (2 * Lc + 1) * 2 * d;  // packed AdaLN modulation width
+  const int d = c.dim, C = c.in_ch, NL = c.wn_layers, K = c.wn_kernel, pad = K / 2, R = B * T, Lc = c.n_layers;
+  const int na2 = (2 * Lc + 1) * 2 * d, dk = d / 16;  // na2: packed AdaLN modulation width
+  const bool few = R < kMfmaRows;
   hipStream_t s = m->s;
   if (itts_status st = ensure_rows(m, B, T)) return st;
   // conditioning vectors: t1, t2, every AdaLN's (w, b), WaveNet's per-layer g, FinalLayer's (shift, scale)
@@ -224,83 +419,88 @@ itts_status forward(itts_cfm *m, const float *x_t, const float *merged, int B, i
   CK(gemm(m, B, 2 * d * NL, d, m->t2.p, d, m->wc_w, d, m->wng.p, 2 * d * NL, 0.0f, m->wc_b));
   CK(cfm_silu(m->t1.p, m->st.p, B * d, s));
   CK(gemm(m, B, 2 * d, d, m->st.p, d, m->fa_w, d, m->fmod.p, 2 * d, 0.0f, m->fa_b));
-  // h = cond_x_merge_linear(x_merged)
-  float *cur = m->hA.p, *oth = m->hB.p;
-  CK(gemm(m, R, d, MD, merged, MD, m->merge_w, MD, cur, d, 0.0f, m->merge_b));
-  // U-ViT blocks with long skips (cfm.rs:553-563)
-  int nsk = 0;
-  for (int i = 0; i < Lc; i++) {
-    const Block &b = m->L[i];
-    float *xin = cur;
-    if (i > split && nsk > 0) {  // skip_in_linear([h, skip]) as two accumulating GEMMs
-      const float *sk = m->skips[--nsk].p;
-      CK(gemm(m, R, d, d, cur, d, b.skip_w, 2 * d, oth, d, 0.0f, b.skip_b));
-      CK(gemm(m, R, d, d, sk, d, b.skip_w + d, 2 * d, oth, d, 1.0f));
-      xin = oth;
-      oth = cur;
-      cur = xin;
-    }
-    const float *mod_a = m->mods.p + (size_t)(2 * i) * 2 * d, *mod_f = m->mods.p + (size_t)(2 * i + 1) * 2 * d;
-    CK(cfm_adaln(xin, m->n.p, R, T, d, mod_a, na2, b.an_w, s));
-    CK(gemm(m, R, 3 * d, d, m->n.p, d, b.wqkv, d, m->qkv.p, 3 * d, 0.0f));
-    CK(cfm_attention(m->qkv.p, m->rope.p, B, T, d, c.n_heads, m->att.p, m->apo.p, m->aml.p,
-                     reinterpret_cast<uint16_t *>(m->kvs.p), m->n_cu, s));
-    // hidden = x_in + attn: in place, except where x_in must be kept (a block of the first
-    // half writes its output straight into its long-skip stash; the middle block's input
-    // is the last stash) and the sum goes out of place
-    if (i <= split) {
-      float *dst = i < split ? m->skips[nsk].p : (cur == m->hA.p ? m->hB.p : m->hA.p);
-      CK(gemm(m, R, d, d, m->att.p, d, b.wo, d, dst, d, 1.0f, nullptr, xin));
-      xin = dst;
-    } else {
-      CK(gemm(m, R, d, d, m->att.p, d, b.wo, d, xin, d, 1.0f));
-    }
-    CK(cfm_adaln(xin, m->n.p, R, T, d, mod_f, na2, b.fn_w, s));
-    if (R >= 64 && F % 32 == 0 && cfm_gemm_fits(m->n.p, d, b.w13, d, d)) {
-      // the SwiGLU in the [w1; w3] product's epilogue, over rows interleaved per 32
-      const uint4 *q13 = split_weights(m, b.w13, d, 2 * F, d, F);
-      if (!q13) return cerr(ITTS_E_DEVICE, "out of device memory for the split FFN weights");
-      CK(cfm_gemm_swiglu(R, F, d, m->n.p, d, q13, m->act.p, F, s));
-    } else {
-      CK(gemm(m, R, 2 * F, d, m->n.p, d, b.w13, d, m->gu.p, 2 * F, 0.0f));
-      CK(cfm_swiglu(m->gu.p, R, F, m->act.p, s));
-    }
-    CK(gemm(m, R, d, F, m->act.p, F, b.w2, F, xin, d, 1.0f));  // hidden + ffn
-    if (i < split) nsk++;
-    if (i <= split) {  // the block's output, in its stash or in the scratch buffer that is not cur
-      if (i == split) oth = cur == m->hA.p || cur == m->hB.p ? cur : (xin == m->hA.p ? m->hB.p : m->hA.p);
-      cur = xin;
-    }
-  }
-  // transformer.norm, x_res = skip_linear([h, x_t]), h = conv1(x_res)
-  CK(cfm_adaln(cur, m->n.p, R, T, d, m->mods.p + (size_t)(2 * Lc) * 2 * d, na2, m->tn_w, s));
-  CK(gemm(m, R, d, d, m->n.p, d, m->skl_w, d + C, m->xres.p, d, 0.0f, m->skl_b));
-  CK(gemm(m, R, d, C, x_t, C, m->skl_w + d, d + C, m->xres.p, d, 1.0f));
-  CK(gemm(m, R, d, d, m->xres.p, d, m->c1_w, d, oth, d, 0.0f, m->c1_b));
-  // WaveNet (cfm.rs:373-408): h in a zero-padded [B][T + 2 pad][d] buffer
-  CK(cfm_pad_rows(oth, B, T, d, pad, m->hpad.p, s));
-  CK(hipMemsetAsync(m->oacc.p, 0, sizeof(float) * R * d, s));
-  const long sp = (long)(T + 2 * pad) * d;
+  if (itts_status st = few ? blocks_few(m, x_t, merged, B, T) : blocks_mfma(m, x_t, merged, B, T)) return st;
+  auto mm = [&](const CfmMm &g, int epi, int batch) { return cfm_mm(g, epi, batch, m->n_cu, s); };
+  // WaveNet (cfm.rs:373-408): h fp32 in hw, and as the convolutions' operand in rows pad ..
+  // of the zero-padded planes; all taps are one product (K step kt reads row m + tap)
+  const long hp = (long)hp_pieces(c, T);
   for (int l = 0; l < NL; l++) {
     const WnLayer &w = m->wn[l];
     const bool last = l + 1 == NL;
     const int rso = last ? d : 2 * d;
-    // all taps as one product: row t of the padded input read K * d wide (rows t .. t+K-1);
-    // d is a multiple of 64, so the operands always suit the MFMA GEMM
-    const uint4 *in_q = split_weights(m, w.in_w, K * d, 2 * d, K * d);
-    if (!in_q) return cerr(ITTS_E_DEVICE, "out of device memory for the split WaveNet weights");
-    CK(cfm_gemm_split_w(B, T, 2 * d, K * d, m->hpad.p, d, sp, in_q, m->acts.p, 2 * d, (long)T * 2 * d, 0.0f, s));
-    CK(cfm_gate(m->acts.p, w.in_b, m->wng.p + (size_t)l * 2 * d, 2 * d * NL, R, T, d, m->act.p, s));
-    CK(gemm(m, R, rso, d, m->act.p, d, w.rs_w, d, m->rs.p, rso, 0.0f));
-    CK(cfm_res_skip(m->rs.p, w.rs_b, last ? 1 : 0, R, T, d, pad, m->hpad.p, m->oacc.p, s));
+    if (few)
+      for (int b = 0; b < B; b++)
+        CK(cfm_rows_frag(m->hw.p + (size_t)b * T * d, d, T, d, dk, pad, pieces(m->hpP) + b * hp, s));
+    WF(in_w, w.in_w, K * d, 2 * d, K * d, few ? 0 : d);
+    CfmMm g = mm_args(pieces(m->hpP), K * d, in_w, T, d);
+    g.sa = hp;
+    g.kt_a = g.taps_kt = dk;
+    if (few) {
+      g.N = 2 * d;
+      g.y = m->acts.p;
+      g.ldy = 2 * d;
+      g.sy = (long)T * 2 * d;
+      CK(mm(g, kMmConv, B));
+      CK(cfm_gate(m->acts.p, w.in_b, m->wng.p + (size_t)l * 2 * d, 2 * d * NL, R, T, d, m->act.p, s));
+      CK(gemm(m, R, rso, d, m->act.p, d, w.rs_w, d, m->rs.p, rso, 0.0f));
+      CK(cfm_res_skip(m->rs.p, w.rs_b, last ? 1 : 0, l == 0, R, d, m->hw.p, m->oacc.p, s));
+      continue;
+    }
+    g.bias = w.in_b;
+    g.g = m->wng.p + (size_t)l * 2 * d;
+    g.ld_g = 2 * d * NL;
+    g.o = pieces(m->actP);
+    g.kt_o = dk;
+    CK(mm(g, kMmGate, B));
+    WF(rs_w, w.rs_w, d, rso, d);
+    CfmMm r = mm_args(pieces(m->actP), d, rs_w, R, rso);
+    r.T = T;
+    r.bias = w.rs_b;
+    r.y = m->hw.p;
+    r.y2 = m->oacc.p;
+    r.ldy = d;
+    r.o = pieces(m->hpP);
+    r.so = hp;
+    r.o_row0 = pad;
+    r.kt_o = dk;
+    r.first = l == 0;
+    CK(mm(r, kMmResSkip, 1));
   }
   // h = wavenet + res_projection(x_res); FinalLayer; conv2
-  CK(cfm_add_bias(m->oacc.p, d, m->rp_b, R, d, s));
-  CK(gemm(m, R, d, d, m->xres.p, d, m->rp_w, d, m->oacc.p, d, 1.0f));
-  CK(cfm_final_norm(m->oacc.p, m->n.p, R, T, d, m->fmod.p, s));
-  CK(gemm(m, R, d, d, m->n.p, d, m->fl_w, d, cur, d, 0.0f, m->fl_b));
-  CK(gemm(m, R, C, d, cur, d, m->c2_w, d, m->v.p, C, 0.0f, m->c2_b));
+  float *h = m->hA.p;
+  if (few) {
+    CK(gemm(m, R, d, d, m->xres.p, d, m->rp_w, d, m->oacc.p, d, 1.0f, m->rp_b));
+    CK(cfm_final_norm(m->oacc.p, m->n.p, R, T, d, m->fmod.p, s));
+    CK(gemm(m, R, d, d, m->n.p, d, m->fl_w, d, h, d, 0.0f, m->fl_b));
+    CK(gemm(m, R, C, d, h, d, m->c2_w, d, m->v.p, C, 0.0f, m->c2_b));
+    return ITTS_OK;
+  }
+  {
+    WF(w, m->rp_w, d, d, d);
+    CfmMm g = mm_args(pieces(m->xresP), d, w, R, d);
+    g.bias = m->rp_b;
+    g.y = m->oacc.p;
+    g.yr = m->oacc.p;
+    g.ldy = d;
+    CK(mm(g, kMmPlain, 1));
+  }
+  CK(cfm_norm_frag(m->oacc.p, R, T, d, m->fmod.p, 2 * d, nullptr, true, pieces(m->nP), s));
+  {
+    WF(w, m->fl_w, d, d, d);
+    CfmMm g = mm_args(pieces(m->nP), d, w, R, d);
+    g.bias = m->fl_b;
+    g.o = pieces(m->attP);
+    g.kt_o = dk;
+    CK(mm(g, kMmPlain, 1));
+  }
+  WF(w, m->c2_w, d, C, d);
+  CfmMm g = mm_args(pieces(m->attP), d, w, R, C);
+  g.bias = m->c2_b;
+  g.y = m->v.p;
+  g.ldy = C;
+  CK(mm(g, kMmPlain, 1));
   return ITTS_OK;
+#undef WF
 }
 
 }  // namespace
@@ -407,6 +607,7 @@ itts_status itts_cfm_create(const itts_cfm_config *cfg, const char *const *names
         hipDeviceGetAttribute(&m->n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       return fail(cerr(ITTS_E_DEVICE, "querying the device's compute units failed"));
   }
+  if (cfm_mm_init() != hipSuccess) return fail(cerr(ITTS_E_DEVICE, "preparing the product kernels failed"));
   if (hipMalloc(&m->arena, top * sizeof(float)) != hipSuccess)
     return fail(cerr(ITTS_E_DEVICE, "out of device memory for the CFM weights (%zu bytes)", top * sizeof(float)));
   for (const auto &kv : seen) {
@@ -455,6 +656,7 @@ itts_status itts_cfm_create(const itts_cfm_config *cfg, const char *const *names
   m->c2_w = at("conv2.weight");
   m->c2_b = at("conv2.bias");
   m->skips.resize(Lc / 2);
+  m->skipP.resize(Lc / 2);
   if (hipEventCreate(&m->e0) != hipSuccess || hipEventCreate(&m->e1) != hipSuccess)
     return fail(cerr(ITTS_E_DEVICE, "hipEventCreate failed"));
   *out = m;
@@ -513,7 +715,18 @@ itts_status itts_cfm_solve_euler(itts_cfm *m, const float *cat_condition, int32_
   CK(hipMemsetAsync(m->merged.p, 0, sizeof(float) * 2 * T * MD, s));
   CK(cfm_static_tail(m->merged.p, MD, C, d, S, T, m->refm.p, T_ref, m->sty.p, s));
   CK(cfm_bias_rows(m->merged.p + 2 * C, MD, m->cond_b, 2 * T, d, s));
-  CK(gemm(m, T, d, d, m->catc.p, d, m->cond_w, d, m->merged.p + 2 * C, MD, 1.0f));
+  if (T >= kMfmaRows) {  // (2 T rows: the planes' path, whose buffers are in place)
+    const uint4 *w = weight_frag(m, m->cond_w, d, d, d);
+    if (!w) return cerr(ITTS_E_DEVICE, "out of device memory for the weights' operand planes");
+    CK(cfm_rows_frag(m->catc.p, d, T, d, d / 16, 0, pieces(m->nP), s));
+    CfmMm g = mm_args(pieces(m->nP), d, w, T, d);
+    g.y = m->merged.p + 2 * C;
+    g.yr = g.y;
+    g.ldy = MD;
+    CK(cfm_mm(g, kMmPlain, 1, m->n_cu, s));
+  } else {
+    CK(gemm(m, T, d, d, m->catc.p, d, m->cond_w, d, m->merged.p + 2 * C, MD, 1.0f));
+  }
   CK(hipEventRecord(m->e0, s));
   const float dt = 1.0f / (float)n_timesteps;
   for (int step = 0; step < n_timesteps; step++) {

@@ -1,0 +1,206 @@
+// Operands of v_mfma_f32_32x32x16_f16 kept in memory in fragment order, and the attention
+// loop that runs on them (gfx950, wave64).
+//
+// A matrix X [rows][K] that a product reads as an MFMA operand is stored as fp16 hi/lo
+// planes in blocks of 32 rows x 16 K: lane l of the operand holds row (l & 31), K values
+// 8 (l >> 5) .. +7, so a block's plane is 64 pieces of 16 bytes in lane order (1 KiB) and
+// an operand load is one fully coalesced 16-byte load per lane straight into registers: no
+// LDS staging, no barrier, and any number of K steps in flight.
+#pragma once
+
+#include "common.h"
+
+namespace itts {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+#define ITTS_MFMA16 __builtin_amdgcn_mfma_f32_32x32x16_f16
+
+// 16-byte piece of (row, 8-value chunk k8 of K), hi plane; the lo plane's is 64 pieces on.
+// nk: K steps of 16 that a row block holds.
+__host__ __device__ inline size_t frag_piece(long row, int k8, int nk) {
+  return (((size_t)(row >> 5) * nk + (k8 >> 1)) * 2) * 64 + (size_t)((k8 & 1) * 32 + (row & 31));
+}
+
+__device__ __forceinline__ void split8(const float v[8], u32x4 &hi, u32x4 &lo) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    uint32_t h, l;
+    split_f16x2(v[2 * j], v[2 * j + 1], h, l);
+    hi[j] = h;
+    lo[j] = l;
+  }
+}
+
+// Exchanges v with lane ^ 32 (one VALU swap, no LDS round trip).
+__device__ __forceinline__ float other_half(float v, int lane) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(lane < 32 ? r[1] : r[0]);
+}
+
+// ---- attention over key tiles of 32, one wave for 32 queries ----------------------------
+// The scores are formed transposed, S^T = K Q^T: a lane then holds 16 keys of one query, so
+// the softmax needs no cross-lane reduction but one exchange between the wave's halves, and
+// the probabilities are already the B operand of O^T = V^T P^T (registers 8 kk .. 8 kk + 7
+// are the keys of K step kk) with no LDS round trip.  V^T's fragments hold their keys in that
+// order: position 8 h + 4 j2 + b of a 16-key step is key 8 j2 + 4 h + b.
+//
+// A key tile holds 8 fragments (4 K steps of K rows over the 64 dims; 2 dim tiles x 2 key
+// steps of V^T) of NP planes each: kFlashFrags * NP KiB, contiguous.  NP = 1 where the lo
+// planes are all zero (bf16 rows: eight significant bits fit fp16 exactly, and below fp16's
+// normal range both forms stop at the same 2^-25).
+constexpr int kFlashFrags = 8;
+__host__ __device__ inline size_t flash_tile_pieces(int np) { return (size_t)kFlashFrags * np * 64; }
+// position of key t (mod 16) within V^T's 16-key step
+__host__ __device__ inline int flash_key_pos(int t) { return ((t >> 2) & 1) * 8 + ((t >> 3) & 1) * 4 + (t & 3); }
+
+struct FlashState {
+  float m, l;      // reference exponent and this lane's share (its half's keys) of the denominator
+  floatx16 O[2];   // O^T: column = query (lane & 31), rows 8 (i >> 2) + 4 (lane >> 5) + (i & 3) of each 32 dims
+};
+
+__device__ __forceinline__ void flash_init(FlashState &st) {
+  st.m = -3.0e38f;
+  st.l = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    st.O[0][i] = 0.0f;
+    st.O[1][i] = 0.0f;
+  }
+}
+
+// Key tiles [t0, t1) at kv (piece index of tile 0 of this head, lane added); q is scaled so
+// that a score's exponential is 2^s.  mask(tile, S) sets scores of masked keys to -inf.  The
+// exponent reference m is raised only when some score passes it by more than 2^8: until then
+// probabilities up to 2^8 are carried, in the same relative precision, and the rescaling of
+// O is skipped.
+template <int NP, class Mask>
+__device__ __forceinline__ void flash_tiles(const u32x4 *kv, int t0, int t1, const f16x8 (&qh)[4],
+                                            const f16x8 (&ql)[4], Mask mask, FlashState &st) {
+  if (t0 >= t1) return;
+  u32x4 kf[4][NP], vf[4][NP];
+  auto load_k = [&](int t) __attribute__((always_inline)) {
+    const u32x4 *p = kv + (size_t)t * flash_tile_pieces(NP);
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int pl = 0; pl < NP; pl++) kf[f][pl] = p[(f * NP + pl) * 64];
+  };
+  auto load_v = [&](int t) __attribute__((always_inline)) {
+    const u32x4 *p = kv + (size_t)t * flash_tile_pieces(NP) + 4 * NP * 64;
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int pl = 0; pl < NP; pl++) vf[f][pl] = p[(f * NP + pl) * 64];
+  };
+  load_k(t0);
+  load_v(t0);
+  for (int t = t0; t < t1; t++) {
+    floatx16 S;
+#pragma unroll
+    for (int i = 0; i < 16; i++) S[i] = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+      const f16x8 kh = __builtin_bit_cast(f16x8, kf[kk][0]);
+      S = ITTS_MFMA16(kh, qh[kk], S, 0, 0, 0);
+      S = ITTS_MFMA16(kh, ql[kk], S, 0, 0, 0);
+      if constexpr (NP == 2) S = ITTS_MFMA16(__builtin_bit_cast(f16x8, kf[kk][1]), qh[kk], S, 0, 0, 0);
+    }
+    // the next tile's K into the registers just read (the last tile's again at the end)
+    load_k(min(t + 1, t1 - 1));
+    mask(t, S);
+    float tmax = fmaxf(S[0], S[1]);
+#pragma unroll
+    for (int i = 2; i < 16; i++) tmax = fmaxf(tmax, S[i]);
+    if (__any(tmax > st.m + 8.0f)) {
+      const float mn = fmaxf(st.m, fmaxf(tmax, other_half(tmax, threadIdx.x & 63)));
+      const float corr = __builtin_amdgcn_exp2f(st.m - mn);
+      st.m = mn;
+      st.l *= corr;
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        st.O[0][i] *= corr;
+        st.O[1][i] *= corr;
+      }
+    }
+    float p[16];
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      p[i] = __builtin_amdgcn_exp2f(S[i] - st.m);
+      sum += p[i];
+    }
+    st.l += sum;
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) {
+      u32x4 h, l;
+      split8(p + 8 * kk, h, l);
+      const f16x8 ph = __builtin_bit_cast(f16x8, h), pl = __builtin_bit_cast(f16x8, l);
+#pragma unroll
+      for (int dt = 0; dt < 2; dt++) {
+        const f16x8 vh = __builtin_bit_cast(f16x8, vf[dt * 2 + kk][0]);
+        st.O[dt] = ITTS_MFMA16(vh, ph, st.O[dt], 0, 0, 0);
+        st.O[dt] = ITTS_MFMA16(vh, pl, st.O[dt], 0, 0, 0);
+        if constexpr (NP == 2)
+          st.O[dt] = ITTS_MFMA16(__builtin_bit_cast(f16x8, vf[dt * 2 + kk][1]), ph, st.O[dt], 0, 0, 0);
+      }
+    }
+    load_v(min(t + 1, t1 - 1));
+  }
+}
+
+// The waves of a block that share queries (wave g of WK took the keys' part g) merge their
+// states through LDS (buf: WK x 2112 floats per query tile); wave 0 of the group returns
+// with O and the full denominator.  Every thread of the block calls it.
+template <int WK>
+__device__ __forceinline__ void flash_merge(FlashState &st, float *buf, int g, int lane) {
+  st.l += other_half(st.l, lane);
+  if constexpr (WK > 1) {
+    float *mine = buf + g * 2112;
+    if (g > 0) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        mine[i * 64 + lane] = st.O[0][i];
+        mine[(16 + i) * 64 + lane] = st.O[1][i];
+      }
+      if (lane < 32) {
+        mine[2048 + lane] = st.m;
+        mine[2080 + lane] = st.l;
+      }
+    }
+    __syncthreads();
+    if (g == 0) {
+      float mg[WK], M = st.m;
+#pragma unroll
+      for (int j = 1; j < WK; j++) {
+        mg[j] = buf[j * 2112 + 2048 + (lane & 31)];
+        M = fmaxf(M, mg[j]);
+      }
+      const float f0 = __builtin_amdgcn_exp2f(st.m - M);
+      st.l *= f0;
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        st.O[0][i] *= f0;
+        st.O[1][i] *= f0;
+      }
+#pragma unroll
+      for (int j = 1; j < WK; j++) {
+        const float *o = buf + j * 2112;
+        const float f = __builtin_amdgcn_exp2f(mg[j] - M);
+        st.l += o[2080 + (lane & 31)] * f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          st.O[0][i] += o[i * 64 + lane] * f;
+          st.O[1][i] += o[(16 + i) * 64 + lane] * f;
+        }
+      }
+      st.m = M;
+    }
+  }
+}
+
+}  // namespace itts

@@ -287,55 +287,80 @@ bool sampler_stage(int dev, SamplerStage *out);
 hipError_t cfm_temb(const float *t, int B, float *emb /*[B][256]*/, hipStream_t s);
 hipError_t cfm_silu(const float *x, float *y, int n, hipStream_t s);
 hipError_t cfm_bias_rows(float *C, int ldc, const float *bias, int rows, int cols, hipStream_t s);
-hipError_t cfm_add_bias(float *C, int ldc, const float *bias, int rows, int cols, hipStream_t s);
 hipError_t cfm_adaln(const float *x, float *y, int R, int T, int d, const float *mod, int ld_mod, const float *norm_w,
                      hipStream_t s);
 hipError_t cfm_final_norm(const float *x, float *y, int R, int T, int d, const float *mod, hipStream_t s);
 // rope (cos, sin) table [T][32][2] for positions 0..T-1
 hipError_t cfm_rope_table(int T, float *tab, hipStream_t s);
-// Key splits the attention uses for this shape on n_cu compute units (1..8); with more than
-// one, part_o holds [S][B][T][d] and part_ml [S][B][H][T][2] floats.
-int cfm_attn_splits(int B, int T, int H, int n_cu);
-// kv_split: workspace of cfm_kv_split_halves(B, T, H) 16-bit values (K with rope and V as
-// fp16 hi/lo planes, built once per call and shared by every query tile).
-int cfm_kv_split_halves(int B, int T, int H);
-// The MFMA GEMM's operand rules: K, lda, ldw multiples of 4 and A, W 16-byte aligned (the
-// split and the launches reject anything else).
-bool cfm_gemm_fits(const float *A, int lda, const float *W, int ldw, int K);
-// The constant operand W [N][ldw] split once into fp16 hi/lo quads (cfm_split_weights_quads(N,
-// K) uint4 at out, rows padded to 64 and k to 128 with zeros), and the products over them:
-// cfm_gemm_split_w y[z] = A[z] W^T (+ bias) + beta y[z] for z < batch (row-major; A rows lda
-// apart and allowed to overlap, batch strides sa / sy in floats) on the MFMA units with fp16
-// hi/lo operands and fp32 accumulation (K, lda multiples of 4, A 16-byte aligned).
-size_t cfm_split_weights_quads(int N, int K);
-hipError_t cfm_split_weights(const float *W, int ldw, int N, int K, uint4 *out, hipStream_t s, int ilv = 0);
-// act [M][ldo] = silu(A W1^T) * (A W3^T) for the packed W = [w1; w3] (2F rows) split with
-// ilv = F: the SwiGLU in the product's epilogue (F a multiple of 32).
-hipError_t cfm_gemm_swiglu(int M, int F, int K, const float *A, int lda, const uint4 *Wp, float *act, int ldo,
-                           hipStream_t s);
-hipError_t cfm_gemm_split_w(int batch, int M, int N, int K, const float *A, int lda, long sa, const uint4 *Wp,
-                            float *y, int ldy, long sy, float beta, hipStream_t s, const float *bias = nullptr,
-                            const float *yr = nullptr);
+// ---- products over fragment planes (kernels_cfm_mm.hip; layout in frag.h) ----
+// 16-byte pieces of the planes of `rows` rows (whole 128-row tiles) with nk K steps of 16.
+size_t cfm_frag_pieces(long rows, int nk);
+// Weight rows W [N][ldw] -> K steps kt0 .. kt0 + ceil(K / 16) of `out` (cfm_frag_pieces(N, nk),
+// zero-filled by the caller where K steps stay unwritten).  With ilv = F (N = 2F) the two
+// halves' rows alternate per 32, as the SwiGLU and gate epilogues take them (cfm_frag_pieces of
+// 64 ceil(F / 32) rows).
+hipError_t cfm_weight_frag(const float *W, int ldw, int N, int K, int kt0, int nk, int ilv, uint4 *out, hipStream_t s);
+// fp32 rows X [R][ld] (K values) -> rows row0 .. of the planes `out`, nk K steps, zeros past K.
+hipError_t cfm_rows_frag(const float *X, int ld, int R, int K, int nk, int row0, uint4 *out, hipStream_t s);
+// AdaLN (or, final_norm, the final layer's norm with mod = shift | scale) of x [R][d] as planes.
+hipError_t cfm_norm_frag(const float *x, int R, int T, int d, const float *mod, int ld_mod, const float *norm_w,
+                         bool final_norm, uint4 *out, hipStream_t s);
+// One product y[z] = A[z] W^T, z < batch; the epilogue by kind:
+//   Plain   (+ bias) (+ yr) to fp32 rows y (ldy, batch stride sy) and / or planes o (kt_o K
+//           steps, batch stride so pieces, rows from o_row0)
+//   Conv    Plain over a convolution's operand: K step kt reads row m + kt / taps_kt
+//   Gate    Conv, tanh(first half) * sigmoid(second half) with bias + g rows, to planes o;
+//           N output columns, W interleaved
+//   Swiglu  silu(first) * second to planes o; N output columns, W interleaved
+//   ResSkip rows r = b T + t: columns < N - ldy add to y [.][ldy] and go to planes o (batch
+//           b, row t + o_row0); the last ldy columns add to (first: set) y2 [.][ldy]
+//   Qkv     N = 3d: o = Q and o2 = K, V fragments of the attention, with rope (g = the table)
+enum CfmEpi : int { kMmPlain, kMmConv, kMmGate, kMmSwiglu, kMmResSkip, kMmQkv };
+struct CfmMm {
+  const uint4 *a, *a2;  // planes; a2 (optional) holds K steps nk1 ..
+  long sa;
+  int zr;               // rows between batch entries that share a's planes
+  int kt_a, kt_a2, nk1;  // K steps a row block of a / a2 holds
+  const uint4 *w;
+  int nk, taps_kt, M, N;
+  int T;                // Plain, ResSkip: rows r = b T + t go to batch b's planes (0: entry z's)
+  const float *bias, *yr;
+  float *y, *y2;
+  int ldy;
+  long sy;
+  uint4 *o, *o2;
+  int kt_o;
+  long so;
+  int o_row0;
+  const float *g;
+  int ld_g, first;
+  int vec, nM, nN, nz, gm;  // set at the launch: y, yr and bias take 16-byte accesses; the tile grid
+};
+hipError_t cfm_mm_init();  // once per device, before the first product
+hipError_t cfm_mm(CfmMm a, int epi, int batch, int n_cu, hipStream_t s);
+// Pieces of the attention's Q and K / V fragments, the fragments from fp32 rows qkv [B][T][3d],
+// and the attention over them (to planes out [B T][d], or fp32 rows out_f).
+size_t cfm_q_pieces(int B, int T, int H);
+size_t cfm_kv_pieces(int B, int T, int H);
+hipError_t cfm_qkv_frag(const float *qkv, const float *rope_tab, int B, int T, int H, uint4 *qf, uint4 *kvf,
+                        hipStream_t s);
+hipError_t cfm_attn_frag(const uint4 *qf, const uint4 *kvf, int B, int T, int H, uint4 *out, float *out_f, int n_cu,
+                         hipStream_t s);
 // The same product in fp32 FMAs for few rows (any M, any alignment; float4 loads when K,
 // lda, ldw, sa, sw are multiples of 4 and A, W are 16-byte aligned); beta 0 never reads y.
-// With bias (here and in cfm_gemm_split_w): y = A W^T + bias[n] + beta y; with yr, beta's
-// old values come from yr (same layout as y) and y is written out of place.
+// With bias: y = A W^T + bias[n] + beta y.
 hipError_t cfm_rows_gemm(int batch, int M, int N, int K, const float *A, int lda, long sa, const float *W, int ldw,
-                         long sw, float *y, int ldy, long sy, float beta, hipStream_t s, const float *bias = nullptr,
-                         const float *yr = nullptr);
-hipError_t cfm_attention(const float *qkv, const float *rope_tab, int B, int T, int d, int H, float *out,
-                         float *part_o, float *part_ml, uint16_t *kv_split, int n_cu, hipStream_t s);
+                         long sw, float *y, int ldy, long sy, float beta, hipStream_t s, const float *bias = nullptr);
 hipError_t cfm_swiglu(const float *gu, int R, int F, float *out, hipStream_t s);
 hipError_t cfm_gate(const float *acts, const float *in_b, const float *g, int ld_g, int R, int T, int d, float *act,
                     hipStream_t s);
-hipError_t cfm_res_skip(const float *rs, const float *rs_b, int last, int R, int T, int d, int pad, float *h,
-                        float *out, hipStream_t s);
+hipError_t cfm_res_skip(const float *rs, const float *rs_b, int last, int first, int R, int d, float *h, float *out,
+                        hipStream_t s);
 hipError_t cfm_euler_prep(float *x, int C, int T, int T_ref, float *xt, float *merged, int MD, hipStream_t s);
 hipError_t cfm_euler_update(float *x, const float *v, int C, int T, float dt, float cfg, hipStream_t s);
 hipError_t cfm_static_tail(float *merged, int MD, int C, int d, int S, int T, const float *ref_mel, int T_ref,
                            const float *style, hipStream_t s);
 hipError_t cfm_transpose_tc(const float *v, int B, int T, int C, float *out, hipStream_t s);
-hipError_t cfm_pad_rows(const float *x, int B, int T, int d, int pad, float *hp, hipStream_t s);
 hipError_t cfm_fill(float *p, int n, float v, hipStream_t s);
 
 }  // namespace itts

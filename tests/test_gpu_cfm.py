@@ -143,3 +143,31 @@ def test_full_size_forward_matches_oracle(T):
         assert rel(got, ref) < 2e-4
     finally:
         m.close()
+
+
+# The products' tiles (64 and 32 rows), the fp32 path's last and the planes path's first row
+# count, key tiles of 32, batch entries whose rows start inside a row block, FFN widths that
+# are not whole 32-column groups, and a wider convolution
+EDGE_CONFIG = dict(SMALL_CONFIG, inter=200, wn_kernel=7)
+
+
+@pytest.mark.parametrize("B,T", [(2, 31), (2, 32), (1, 64), (1, 65), (2, 65), (3, 33), (2, 129), (1, 193), (4, 250)])
+def test_forward_tile_edges(B, T):
+    say(f"[gpu] cfm forward edges B={B} T={T}")
+    W = synth.make_cfm_weights(EDGE_CONFIG, seed=8)
+    m = CfmDit(W, EDGE_CONFIG)
+    try:
+        rng = np.random.default_rng(100 * B + T)
+        M = ito.CfmModel(W, EDGE_CONFIG)
+        # a longer forward first: what it leaves in the buffers must not reach the next one
+        for frames in (T + 70, T):
+            x_t = rng.standard_normal((B, frames, EDGE_CONFIG["in_ch"])).astype(np.float32)
+            x_m = rng.standard_normal((B, frames, merged_dim(EDGE_CONFIG))).astype(np.float32)
+            x_m[..., :EDGE_CONFIG["in_ch"]] = x_t
+            t = rng.random(B).astype(np.float32)
+            got = m.forward_merged(x_t, x_m, t)
+        ref = M.forward_merged(x_t, x_m, t)
+        # 2e-4 as above: the operands' 2^-22 through a handful of layers leaves two orders of margin
+        assert rel(got, ref) < 2e-4
+    finally:
+        m.close()
