@@ -123,17 +123,6 @@ hipError_t launch_attn_probe(const float *q, int M, const int *kstart, const voi
 // (head, row) (short prompts); the output rows are written in the GEMM's split form.
 hipError_t launch_attn_prefill(const float *q, int T, int base, const void *kc, const void *vc,
                                int n_head, int max_seq, const SplitOut &out, int kvt, hipStream_t s);
-// Causal attention of T rows on the MFMA units: row t sits at position base + t of the
-// K/V [n_head][ld][64] (bf16 or fp32) and attends to keys ks(t)..base + t, ks(t) =
-// kstart[t] or 0; output rows in the GEMM's split form.
-// With kv_split (attn_kv_split_halves(n_head, base + T) 16-bit values), K and V are split into
-// fp16 hi/lo planes once per call instead of once per query tile.  With tile_order (a
-// permutation of the ceil(T / 64) query tiles), grid row y runs query tile tile_order[y]:
-// callers list the tiles with the most keys first so the short ones fill in behind them.
-size_t attn_kv_split_halves(int n_head, int keys);
-hipError_t launch_attn_flash(const float *q, int T, int base, const int *kstart, const void *kc, const void *vc,
-                             int ld, int n_head, const SplitOut &out, int kvt, hipStream_t s,
-                             uint16_t *kv_split = nullptr, const int *tile_order = nullptr);
 // out[r] = log_softmax(logits[r])[codes[r]] for R rows of V logits.
 hipError_t launch_log_softmax_pick(const float *logits, int R, int V, const int *codes, float *out, hipStream_t s);
 
@@ -182,12 +171,53 @@ struct GemmArgs {
   int n_cu;         // compute units (grid sizing)
 };
 hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt, hipStream_t s);
-// The tiled product uses 64 x 64 tiles up to this many rows, 128 x 128 tiles above.
-constexpr int kGemmSmallTileRows = 512;
 // Sets the LDS attributes of every GEMM instantiation (before any graph capture).
 hipError_t gemm_init();
 size_t gemm_ws_floats(int n_cu);
 constexpr int kGemmCounters = 4096;
+
+// ---- multi-row forwards on operands in fragment order (kernels_rows.hip) ----
+// Activation planes of M rows of K values (16-byte pieces; the group sums' last step must be
+// zero-filled once), the attention's Q and K / V fragments, and a weight's codes in fragment
+// order, scale table and bias planes (made once by rows_params).
+size_t rows_planes_pieces(int M, int K);
+size_t rows_q_pieces(int M, int H);
+size_t rows_kv_pieces(int M, int H);
+int rows_ldn(int N);
+size_t rows_scale_floats(int N, int K);
+size_t rows_bias_pieces(int N, int K);
+size_t rows_codes_bytes(int N, int K, int bits);
+hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, hipStream_t s);
+// LN (and a second one with w2; none without w) of M rows [M][d] as planes.
+hipError_t rows_ln(const float *x, const float *w, const float *b, const float *w2, const float *b2, int M, int d,
+                   uint4 *out, hipStream_t s);
+// One product over planes x, with the epilogues of launch_gemm: store y [M][N]; residual y +=,
+// and with `o` the next folded LayerNorm's input (planes of gamma x, group statistics so);
+// GELU to planes o; QKV to the fragments qf / kvf, to the cache rows 0.. [n_head][max_seq][64]
+// where kc / vc are set, and q to q_out [M][N / 3] where set.  st, fG, fc: folded LayerNorm input.
+struct RowsMm {
+  const uint4 *x, *codes;
+  const float *scale;
+  const uint4 *bw;
+  const float *bias;
+  int ldn, M, N, K;
+  const float2 *st;
+  const float *fG, *fc;
+  float *y;
+  uint4 *o;
+  const float *gamma;
+  float2 *so;
+  uint4 *qf, *kvf;
+  float *q_out;
+  void *kc, *vc;
+  int max_seq, n_cu;
+  int nM, nN, gm;  // tile grid, set at the launch
+};
+hipError_t rows_mm(const RowsMm &a, int bits, int epi, int kvt, hipStream_t s);
+// Causal attention: row t attends to keys kstart[t] (or 0) .. t; order (optional) lists the
+// ceil(M / 32) query tiles, most keys first.  Output as planes [M][64 H].
+hipError_t rows_attn(const uint4 *qf, const uint4 *kvf, int M, int H, const int *kstart, const int *order, int kvt,
+                     uint4 *out, hipStream_t s);
 
 // fp32 rows [M][K] -> the GEMM's split form.
 hipError_t launch_split_rows(const float *x, int M, int K, const SplitOut &o, hipStream_t s);

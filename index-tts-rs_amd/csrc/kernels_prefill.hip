@@ -312,9 +312,9 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
           acc[i][j][e] = fmaf(sbp[j].x, P[i][j][e], fmaf(sbp[j].y, gsp[i][e >> 2][e & 3], acc[i][j][e]));
   };
 
-  // The fold straight from the stage in LDS (128 x 128 tiles): the group sums of one M
+  // The fold straight from the stage in LDS: the group sums of one M
   // sub-tile at a time are held in registers, so the fold adds 16 registers to the
-  // partial tile instead of 32 (those tiles run at the 256-register limit).
+  // partial tile instead of 32.
   auto apply_from = [&](const char *st, const floatx16(&P)[TM][TN]) __attribute__((always_inline)) {
     read_params(st);
 #pragma unroll
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     if (copier && i + NS - 1 < ng) issue(g0 + i + NS - 1, stage(i + NS - 1));
     if (worker) {
       if constexpr (PROD) {
-        // 128 x 128 tiles at two waves per SIMD: the group's affine is applied at once, so
+        // at two waves per SIMD the group's affine is applied at once, so
         // only one partial tile is live (the other wave on the SIMD covers the MFMA latency)
         mma(stage(i), Pc);
         apply_from(stage(i), Pc);
@@ -1177,12 +1177,11 @@ __global__ __launch_bounds__(256) void dequant_kernel(DevQL ql, float *out) {
   }
 }
 
-// Tile configurations: small (64 x 64, two blocks per CU) for the prefill of one
-// utterance, large (128 x 128, one block per CU) for many rows.
+// 64 x 64 tiles, two blocks per CU.
 constexpr int kStages = 3;
 
 struct Plan {
-  int TM, TN, mode, nN, mt, S, gps, blocks;
+  int mode, nN, mt, S, gps, blocks;
   size_t lds;
 };
 
@@ -1193,20 +1192,17 @@ constexpr size_t lds_bytes() {
 
 Plan make_plan(const GemmArgs &a, int bits, int ptype) {
   Plan p{};
-  const bool large = a.M > kGemmSmallTileRows;
-  p.TM = p.TN = large ? 2 : 1;
-  const int BM = 64 * p.TM, BN = 64 * p.TN;
+  const int BM = 64, BN = 64;
   const int G = a.ql.K / kGroup;
   p.nN = (a.ql.N + BN - 1) / BN;
   p.mt = (a.M + BM - 1) / BM;
   const int tiles = p.nN * p.mt;
-  const int slots = std::max(1, a.n_cu) * (large ? 1 : 2);
+  const int slots = std::max(1, a.n_cu) * 2;
   // Split count with the lowest modelled time; partial tiles must fit the workspace.
   // Small tiles (copier waves, two blocks per CU), in microseconds, fitted to MI355X timings
   // of the decoder's four GEMM shapes at 8, 99, 163 and 235 rows: ~0.95 us per split (the
   // last block of a tile adds every partial), and per K group of a block ~0.42 us while the
-  // blocks fit one per CU, rising with the blocks per CU.  Large tiles (one block per CU):
-  // rounds x (groups + fill) in group units plus a reduction term.
+  // blocks fit one per CU, rising with the blocks per CU.
   int bestS = 1;
   double best = 1e30;
   for (int S = 1; S <= std::min(G, 32); S++) {
@@ -1215,13 +1211,8 @@ Plan make_plan(const GemmArgs &a, int bits, int ptype) {
     if (S > 1 && ((size_t)tiles * S * BM * BN > a.ws_floats || tiles > a.cnt_words)) break;
     const int blocks = tiles * S;
     const int rounds = (blocks + slots - 1) / slots;
-    double cost;
-    if (large) {
-      cost = rounds * (gps + 3) + (S > 1 ? 2 : 0);
-    } else {
-      const double per_cu = (double)blocks / std::max(1, a.n_cu);
-      cost = 0.953 * S - 1.044 * gps * rounds + 1.462 * gps * std::max(1.0, per_cu);
-    }
+    const double per_cu = (double)blocks / std::max(1, a.n_cu);
+    const double cost = 0.953 * S - 1.044 * gps * rounds + 1.462 * gps * std::max(1.0, per_cu);
     if (cost < best) {
       best = cost;
       bestS = S;
@@ -1244,7 +1235,6 @@ hipError_t set_cfg_attr() {
 
 template <int BITS, int PT, int EPI, int KVT, int TM, int TN>
 hipError_t launch_cfg(const GemmArgs &a, const Plan &p, hipStream_t s) {
-  // large tiles (one block per CU) run with copier waves; small tiles keep two blocks per CU
   constexpr bool prod = true;
   auto *fn = gemm_kernel<BITS, PT, EPI, KVT, TM, TN, kStages, prod>;
   constexpr size_t lds = lds_bytes<BITS, PT, TM, TN>();
@@ -1259,21 +1249,15 @@ hipError_t init_bits() {
     if (e == hipSuccess) e = x;
   };
   chk(set_cfg_attr<BITS, PT, kEpiStore, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiStore, 0, 2, 2>());
   chk(set_cfg_attr<BITS, PT, kEpiResid, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiResid, 0, 2, 2>());
   chk(set_cfg_attr<BITS, PT, kEpiGelu, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiGelu, 0, 2, 2>());
   chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvBf16, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvBf16, 2, 2>());
   chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvF32, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvF32, 2, 2>());
   return e;
 }
 
 template <int BITS, int PT, int EPI, int KVT>
 hipError_t launch_epi(const GemmArgs &a, const Plan &p, hipStream_t s) {
-  if (p.TM == 2) return launch_cfg<BITS, PT, EPI, KVT, 2, 2>(a, p, s);
   return launch_cfg<BITS, PT, EPI, KVT, 1, 1>(a, p, s);
 }
 

@@ -1,0 +1,778 @@
+// Multi-row products and causal attention of the decoder (prefill of long prompts, replay,
+// all-row forward) on operands kept in MFMA fragment order (frag.h).
+//
+// y[M][N] = x[M][K] Wdeq^T + bias contracts fp16 hi/lo activation fragments (~22 bits) with
+// the codes, exact in fp16 as q - 128 (8-bit) or q - 8 (4-bit), two products on
+// v_mfma_f32_32x32x16_f16 per K step, and folds each 64-group's scale into an fp32
+// accumulator: acc += s[g, n] P.  The groups' bias term, sum_g b'[n, g] sum_{k in g} x[m, k]
+// with b' = b + 128 s (or 8 s), is itself a product over G more K values: the activation
+// planes carry the group sums as further K steps, the weights' b' planes hold the other
+// operand (both hi/lo, three products).
+//
+// Activation planes ("rows"): per 32-row block, K / 16 steps, then ceil(G / 16) steps of group
+// sums.  Inside a 64-group the K order is permuted so that a lane's codes of two steps are one
+// contiguous read: chunk c8 (8 values) is half (c8 >> 1) & 1 of step 2 (c8 >> 2) + (c8 & 1).
+// The codes are held a second time in that order (per 32 columns and group, two 32-value
+// halves of 64 lanes x 16 codes): a fragment load is then one coalesced run, where the
+// row-major codes touch 32 rows (886 x 5120 x 1280: 32.7 against 46.7 us).
+#include "frag.h"
+#include "kernels.h"
+
+#include <algorithm>
+
+namespace itts {
+
+namespace {
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// piece of (row, chunk c of K): hi plane; lo 64 pieces on.  ns: steps a row block holds.
+__device__ __forceinline__ size_t rows_piece(int row, int c, int ns) {
+  const int step = (c >> 3) * 4 + ((c >> 2) & 1) * 2 + (c & 1);
+  return (((size_t)(row >> 5) * ns + step) * 2) * 64 + (size_t)(((c >> 1) & 1) * 32 + (row & 31));
+}
+// the group sum of group g: element of the extra steps
+__device__ __forceinline__ void put_group_sum(u32x4 *o, int row, int g, int nk, int ns, float v) {
+  uint32_t h, l;
+  split_f16(v, h, l);
+  uint16_t *p = reinterpret_cast<uint16_t *>(o + (((size_t)(row >> 5) * ns + nk + (g >> 4)) * 2) * 64 +
+                                             (size_t)(((g >> 3) & 1) * 32 + (row & 31))) +
+                (g & 7);
+  p[0] = (uint16_t)h;
+  p[64 * 8] = (uint16_t)l;
+}
+
+__device__ __forceinline__ float sum8(float v) {  // over eight consecutive lanes
+  v += dpp_pair<0xB1>(v);
+  v += dpp_pair<0x4E>(v);
+  return v + dpp_pair<0x141>(v);
+}
+
+// LayerNorm of rows (a second one with w2; none without w) as planes and group sums; one wave a row.
+__global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const float *w, const float *b, const float *w2,
+                                                       const float *b2, int d, u32x4 *out) {
+  const int row = blockIdx.x, lane = threadIdx.x, nc = d / 8, nk = d / 16, ns = nk + (d / 64 + 15) / 16;
+  const float *xr = x + (size_t)row * d;
+  // mean and 1 / std over f(element) (the row is read again for each pass, from the caches)
+  auto stats = [&](auto f, float &mean, float &rstd) __attribute__((always_inline)) {
+    float s = 0.0f;
+    for (int i = lane; i < d; i += 64) s += f(i);
+    mean = wave64_sum_dpp(s) / (float)d;
+    float q = 0.0f;
+    for (int i = lane; i < d; i += 64) {
+      const float e = f(i) - mean;
+      q += e * e;
+    }
+    rstd = 1.0f / sqrtf(wave64_sum_dpp(q) / (float)d + 1e-5f);
+  };
+  float m1 = 0.0f, r1 = 1.0f, m2 = 0.0f, r2 = 1.0f;
+  auto f1 = [&](int i) __attribute__((always_inline)) { return w ? (xr[i] - m1) * r1 * w[i] + b[i] : xr[i]; };
+  if (w) stats([&](int i) __attribute__((always_inline)) { return xr[i]; }, m1, r1);
+  if (w2) stats(f1, m2, r2);
+  for (int c = lane; c < (nc + 63) / 64 * 64; c += 64) {
+    float v[8], g = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int i = min(c, nc - 1) * 8 + j;
+      float y = f1(i);
+      if (w2) y = (y - m2) * r2 * w2[i] + b2[i];
+      v[j] = y;
+      g += y;
+    }
+    g = sum8(g);
+    if (c >= nc) continue;
+    u32x4 hi, lo;
+    split8(v, hi, lo);
+    const size_t p = rows_piece(row, c, ns);
+    out[p] = hi;
+    out[p + 64] = lo;
+    if ((c & 7) == 0) put_group_sum(out, row, c >> 3, nk, ns, g);
+  }
+}
+
+// ---- weights ----------------------------------------------------------------------------
+// scale [G][ldn] fp32 (columns past N zero) and b' = b + off s as fragment planes of G values
+template <int PT>
+__global__ __launch_bounds__(256) void rows_params_kernel(const void *params, int N, int G, int ldn, float off,
+                                                          float *scale, u32x4 *bw) {
+  const int nx = (G + 15) / 16;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long)ldn * nx * 2) return;
+  const int n = (int)(i % ldn), g8 = (int)(i / ldn);
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const int g = g8 * 8 + j;
+    float2 sb = make_float2(0.0f, 0.0f);
+    if (n < N && g < G) sb = load_param<PT>(params, (size_t)n * G + g);
+    if (g < G) scale[(size_t)g * ldn + n] = sb.x;
+    v[j] = fmaf(off, sb.x, sb.y);
+  }
+  u32x4 hi, lo;
+  split8(v, hi, lo);
+  const size_t p = frag_piece(n, g8, nx);
+  bw[p] = hi;
+  bw[p + 64] = lo;
+}
+
+// codes in fragment order: lane's 16 codes (BITS * 2 bytes) of (32 columns, group, half), zero past N
+template <int BITS>
+__global__ __launch_bounds__(256) void rows_codes_kernel(const uint8_t *codes, int N, int K, long n, uint8_t *out) {
+  constexpr int B = BITS * 2;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int lane = (int)(i & 63), kp = (int)((i >> 6) & 1), G = K / 64;
+  const long r = i >> 7;
+  const int g = (int)(r % G), col = (int)(r / G) * 32 + (lane & 31);
+  uint32_t w[B / 4];
+#pragma unroll
+  for (int j = 0; j < B / 4; j++) w[j] = 0u;
+  if (col < N) {
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(codes + (size_t)col * (K * BITS / 8) + g * (BITS * 8) +
+                                                           kp * (BITS * 4) + (lane >> 5) * B);
+#pragma unroll
+    for (int j = 0; j < B / 4; j++) w[j] = p[j];
+  }
+  uint32_t *o = reinterpret_cast<uint32_t *>(out + (size_t)i * B);
+#pragma unroll
+  for (int j = 0; j < B / 4; j++) o[j] = w[j];
+}
+
+// ---- the product ------------------------------------------------------------------------
+// Block: one tile of BM = 32 TM rows x 64 columns by KS waves that split the K groups, their
+// partial tiles added through LDS (two halves of the waves at a time).  A wave keeps CH
+// groups of activation fragments, codes and scales in flight.
+template <int TM_, int KS_, int CH_>
+struct RmCfg {
+  static constexpr int TM = TM_, TN = 2, KS = KS_, CH = CH_;
+  static constexpr int BM = 32 * TM, BN = 64, LD = BN + 4, NT = 64 * KS, KL = KS > 2 ? KS / 2 : KS;
+  static constexpr size_t LDS = sizeof(float) * (KL * BM * LD + 2 * BM);
+  static_assert(LDS <= 65536, "dynamic LDS of a plain launch");
+};
+
+// eight 8-bit codes (two words) or 4-bit codes (one word) as fp16 q - 128 / q - 8
+template <int BITS>
+__device__ __forceinline__ f16x8 codes_f16(uint32_t w0, uint32_t w1) {
+  u32x4 r;
+  if constexpr (BITS == 8) {
+    // bytes q and 0x64 make the half 1024 + q
+    r[0] = __builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u);
+    r[1] = __builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u);
+    r[2] = __builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u);
+    r[3] = __builtin_amdgcn_perm(0x64646464u, w1, 0x04030402u);
+  } else {
+    const uint32_t e = w0 & 0x0f0f0f0fu, o = (w0 >> 4) & 0x0f0f0f0fu;
+    r[0] = __builtin_amdgcn_perm(o, e, 0x0c040c00u) | 0x64006400u;
+    r[1] = __builtin_amdgcn_perm(o, e, 0x0c050c01u) | 0x64006400u;
+    r[2] = __builtin_amdgcn_perm(o, e, 0x0c060c02u) | 0x64006400u;
+    r[3] = __builtin_amdgcn_perm(o, e, 0x0c070c03u) | 0x64006400u;
+  }
+  const _Float16 z = BITS == 8 ? (_Float16)1152.0f : (_Float16)1032.0f;
+  const f16x2 zz = {z, z};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t w = r[i];  // (a bit cast of a vector's element reads its first)
+    r[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, w) - zz);
+  }
+  return __builtin_bit_cast(f16x8, r);
+}
+
+template <int BITS, int EPI, int KVT, class C>
+__global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(RowsMm a) {
+  constexpr int TM = C::TM, TN = C::TN, KS = C::KS, KL = C::KL, BM = C::BM, BN = C::BN, LD = C::LD, NT = C::NT;
+  constexpr int CH = C::CH, CW = BITS == 8 ? 4 : 2;  // words of a lane's codes per 32 K values
+  extern __shared__ __attribute__((aligned(16))) float red[];
+  float2 *row_stat = reinterpret_cast<float2 *>(red + KL * BM * LD);
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r31 = lane & 31;
+  const int kq = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // block -> tile: XCD x takes every gm-th row tile and every gn-th column tile
+  const int gn = 8 / a.gm, x = blockIdx.x & 7, jb = blockIdx.x >> 3, pn = (a.nN + gn - 1) / gn;
+  const int tm = jb / pn * a.gm + x % a.gm, tn = jb % pn * gn + x / a.gm;
+  if (tm >= a.nM || tn >= a.nN) return;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int G = a.K / 64, nk = a.K / 16, nx = (G + 15) / 16, ns = nk + nx;
+  const int g0 = G * kq / KS, g1 = G * (kq + 1) / KS;
+
+  // wave-uniform bases with 32-bit lane offsets (registers, not 64-bit addresses, are short here)
+  const u32x4 *ab = reinterpret_cast<const u32x4 *>(a.x) + ((size_t)(m0 >> 5) * ns) * 128;
+  const uint8_t *cb = reinterpret_cast<const uint8_t *>(a.codes) + (size_t)(n0 >> 5) * G * (BITS * 256);
+
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+  struct Codes {
+    uint32_t q[TN][2][CW];
+    float s[TN];
+  };
+  u32x4 fa[CH][4][TM][2];
+  Codes cq[CH];
+  auto load_a = [&](int g, int s4, u32x4(&f)[TM][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const u32x4 *p = ab + ((size_t)i * ns + min(g, g1 - 1) * 4 + s4) * 128;
+      f[i][0] = p[lane];
+      f[i][1] = p[lane + 64];
+    }
+  };
+  auto load_c = [&](int g, Codes &c) __attribute__((always_inline)) {
+    const int gc = min(g, g1 - 1);
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+#pragma unroll
+      for (int kp = 0; kp < 2; kp++) {
+        const uint8_t *p = cb + (((size_t)j * G + gc) * 2 + kp) * (BITS * 128) + lane * (BITS * 2);
+        if constexpr (BITS == 8) {
+          const u32x4 v = *reinterpret_cast<const u32x4 *>(p);
+#pragma unroll
+          for (int w = 0; w < 4; w++) c.q[j][kp][w] = v[w];
+        } else {
+          const u32x2 v = *reinterpret_cast<const u32x2 *>(p);
+#pragma unroll
+          for (int w = 0; w < 2; w++) c.q[j][kp][w] = v[w];
+        }
+      }
+      c.s[j] = (a.scale + (size_t)gc * a.ldn + n0 + j * 32)[r31];
+    }
+  };
+  auto load_rings = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < CH; u++) {
+      load_c(g0 + u, cq[u]);
+#pragma unroll
+      for (int s4 = 0; s4 < 4; s4++) load_a(g0 + u, s4, fa[u][s4]);
+    }
+  };
+  // the bias term's steps first (their loads go out ahead of the rings')
+  const int x0 = nx * kq / KS, x1 = nx * (kq + 1) / KS;
+  for (int kx = x0; kx < x1; kx++) {
+    u32x4 xa[TM][2], xb[TN][2];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const u32x4 *p = ab + ((size_t)i * ns + nk + kx) * 128;
+      xa[i][0] = p[lane];
+      xa[i][1] = p[lane + 64];
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const u32x4 *p = reinterpret_cast<const u32x4 *>(a.bw) + ((size_t)((n0 >> 5) + j) * nx + kx) * 128;
+      xb[j][0] = p[lane];
+      xb[j][1] = p[lane + 64];
+    }
+    if (kx == x0 && g0 < g1) {
+      load_rings();
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, xa[i][p == 2]), __builtin_bit_cast(f16x8, xb[j][p == 1]),
+                                  acc[i][j], 0, 0, 0);
+  }
+  if (x0 == x1 && g0 < g1) {
+    load_rings();
+  }
+  // What the epilogue needs, loaded here so that its latency passes under the K loop.  A
+  // thread's items are the tile's rows tid / 8 + i NT / 8 at columns 8 (tid & 7) .. +7.
+  // Folded LayerNorm input: LPR lanes a row hold its groups' (mean, sum of squared
+  // deviations), combined after the loop.
+  constexpr bool kFold = EPI == kEpiQKV || EPI == kEpiGelu;
+  constexpr int LPR = NT / BM, SG = 32 / LPR, IT = (BM * 8 + NT - 1) / NT;
+  const bool fin = kFold && a.st != nullptr;
+  const int ic = n0 + (tid & 7) * 8;
+  float2 sv[kFold ? SG : 1];
+  if constexpr (kFold) {
+    const float2 *st = a.st + (size_t)min(m0 + tid / LPR, a.M - 1) * G;
+#pragma unroll
+    for (int i = 0; i < SG; i++) {
+      const int gg = tid % LPR + i * LPR;
+      sv[i] = fin && gg < G ? st[gg] : make_float2(0.0f, 0.0f);
+    }
+  }
+  float cadd[8], cG[kFold ? 8 : 1], gam[EPI == kEpiResid ? 8 : 1];
+  float4 old[EPI == kEpiResid ? IT : 1][2];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const int n = min(ic + e, a.N - 1);
+    cadd[e] = (fin ? a.fc : a.bias)[n];
+    if constexpr (kFold) cG[e] = fin ? a.fG[n] : 0.0f;
+    if constexpr (EPI == kEpiResid) gam[e] = a.o ? a.gamma[n] : 0.0f;
+  }
+  if constexpr (EPI == kEpiResid) {
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const float4 *o = reinterpret_cast<const float4 *>(a.y + (size_t)min(m0 + min((tid >> 3) + i * (NT / 8), BM - 1), a.M - 1) * a.N + ic);
+      old[i][0] = o[0];
+      old[i][1] = o[1];
+    }
+  }
+  auto group = [&](int g, u32x4(&f)[4][TM][2], Codes &c) __attribute__((always_inline)) {
+    floatx16 P[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) P[i][j][e] = 0.0f;
+#pragma unroll
+    for (int s4 = 0; s4 < 4; s4++) {
+      f16x8 b[TN];
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const uint32_t *q = c.q[j][s4 >> 1];
+        b[j] = BITS == 8 ? codes_f16<BITS>(q[(s4 & 1) * 2], q[(s4 & 1) * 2 + (BITS == 8 ? 1 : 0)])
+                         : codes_f16<BITS>(q[s4 & 1], 0);
+      }
+#pragma unroll
+      for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++) P[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, f[s4][i][p]), b[j], P[i][j], 0, 0, 0);
+      load_a(g + CH, s4, f[s4]);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const float s = c.s[j];
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(s, P[i][j][e], acc[i][j][e]);
+    }
+    load_c(g + CH, c);
+  };
+  int g = g0;
+  for (; g + CH <= g1; g += CH) {
+#pragma unroll
+    for (int u = 0; u < CH; u++) group(g + u, fa[u], cq[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < CH - 1; u++)
+    if (g + u < g1) group(g + u, fa[u], cq[u]);
+
+  if constexpr (kFold) {
+    if (fin) {
+      auto lanes_sum = [&](float v) __attribute__((always_inline)) {
+        v += dpp_pair<0xB1>(v);
+        v += dpp_pair<0x4E>(v);
+        if constexpr (LPR >= 8) v += dpp_pair<0x141>(v);
+        if constexpr (LPR >= 16) v += dpp_pair<0x140>(v);
+        return v;
+      };
+      float sm = 0.0f;
+#pragma unroll
+      for (int i = 0; i < SG; i++) sm += sv[i].x;
+      const float mean = lanes_sum(sm) / (float)G;
+      float m2 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < SG; i++)
+        if (tid % LPR + i * LPR < G) m2 += sv[i].y + 64.0f * ((sv[i].x - mean) * (sv[i].x - mean));
+      m2 = lanes_sum(m2);
+      if (tid % LPR == 0) row_stat[tid / LPR] = make_float2(mean, 1.0f / sqrtf(m2 / (float)a.K + 1e-5f));
+    }
+  }
+  // the tile to LDS: the upper half of the waves adds its partials to the lower half's
+  auto part = [&](int k) __attribute__((always_inline)) { return red + (size_t)k * BM * LD; };
+  auto place = [&](int i, int j, int e) __attribute__((always_inline)) {
+    return (i * 32 + (e >> 2) * 8 + h * 4 + (e & 3)) * LD + j * 32 + r31;
+  };
+  if constexpr (KS > KL) {
+    if (kq >= KL) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) part(kq - KL)[place(i, j, e)] = acc[i][j][e];
+    }
+    __syncthreads();
+  }
+  if (kq < KL) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          float *t = part(kq) + place(i, j, e);
+          *t = KS > KL ? acc[i][j][e] + *t : acc[i][j][e];
+        }
+  }
+  __syncthreads();
+
+  // eight columns of a tile row: the parts added, then the folded LayerNorm or the bias
+  auto tile8 = [&](int row, int col, float v[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      float4 s = *reinterpret_cast<const float4 *>(red + (size_t)row * LD + col + 4 * q);
+#pragma unroll
+      for (int k = 1; k < KL; k++) {
+        const float4 p = *reinterpret_cast<const float4 *>(red + ((size_t)k * BM + row) * LD + col + 4 * q);
+        s.x += p.x, s.y += p.y, s.z += p.z, s.w += p.w;
+      }
+      v[4 * q] = s.x, v[4 * q + 1] = s.y, v[4 * q + 2] = s.z, v[4 * q + 3] = s.w;
+    }
+    if constexpr (kFold) {
+      if (fin) {
+        const float2 rs = row_stat[row];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = rs.y * (v[e] - rs.x * cG[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] += cadd[e];
+  };
+  constexpr int ITEMS = BM * 8;
+  if constexpr (EPI == kEpiStore) {
+    for (int q = tid; q < ITEMS; q += NT) {
+      const int c = q & 7, row = q >> 3, r = m0 + row, n = n0 + c * 8;
+      if (r >= a.M || n >= a.N) continue;
+      float v[8];
+      tile8(row, c * 8, v);
+      float *o = a.y + (size_t)r * a.N + n;
+      if (a.N % 4 == 0 && n + 8 <= a.N) {
+        reinterpret_cast<float4 *>(o)[0] = make_float4(v[0], v[1], v[2], v[3]);
+        reinterpret_cast<float4 *>(o)[1] = make_float4(v[4], v[5], v[6], v[7]);
+      } else {
+        for (int e = 0; e < 8 && n + e < a.N; e++) o[e] = v[e];
+      }
+    }
+  } else if constexpr (EPI == kEpiResid) {
+    // x = y + v; with the fold-out, gamma x as planes, its group sum, and the group's mean and
+    // sum of squared deviations (eight lanes hold a row's 64 columns)
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const int q = tid + i * NT, c = q & 7, row = q >> 3, r = m0 + row, n = n0 + c * 8;
+      if (q >= ITEMS) break;  // whole waves
+      const bool live = r < a.M;
+      float v[8];
+      tile8(row, c * 8, v);
+      float4 *o = reinterpret_cast<float4 *>(a.y + (size_t)min(r, a.M - 1) * a.N + n);
+      const float4 p = old[i][0], t = old[i][1];
+      const float yv[8] = {p.x, p.y, p.z, p.w, t.x, t.y, t.z, t.w};
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[e] += yv[e];
+      if (live) {
+        o[0] = make_float4(v[0], v[1], v[2], v[3]);
+        o[1] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+      if (!a.o) continue;
+      const float mean = sum8(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]))) / 64.0f;
+      float m2 = 0.0f, gs = 0.0f, y[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float d = v[e] - mean;
+        m2 += d * d;
+        y[e] = gam[e] * v[e];
+        gs += y[e];
+      }
+      m2 = sum8(m2);
+      gs = sum8(gs);
+      if (!live) continue;
+      const int onk = a.N / 16, ons = onk + (a.N / 64 + 15) / 16;
+      u32x4 hi, lo;
+      split8(y, hi, lo);
+      u32x4 *out = reinterpret_cast<u32x4 *>(a.o);
+      const size_t pc = rows_piece(r, n >> 3, ons);
+      out[pc] = hi;
+      out[pc + 64] = lo;
+      if (c == 0) {
+        put_group_sum(out, r, n >> 6, onk, ons, gs);
+        a.so[(size_t)r * (a.N / 64) + (n >> 6)] = make_float2(mean, m2);
+      }
+    }
+  } else if constexpr (EPI == kEpiGelu) {
+    for (int q = tid; q < ITEMS; q += NT) {
+      const int c = q & 7, row = q >> 3, r = m0 + row, n = n0 + c * 8;
+      float v[8], gs = 0.0f;
+      tile8(row, c * 8, v);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        v[e] = gelu_tanh_exp(v[e]);
+        gs += v[e];
+      }
+      gs = sum8(gs);
+      if (r >= a.M) continue;
+      const int onk = a.N / 16, ons = onk + (a.N / 64 + 15) / 16;
+      u32x4 hi, lo;
+      split8(v, hi, lo);
+      u32x4 *out = reinterpret_cast<u32x4 *>(a.o);
+      const size_t pc = rows_piece(r, n >> 3, ons);
+      out[pc] = hi;
+      out[pc + 64] = lo;
+      if (c == 0) put_group_sum(out, r, n >> 6, onk, ons, gs);
+    }
+  } else {
+    // the 64 columns are one head of q, k or v: the attention's fragments (q scaled by
+    // log2(e) / 8; rows past M, up to whole tiles of 64 keys, zero), and the cache rows
+    constexpr int NP = KVT == kKvBf16 ? 1 : 2;
+    const int d = a.N / 3, which = n0 / d, head = (n0 - which * d) / 64, Tt = (a.M + 63) / 64 * 2;
+    auto round_kv = [&](float v[8]) __attribute__((always_inline)) {
+      if constexpr (KVT == kKvBf16) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = bf16_bits_to_float(float_to_bf16_bits(v[e]));
+      }
+    };
+    u32x4 *kvf = reinterpret_cast<u32x4 *>(a.kvf) + (size_t)head * Tt * flash_tile_pieces(NP);
+    for (int q = tid; q < ITEMS; q += NT) {
+      const int c = q & 7, row = q >> 3, t = m0 + row;
+      float v[8];
+      tile8(row, c * 8, v);
+      if (which == 0) {
+        if (t >= Tt * 32) continue;
+        if (a.q_out && t < a.M) {
+          float4 *o = reinterpret_cast<float4 *>(a.q_out + (size_t)t * d + head * 64 + c * 8);
+          o[0] = make_float4(v[0], v[1], v[2], v[3]);
+          o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = t < a.M ? v[e] * (0.125f * 1.4426950408889634f) : 0.0f;
+        u32x4 hi, lo;
+        split8(v, hi, lo);
+        u32x4 *dst = reinterpret_cast<u32x4 *>(a.qf) + (((size_t)head * Tt + (t >> 5)) * 4 + (c >> 1)) * 128 +
+                     (c & 1) * 32 + (t & 31);
+        dst[0] = hi;
+        dst[64] = lo;
+        continue;
+      }
+      round_kv(v);
+      void *cache = which == 1 ? a.kc : a.vc;
+      if (cache && t < a.M) {
+        const size_t ci = ((size_t)head * a.max_seq + t) * 64 + c * 8;
+        if constexpr (KVT == kKvBf16) {
+          u32x4 w;
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            w[e] = (__float_as_uint(v[2 * e]) >> 16) | (__float_as_uint(v[2 * e + 1]) & 0xffff0000u);
+          *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(cache) + ci) = w;
+        } else {
+          float4 *o = reinterpret_cast<float4 *>(static_cast<float *>(cache) + ci);
+          o[0] = make_float4(v[0], v[1], v[2], v[3]);
+          o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+      }
+      if (which == 1 && t < Tt * 32) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = t < a.M ? v[e] : 0.0f;
+        u32x4 hi, lo;
+        split8(v, hi, lo);
+        u32x4 *dst = kvf + (size_t)(t >> 5) * flash_tile_pieces(NP) + (c >> 1) * NP * 64 + (c & 1) * 32 + (t & 31);
+        dst[0] = hi;
+        if constexpr (NP == 2) dst[64] = lo;
+      }
+    }
+    if (which == 2) {
+      // dim e, key positions 8 k8 .. +7: keys 16 s + 4 hh + {0..3, 8..11}
+      // (e is the same for a thread's items)
+      const float vG = fin ? a.fG[n0 + (tid & 63)] : 0.0f, vadd = (fin ? a.fc : a.bias)[n0 + (tid & 63)];
+      for (int q = tid; q < ITEMS; q += NT) {
+        const int e = q & 63, k8 = q >> 6, rb = (k8 >> 1) * 16 + (k8 & 1) * 4, t = m0 + rb;
+        if (t >= Tt * 32) continue;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const int row = rb + (j >> 2) * 8 + (j & 3);
+          float s = red[(size_t)row * LD + e];
+#pragma unroll
+          for (int k = 1; k < KL; k++) s += red[((size_t)k * BM + row) * LD + e];
+          if (fin) s = row_stat[row].y * (s - row_stat[row].x * vG);
+          v[j] = s + vadd;
+        }
+        round_kv(v);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = m0 + rb + (j >> 2) * 8 + (j & 3) < a.M ? v[j] : 0.0f;
+        u32x4 hi, lo;
+        split8(v, hi, lo);
+        u32x4 *dst = kvf + (size_t)(t >> 5) * flash_tile_pieces(NP) +
+                     (4 + (e >> 5) * 2 + ((t >> 4) & 1)) * NP * 64 + (k8 & 1) * 32 + (e & 31);
+        dst[0] = hi;
+        if constexpr (NP == 2) dst[64] = lo;
+      }
+    }
+  }
+}
+
+// ---- causal attention -------------------------------------------------------------------
+// Block: 32 query rows of one head, its four waves on a quarter of the key tiles each.  Row t
+// attends to keys kstart[t] (or 0) .. t; order lists the query tiles, most keys first.
+template <int NP>
+__global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, const u32x4 *kvf, int M, const int *kstart,
+                                                           const int *order, u32x4 *out) {
+  __shared__ float buf[4 * 2112];
+  const int lane = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head = blockIdx.x, d = gridDim.x * 64, Tt = (M + 63) / 64 * 2;
+  const int qt = order ? order[blockIdx.y] : (int)(gridDim.y - 1 - blockIdx.y);
+  const int t = qt * 32 + (lane & 31), tc = min(t, M - 1);
+  const int ks = kstart ? kstart[tc] : 0;
+  f16x8 qh[4], ql[4];
+  const u32x4 *qp = qf + (((size_t)head * Tt + qt) * 4) * 128 + lane;
+#pragma unroll
+  for (int kk = 0; kk < 4; kk++) {
+    qh[kk] = __builtin_bit_cast(f16x8, qp[kk * 128]);
+    ql[kk] = __builtin_bit_cast(f16x8, qp[kk * 128 + 64]);
+  }
+  FlashState st;
+  flash_init(st);
+  const int tb = kstart ? kstart[qt * 32] / 32 : 0, nt = qt + 1 - tb;
+  const int kmax = kstart ? kstart[min(qt * 32 + 31, M - 1)] : 0;
+  const int per = (nt + 3) / 4, t0 = tb + g * per, t1 = min(qt + 1, t0 + per);
+  auto mask = [&](int kt, floatx16 &S) __attribute__((always_inline)) {
+    if (kt == qt || kt * 32 < kmax) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int key = kt * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
+        if (key > tc || key < ks) S[i] = -INFINITY;
+      }
+    }
+  };
+  flash_tiles<NP>(kvf + (size_t)head * Tt * flash_tile_pieces(NP) + lane, t0, t1, qh, ql, mask, st);
+  flash_merge<4>(st, buf, g, lane);
+  if (g != 0) return;
+  const float inv = 1.0f / st.l;
+  const int nk = d / 16, ns = nk + (d / 64 + 15) / 16;
+  float gs = 0.0f;
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      st.O[dt][i] *= inv;
+      gs += st.O[dt][i];
+    }
+  gs += other_half(gs, lane);
+  if (t >= M) return;
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int a8 = 0; a8 < 4; a8++) {
+      u32x2 hi, lo;
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        uint32_t hw, lw;
+        split_f16x2(st.O[dt][a8 * 4 + 2 * j], st.O[dt][a8 * 4 + 2 * j + 1], hw, lw);
+        hi[j] = hw;
+        lo[j] = lw;
+      }
+      u32x2 *p = reinterpret_cast<u32x2 *>(out + rows_piece(t, head * 8 + dt * 4 + a8, ns)) + (lane >> 5);
+      p[0] = hi;
+      p[128] = lo;
+    }
+  if (lane < 32) put_group_sum(out, t, head, nk, ns, gs);
+}
+
+// (row parts of the XCDs: the split with the fewest operand bytes read by each)
+int xcd_rows(int nM, int nN, double a_tile, double w_tile) {
+  int best = 1;
+  double least = 1e300;
+  for (int gm = 1; gm <= 8; gm *= 2) {
+    const int gn = 8 / gm, pm = (nM + gm - 1) / gm, pn = (nN + gn - 1) / gn;
+    double bytes = pm * a_tile + pn * w_tile;
+    if (bytes > 3e6)
+      bytes = std::max(bytes, pm * pn / 64.0 * (std::max(1.0, 64.0 / pn) * a_tile + std::min(pn, 64) * w_tile));
+    if (bytes < least) least = bytes, best = gm;
+  }
+  return best;
+}
+
+template <int BITS, int EPI, int KVT, class C>
+hipError_t run(RowsMm a, hipStream_t s) {
+  a.nM = (a.M + C::BM - 1) / C::BM;
+  a.nN = (a.N + C::BN - 1) / C::BN;
+  a.gm = xcd_rows(a.nM, a.nN, 4.0 * C::BM * a.K, (double)C::BN * a.K * BITS / 8);
+  const int gn = 8 / a.gm, blocks = 8 * ((a.nM + a.gm - 1) / a.gm) * ((a.nN + gn - 1) / gn);
+  hipLaunchKernelGGL((rows_mm_kernel<BITS, EPI, KVT, C>), dim3(blocks), dim3(C::NT), C::LDS, s, a);
+  return hipGetLastError();
+}
+
+// 32 x 64 tiles by four waves; by eight where K is long and the tiles few, 64 x 64 tiles where K is
+// long and the tiles many.  M x N x K in us, 32 x 64 by four / by eight / 64 x 64: 35 x 1280 x 1280
+// 7.2 / 7.5 / 10.1, 35 x 1280 x 5120 16.0 / 14.8 / 22.6, 235 x 1280 x 5120 17.0 / 15.9 / 23.5, 235 x
+// 5120 x 1280 13.5 / 18.9 / 16.4, 886 x 5120 x 1280 32.7 (355 TFLOP/s) / 52.5 / 34.4, 886 x 1280 x
+// 5120 34.5 / 44.3 / 42.3, 2188 x 5120 x 1280 72.5 / 122 / 72.4, 2188 x 1280 x 5120 69.7 / 88.4 / 62.5
+// (459 TFLOP/s, 918 of fp16 products).  (Two groups of codes in flight instead of one: 10-40 %
+// slower, fewer waves in flight.)
+using RmSmall = RmCfg<1, 4, 1>;
+using RmLong = RmCfg<1, 8, 1>;
+using RmLarge = RmCfg<2, 4, 1>;
+
+template <int BITS, int EPI, int KVT>
+hipError_t pick(const RowsMm &a, hipStream_t s) {
+  const long tn = (a.N + 63) / 64, t32 = (a.M + 31) / 32 * tn, t64 = (a.M + 63) / 64 * tn;
+  if (a.K >= 4096 && 4 * t32 <= 5L * a.n_cu) return run<BITS, EPI, KVT, RmLong>(a, s);
+  if (a.K >= 4096 && t64 >= 2L * a.n_cu) return run<BITS, EPI, KVT, RmLarge>(a, s);
+  return run<BITS, EPI, KVT, RmSmall>(a, s);
+}
+
+template <int BITS>
+hipError_t dispatch(const RowsMm &a, int epi, int kvt, hipStream_t s) {
+  switch (epi) {
+    case kEpiStore: return pick<BITS, kEpiStore, 0>(a, s);
+    case kEpiResid: return a.N % 64 == 0 ? pick<BITS, kEpiResid, 0>(a, s) : hipErrorInvalidValue;
+    case kEpiGelu: return a.N % 64 == 0 && a.o ? pick<BITS, kEpiGelu, 0>(a, s) : hipErrorInvalidValue;
+    case kEpiQKV:
+      if (a.N % 192 != 0 || !a.qf || !a.kvf) return hipErrorInvalidValue;
+      return kvt == kKvBf16 ? pick<BITS, kEpiQKV, kKvBf16>(a, s) : pick<BITS, kEpiQKV, kKvF32>(a, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+size_t rows_planes_pieces(int M, int K) { return (size_t)((M + 63) / 64 * 2) * (K / 16 + (K / 64 + 15) / 16) * 128; }
+size_t rows_q_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * 4 * 128; }
+size_t rows_kv_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * flash_tile_pieces(2); }
+int rows_ldn(int N) { return (N + 63) / 64 * 64; }
+size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64) * rows_ldn(N); }
+size_t rows_codes_bytes(int N, int K, int bits) { return (size_t)rows_ldn(N) * K * bits / 8; }
+size_t rows_bias_pieces(int N, int K) { return (size_t)(rows_ldn(N) / 32) * ((K / 64 + 15) / 16) * 128; }
+
+hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, hipStream_t s) {
+  const long nc = (long)(rows_ldn(ql.N) / 32) * (ql.K / 64) * 128;
+  const dim3 cg((unsigned)((nc + 255) / 256));
+  uint8_t *co = reinterpret_cast<uint8_t *>(codes);
+  if (bits == 8) hipLaunchKernelGGL(rows_codes_kernel<8>, cg, dim3(256), 0, s, ql.codes, ql.N, ql.K, nc, co);
+  else hipLaunchKernelGGL(rows_codes_kernel<4>, cg, dim3(256), 0, s, ql.codes, ql.N, ql.K, nc, co);
+  const int G = ql.K / 64, ldn = rows_ldn(ql.N);
+  const long n = (long)ldn * ((G + 15) / 16) * 2;
+  const float off = bits == 8 ? 128.0f : 8.0f;
+  const dim3 grid((unsigned)((n + 255) / 256));
+  if (ptype == kParamF32)
+    hipLaunchKernelGGL(rows_params_kernel<kParamF32>, grid, dim3(256), 0, s, ql.params, ql.N, G, ldn, off, scale,
+                       reinterpret_cast<u32x4 *>(bw));
+  else
+    hipLaunchKernelGGL(rows_params_kernel<kParamF16>, grid, dim3(256), 0, s, ql.params, ql.N, G, ldn, off, scale,
+                       reinterpret_cast<u32x4 *>(bw));
+  return hipGetLastError();
+}
+
+hipError_t rows_ln(const float *x, const float *w, const float *b, const float *w2, const float *b2, int M, int d,
+                   uint4 *out, hipStream_t s) {
+  hipLaunchKernelGGL(ln_planes_kernel, dim3(M), dim3(64), 0, s, x, w, b, w2, b2, d, reinterpret_cast<u32x4 *>(out));
+  return hipGetLastError();
+}
+
+hipError_t rows_mm(const RowsMm &a, int bits, int epi, int kvt, hipStream_t s) {
+  if (a.M < 1 || a.N < 1 || a.K < 64 || a.K % 64 != 0 || !a.x || !a.codes || !a.scale || !a.bw || !a.bias ||
+      (a.st && (a.K > 2048 || !a.fG || !a.fc)))
+    return hipErrorInvalidValue;
+  return bits == 8 ? dispatch<8>(a, epi, kvt, s) : dispatch<4>(a, epi, kvt, s);
+}
+
+hipError_t rows_attn(const uint4 *qf, const uint4 *kvf, int M, int H, const int *kstart, const int *order, int kvt,
+                     uint4 *out, hipStream_t s) {
+  if (M < 1 || H < 1) return hipErrorInvalidValue;
+  const dim3 grid(H, (M + 31) / 32);
+  const u32x4 *q = reinterpret_cast<const u32x4 *>(qf), *kv = reinterpret_cast<const u32x4 *>(kvf);
+  if (kvt == kKvBf16)
+    hipLaunchKernelGGL(rows_attn_kernel<1>, grid, dim3(256), 0, s, q, kv, M, kstart, order, reinterpret_cast<u32x4 *>(out));
+  else
+    hipLaunchKernelGGL(rows_attn_kernel<2>, grid, dim3(256), 0, s, q, kv, M, kstart, order, reinterpret_cast<u32x4 *>(out));
+  return hipGetLastError();
+}
+
+}  // namespace itts

@@ -152,6 +152,14 @@ bool valid_config(const itts_config &c, std::string &why) {
 
 struct QLHost {
   DevBuf codes, params, bias;
+  DevBuf rcodes, rscale, rbias;  // the multi-row products' codes, scale table and bias planes
+  hipError_t ready_rows(int bits, int ptype, hipStream_t s) {
+    hipError_t e = rcodes.ensure(rows_codes_bytes(N, K, bits));
+    if (e == hipSuccess) e = rscale.ensure(sizeof(float) * rows_scale_floats(N, K));
+    if (e == hipSuccess) e = rbias.ensure(sizeof(uint4) * rows_bias_pieces(N, K));
+    if (e == hipSuccess) e = rows_params(dev(), bits, ptype, rcodes.as<uint4>(), rscale.as<float>(), rbias.as<uint4>(), s);
+    return e;
+  }
   DevQL dev() const { return DevQL{codes.as<uint8_t>(), params.p, bias.as<float>(), N, K}; }
   int N = 0, K = 0;
 };
@@ -192,9 +200,12 @@ struct itts_gpt {
   // the folded LayerNorms' group statistics of the residual rows [M][d/64] (mean, M2)
   DevBuf pst;
   DevBuf gws, gcnt;
+  // the multi-row forward's operands in fragment order: LayerNorm, attention and GELU outputs,
+  // Q, K / V
+  DevBuf fh, fa, ff, fq, fkv;
   // replay / all-row forward: per-layer scratch K/V (fp32 [n_head][M][64]), key starts,
   // head logits, probe maps, codes and log-probabilities
-  DevBuf rk, rv, kstart, plog, pmap, pcodes, plp, pkvs;
+  DevBuf rk, rv, kstart, plog, pmap, pcodes, plp;
   int align_pairs[2][2] = {{4, 10}, {5, 10}};  // (layer, head), align/mod.rs:37
   int n_align = 2;
   // batched decode: residual rows, q rows, split-form rows, attention partials, logits,
@@ -303,10 +314,6 @@ DevSampling to_dev_sampling(const itts_sampling &p, int n) {
   return d;
 }
 
-// Prompts up to this many rows use the per-row attention kernel, longer ones the MFMA
-// flash kernel (measured crossover on MI355X at 24 layers x 20 heads).
-constexpr int kFlashMinRows = 384;
-
 // GEMM arguments over M rows with the decoder's split-K workspace.
 GemmArgs gemm_args(const itts_gpt *g, const DevQL &ql, SplitAct x, int M) {
   GemmArgs ga{};
@@ -321,35 +328,73 @@ GemmArgs gemm_args(const itts_gpt *g, const DevQL &ql, SplitAct x, int M) {
   return ga;
 }
 
+// Prompts of more than this many rows run on operands in fragment order (kernels_rows.hip), fewer
+// on the 64 x 64 tiles whose K is split over blocks (kernels_prefill.hip).  Whole prefill in us,
+// fragments / tiles: 20 rows 1423 / 1329, 35 rows 1392 / 1373, 64 rows 1406 / 1435, 99 rows 1405 /
+// 1544, 235 rows 1630 / 2005.
+constexpr int kRowsMin = 48;
+
+// Grows buf to the planes of M rows of K values, zero where nothing is written.
+hipError_t ensure_planes(itts_gpt *g, DevBuf &buf, int M, int K) {
+  const size_t bytes = sizeof(uint4) * rows_planes_pieces(M, K);
+  if (bytes <= buf.bytes) return hipSuccess;
+  hipError_t e = buf.ensure(bytes);
+  if (e == hipSuccess) e = hipMemsetAsync(buf.p, 0, buf.bytes, g->stream);
+  return e;
+}
+
+// A multi-row product over planes x.
+RowsMm rows_args(const itts_gpt *g, const QLHost &q, const DevBuf &x, int M) {
+  RowsMm a{};
+  a.x = x.as<uint4>();
+  a.codes = q.rcodes.as<uint4>();
+  a.scale = q.rscale.as<float>();
+  a.bw = q.rbias.as<uint4>();
+  a.bias = q.bias.as<float>();
+  a.ldn = rows_ldn(q.N);
+  a.M = M;
+  a.N = q.N;
+  a.K = q.K;
+  a.n_cu = g->n_cu;
+  return a;
+}
+
+// ... of decoder weight i (4 per layer, then mel_head).
+RowsMm rows_args(const itts_gpt *g, size_t i, const DevBuf &x, int M) { return rows_args(g, g->qls[i], x, M); }
+
 // Grows the per-row buffers of a multi-row forward to M rows.
 itts_status ensure_rows(itts_gpt *g, int M) {
   const int d = g->cfg.d_model;
   HIP_TRY(g->px.ensure(sizeof(float) * (size_t)M * d));
+  HIP_TRY(g->pst.ensure(sizeof(float2) * (size_t)M * (d / kGroup)));
+  HIP_TRY(ensure_planes(g, g->fh, M, d));
+  HIP_TRY(ensure_planes(g, g->fa, M, d));
+  HIP_TRY(ensure_planes(g, g->ff, M, g->cfg.d_ffn));
+  HIP_TRY(g->fq.ensure(sizeof(uint4) * rows_q_pieces(M, g->cfg.n_head)));
+  HIP_TRY(g->fkv.ensure(sizeof(uint4) * rows_kv_pieces(M, g->cfg.n_head)));
+  if (M > kRowsMin) return ITTS_OK;
   HIP_TRY(g->ph.ensure(M, d));
   HIP_TRY(g->pq.ensure(sizeof(float) * (size_t)M * d));
   HIP_TRY(g->pa.ensure(M, d));
   HIP_TRY(g->pf.ensure(M, g->cfg.d_ffn));
-  HIP_TRY(g->pst.ensure(sizeof(float2) * (size_t)M * (d / kGroup)));
   return ITTS_OK;
 }
 
-// LayerNorms of the multi-row stacks after layer 0's ln_1 folded into the products: each
+// LayerNorms of a short prompt's stack after layer 0's ln_1 folded into the products: each
 // residual product writes gamma * x of the next LayerNorm in split form with the group
 // statistics of x (TileFoldOut), and the QKV / c_fc product applies them (TileFoldIn).
-// Layer 0's ln_1 input comes from the embeddings and keeps its row kernel.  Used on the
-// 64 x 64 tiles (235-row prefill 2.42 -> 2.35 ms on MI355X); on 128 x 128 tiles the fold's
-// epilogues cost more than the row kernels (4 x 547 rows: 11.05 -> 11.32 ms), and d <= 2048
-// (the statistics' reduction holds at most 32 groups a row).
+// Layer 0's ln_1 input comes from the embeddings and keeps its row kernel.  d <= 2048 (the
+// statistics' reduction holds at most 32 groups a row).
 struct StackFold {
   bool on;
   size_t per;
   const float *fold;
   float2 *st;
   int d, F;
-  StackFold(const itts_gpt *g, int M) {
+  explicit StackFold(const itts_gpt *g) {
     d = g->cfg.d_model;
     F = g->cfg.d_ffn;
-    on = g->fold.p != nullptr && d % kGroup == 0 && d <= 32 * kGroup && M <= kGemmSmallTileRows;
+    on = g->fold.p != nullptr && d % kGroup == 0 && d <= 32 * kGroup;
     per = fold_floats(d, F);
     fold = g->fold.as<float>();
     st = g->pst.as<float2>();
@@ -426,6 +471,87 @@ itts_status embed_prompts(itts_gpt *g, const itts_code_prompt *ps, int B, std::v
   return ITTS_OK;
 }
 
+// A requested attention export: probabilities of (layer, head) for the query rows q0..
+// over the key columns [k0, k1), into device memory.
+struct ProbeSpec {
+  int layer, head, q0, k0, k1;
+  float *out;
+};
+
+// Runs n_layers blocks over the M rows in gpt->px on operands in fragment order.  Row
+// r attends to keys kstart[r] (or 0) .. r; K/V rows go to kv's cache (prefill) or, for the
+// layers that are probed, to the fp32 scratch rk / rv.  ln_1 (after layer 0) and ln_2 are
+// folded: each residual product writes gamma x and its group statistics, and the product
+// after it applies them.
+itts_status rows_stack(itts_gpt *g, itts_kv *kv, int M, int n_layers, const int *kstart, const int *order,
+                       const std::vector<ProbeSpec> &probes) {
+  const itts_config &c = g->cfg;
+  const int d = c.d_model, F = c.d_ffn, bits = c.quant_bits, kvt = kv ? kv->kvt : kKvF32;
+  hipStream_t s = g->stream;
+  float *X = g->px.as<float>();
+  const bool folded = g->fold.p != nullptr && d <= 32 * kGroup;  // (a row's group statistics in registers)
+  const size_t per = fold_floats(d, F);
+  float2 *st = g->pst.as<float2>();
+  for (int l = 0; l < n_layers; l++) {
+    const DevLayer &L = g->layers[l];
+    const float *fo = g->fold.as<float>() + per * l;
+    if (!folded || l == 0)
+      HIP_TRY(rows_ln(X, L.ln1_w, L.ln1_b, nullptr, nullptr, M, d, g->fh.as<uint4>(), s));
+    RowsMm a = rows_args(g, 4 * l, g->fh, M);
+    if (folded && l > 0) {
+      a.st = st;
+      a.fG = fo;
+      a.fc = fo + 3 * d;
+    }
+    a.qf = g->fq.as<uint4>();
+    a.kvf = g->fkv.as<uint4>();
+    bool probed = false;
+    for (const ProbeSpec &p : probes) probed = probed || p.layer == l;
+    if (kv) {
+      a.kc = kv->k_layer(l);
+      a.vc = kv->v_layer(l);
+      a.max_seq = kv->max_seq;
+    } else if (probed) {
+      a.kc = g->rk.p;
+      a.vc = g->rv.p;
+      a.max_seq = M;
+      a.q_out = g->pq.as<float>();
+    }
+    HIP_TRY(rows_mm(a, bits, kEpiQKV, kvt, s));
+    for (const ProbeSpec &p : probes)  // read-only exports of this layer's attention
+      if (p.layer == l)
+        HIP_TRY(launch_attn_probe(g->pq.as<float>(), M, kstart, g->rk.p, g->rv.p, c.n_head,
+                                  AttnProbe{p.head, p.q0, p.k0, p.k1, p.out}, kKvF32, s));
+    HIP_TRY(rows_attn(g->fq.as<uint4>(), g->fkv.as<uint4>(), M, c.n_head, kstart, order, kvt, g->fa.as<uint4>(), s));
+    a = rows_args(g, 4 * l + 1, g->fa, M);
+    a.y = X;
+    if (folded) {
+      a.o = g->fh.as<uint4>();
+      a.gamma = L.ln2_w;
+      a.so = st;
+    }
+    HIP_TRY(rows_mm(a, bits, kEpiResid, kvt, s));
+    if (!folded) HIP_TRY(rows_ln(X, L.ln2_w, L.ln2_b, nullptr, nullptr, M, d, g->fh.as<uint4>(), s));
+    a = rows_args(g, 4 * l + 2, g->fh, M);
+    if (folded) {
+      a.st = st;
+      a.fG = fo + 6 * d;
+      a.fc = fo + 6 * d + F;
+    }
+    a.o = g->ff.as<uint4>();
+    HIP_TRY(rows_mm(a, bits, kEpiGelu, kvt, s));
+    a = rows_args(g, 4 * l + 3, g->ff, M);
+    a.y = X;
+    if (folded && l + 1 < n_layers) {
+      a.o = g->fh.as<uint4>();
+      a.gamma = g->layers[l + 1].ln1_w;
+      a.so = st;
+    }
+    HIP_TRY(rows_mm(a, bits, kEpiResid, kvt, s));
+  }
+  return ITTS_OK;
+}
+
 // Enqueues the stack over the rows already embedded in gpt->px (prefill, T rows at
 // cache positions 0..T-1) and the head of the last row into gpt->logits.
 itts_status enqueue_prefill_stack(itts_gpt *g, itts_kv *kv, int T) {
@@ -434,21 +560,19 @@ itts_status enqueue_prefill_stack(itts_gpt *g, itts_kv *kv, int T) {
   hipStream_t s = g->stream;
   float *X = g->px.as<float>(), *Q = g->pq.as<float>();
   auto gemm = [&](const DevQL &ql, SplitAct x) { return gemm_args(g, ql, x, T); };
-  const StackFold sf(g, T);
-  for (int l = 0; l < c.n_layer; l++) {
+  if (T > kRowsMin) {
+    if (itts_status st = rows_stack(g, kv, T, c.n_layer, nullptr, nullptr, {})) return st;
+  }
+  const StackFold sf(g);
+  for (int l = 0; T <= kRowsMin && l < c.n_layer; l++) {
     const DevLayer &L = g->layers[l];
     if (!sf.on || l == 0) HIP_TRY(launch_ln_rows(X, L.ln1_w, L.ln1_b, T, d, g->ph.out(), s));
     GemmArgs ga = gemm(L.attn, g->ph.act());
     if (sf.on && l > 0) ga.tfi = sf.qkv(l);
     ga.qkv = QkvDst{Q, kv->k_layer(l), kv->v_layer(l), kv->max_seq, 0, d};
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiQKV, kv->kvt, s));
-    if (T <= kFlashMinRows) {  // few query tiles: one block per (head, row) spreads wider
-      HIP_TRY(launch_attn_prefill(Q, T, 0, kv->k_layer(l), kv->v_layer(l), c.n_head, kv->max_seq, g->pa.out(),
-                                  kv->kvt, s));
-    } else {
-      HIP_TRY(launch_attn_flash(Q, T, 0, nullptr, kv->k_layer(l), kv->v_layer(l), kv->max_seq, c.n_head,
-                                g->pa.out(), kv->kvt, s));
-    }
+    HIP_TRY(launch_attn_prefill(Q, T, 0, kv->k_layer(l), kv->v_layer(l), c.n_head, kv->max_seq, g->pa.out(),
+                                kv->kvt, s));
     ga = gemm(L.proj, g->pa.act());
     ga.y = X;
     if (sf.on) ga.tfo = sf.out(g->ph, L.ln2_w);
@@ -618,66 +742,29 @@ itts_status run_prefill(itts_gpt *g, itts_kv *kv, const int32_t *text, int32_t n
   return ITTS_OK;
 }
 
-// A requested attention export: probabilities of (layer, head) for the query rows q0..
-// over the key columns [k0, k1), into device memory.
-struct ProbeSpec {
-  int layer, head, q0, k0, k1;
-  float *out;
-};
-
 // Runs n_layers blocks over the M rows in gpt->px (row r attends to keys kstart[r]..r)
 // with fp32 scratch K/V for one layer at a time, filling the probes on the way.
 itts_status forward_rows_stack(itts_gpt *g, int M, const std::vector<int> &kstart, int n_layers,
                                const std::vector<ProbeSpec> &probes) {
-  const itts_config &c = g->cfg;
-  const int d = c.d_model, bits = c.quant_bits, pt = g->ptype();
+  const int d = g->cfg.d_model;
   hipStream_t s = g->stream;
   HIP_TRY(g->rk.ensure(sizeof(float) * (size_t)M * d));
-  HIP_TRY(g->pkvs.ensure(sizeof(uint16_t) * attn_kv_split_halves(c.n_head, M)));
   HIP_TRY(g->rv.ensure(sizeof(float) * (size_t)M * d));
-  // kstart, then the attention's query tiles (64 rows) ordered by their key count, most first
-  const int n_tiles = (M + 63) / 64;
+  HIP_TRY(g->pq.ensure(sizeof(float) * (size_t)M * d));
+  // kstart, then the attention's query tiles (32 rows) ordered by their key count, most first
+  const int n_tiles = (M + 31) / 32;
   std::vector<int> ks_order(kstart);
   ks_order.resize((size_t)M + n_tiles);
   {
     std::vector<int> keys(n_tiles);
-    for (int i = 0; i < n_tiles; i++) keys[i] = std::min(M - 1, 64 * i + 63) - kstart[64 * i] + 1;
+    for (int i = 0; i < n_tiles; i++) keys[i] = std::min(M - 1, 32 * i + 31) - kstart[32 * i] + 1;
     int *order = ks_order.data() + M;
     for (int i = 0; i < n_tiles; i++) order[i] = i;
     std::stable_sort(order, order + n_tiles, [&](int a, int b) { return keys[a] > keys[b]; });
   }
   HIP_TRY(g->kstart.ensure(sizeof(int) * ks_order.size()));
   HIP_TRY(hipMemcpyAsync(g->kstart.p, ks_order.data(), sizeof(int) * ks_order.size(), hipMemcpyHostToDevice, s));
-  float *X = g->px.as<float>(), *Q = g->pq.as<float>();
-  const StackFold sf(g, M);
-  for (int l = 0; l < n_layers; l++) {
-    const DevLayer &L = g->layers[l];
-    if (!sf.on || l == 0) HIP_TRY(launch_ln_rows(X, L.ln1_w, L.ln1_b, M, d, g->ph.out(), s));
-    GemmArgs ga = gemm_args(g, L.attn, g->ph.act(), M);
-    if (sf.on && l > 0) ga.tfi = sf.qkv(l);
-    ga.qkv = QkvDst{Q, g->rk.p, g->rv.p, M, 0, d};
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiQKV, kKvF32, s));
-    for (const ProbeSpec &p : probes)  // read-only exports of this layer's attention
-      if (p.layer == l)
-        HIP_TRY(launch_attn_probe(Q, M, g->kstart.as<int>(), g->rk.p, g->rv.p, c.n_head,
-                                  AttnProbe{p.head, p.q0, p.k0, p.k1, p.out}, kKvF32, s));
-    HIP_TRY(launch_attn_flash(Q, M, 0, g->kstart.as<int>(), g->rk.p, g->rv.p, M, c.n_head, g->pa.out(), kKvF32, s,
-                              g->pkvs.as<uint16_t>(), g->kstart.as<int>() + M));
-    ga = gemm_args(g, L.proj, g->pa.act(), M);
-    ga.y = X;
-    if (sf.on) ga.tfo = sf.out(g->ph, L.ln2_w);
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kKvF32, s));
-    if (!sf.on) HIP_TRY(launch_ln_rows(X, L.ln2_w, L.ln2_b, M, d, g->ph.out(), s));
-    ga = gemm_args(g, L.fc, g->ph.act(), M);
-    if (sf.on) ga.tfi = sf.fc(l);
-    ga.xo = g->pf.out();
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiGelu, kKvF32, s));
-    ga = gemm_args(g, L.mproj, g->pf.act(), M);
-    ga.y = X;
-    if (sf.on && l + 1 < n_layers) ga.tfo = sf.out(g->ph, g->layers[l + 1].ln1_w);
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kKvF32, s));
-  }
-  return ITTS_OK;
+  return rows_stack(g, nullptr, M, n_layers, g->kstart.as<int>(), g->kstart.as<int>() + M, probes);
 }
 
 // Head logits of R rows of gpt->px from row0: ln_f, final_norm, mel_head (gpt.rs:838-846)
@@ -686,11 +773,11 @@ itts_status head_rows(itts_gpt *g, int row0, int R) {
   const itts_config &c = g->cfg;
   const int d = c.d_model;
   HIP_TRY(g->plog.ensure(sizeof(float) * (size_t)R * c.mel_vocab));
-  HIP_TRY(launch_ln_rows(g->px.as<float>() + (size_t)row0 * d, g->ln_f_w.as<float>(), g->ln_f_b.as<float>(), R, d,
-                         g->ph.out(), g->stream, g->fn_w.as<float>(), g->fn_b.as<float>()));
-  GemmArgs ga = gemm_args(g, g->head, g->ph.act(), R);
-  ga.y = g->plog.as<float>();
-  HIP_TRY(launch_gemm(ga, c.quant_bits, g->ptype(), kEpiStore, kKvF32, g->stream));
+  HIP_TRY(rows_ln(g->px.as<float>() + (size_t)row0 * d, g->ln_f_w.as<float>(), g->ln_f_b.as<float>(),
+                  g->fn_w.as<float>(), g->fn_b.as<float>(), R, d, g->fh.as<uint4>(), g->stream));
+  RowsMm a = rows_args(g, 4 * (size_t)c.n_layer, g->fh, R);
+  a.y = g->plog.as<float>();
+  HIP_TRY(rows_mm(a, c.quant_bits, kEpiStore, kKvF32, g->stream));
   return ITTS_OK;
 }
 
@@ -1092,6 +1179,9 @@ itts_status itts_gpt_create(const itts_weights *w, itts_gpt **out) {
       if (hipStreamSynchronize(g->stream) != hipSuccess)
         return fail(set_error(ITTS_E_DEVICE, "LayerNorm fold failed"));
     }
+    for (QLHost &q : g->qls)
+      if (q.ready_rows(bits, g->ptype(), g->stream) != hipSuccess)
+        return fail(set_error(ITTS_E_DEVICE, "laying out the multi-row products' weights failed"));
     if (sampler_stage_init(dev) != hipSuccess)
       return fail(set_error(ITTS_E_DEVICE, "sampler staging area lookup failed"));
   }
@@ -1979,6 +2069,15 @@ itts_status itts_qlinear_forward(itts_gpt *gpt, const itts_qlinear *ql, int32_t 
     a.x = dx.as<float>();
     a.y = dy.as<float>();
     HIP_TRY(launch_gemv(a, bits, pt, kProNone, kEpiStore, kKvBf16, gpt->stream));
+  } else if (M > kRowsMin) {
+    DevBuf planes;
+    HIP_TRY(ensure_planes(gpt, planes, M, K));
+    HIP_TRY(q.ready_rows(bits, pt, gpt->stream));
+    HIP_TRY(rows_ln(dx.as<float>(), nullptr, nullptr, nullptr, nullptr, M, K, planes.as<uint4>(), gpt->stream));
+    RowsMm a = rows_args(gpt, q, planes, M);
+    a.y = dy.as<float>();
+    HIP_TRY(rows_mm(a, bits, kEpiStore, kKvF32, gpt->stream));
+    HIP_TRY(hipStreamSynchronize(gpt->stream));
   } else {
     SplitBuf xs;
     HIP_TRY(xs.ensure(M, K));

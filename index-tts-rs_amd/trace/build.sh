@@ -12,5 +12,5 @@ $HIPCC --offload-arch=gfx950 -O3 -std=c++17 -fPIC -Wall -Wno-unused-function \
   -Xclang -target-feature -Xclang -packed-fp32-ops -I../csrc -c _gen/kernels_persist_trace.hip -o _gen/kp_trace.o
 B=../_build
 $HIPCC --offload-arch=gfx950 -shared -fPIC -o lib/libitts_trace.so $B/kernels_decode.o $B/kernels_prefill.o \
-  $B/kernels_sampler.o _gen/kp_trace.o $B/kernels_attn.o $B/kernels_cfm.o $B/runtime.o $B/loader.o $B/cfm.o -lpthread
+  $B/kernels_sampler.o _gen/kp_trace.o $B/kernels_rows.o $B/kernels_cfm.o $B/kernels_cfm_mm.o $B/runtime.o $B/loader.o $B/cfm.o -lpthread
 echo "built trace/lib/libitts_trace.so"

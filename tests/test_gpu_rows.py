@@ -1,0 +1,97 @@
+"""The multi-row forward on operands in fragment order (prompts of more than 48 rows, replay,
+all-row forward): its tiles' edges against the oracle and, for the product alone, against
+float64."""
+import sys
+
+import numpy as np
+import pytest
+
+import ito
+import itts_hip as H
+from itts_hip import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+_models = {}
+
+
+def _model(bits, pd, over=()):
+    key = (bits, pd, over)
+    if key not in _models:
+        cfg = dict(synth.SMALL_CONFIG, quant_bits=bits, param_dtype=pd, **dict(over))
+        W = synth.make_weights(cfg, seed=23, init="rich")
+        _models[key] = (W, H.Gpt(W), ito.Model(W))
+    return _models[key]
+
+
+# 49: the first row count of this path; tiles of 32 and 64 rows and of 32 and 64 keys
+@pytest.mark.parametrize("T", [48, 49, 63, 64, 65, 96, 97, 129, 320, 321])
+@pytest.mark.parametrize("bits,pd,kv", [(8, H.ITTS_F16, H.ITTS_F32), (8, H.ITTS_F32, H.ITTS_BF16),
+                                        (4, H.ITTS_F16, H.ITTS_BF16), (4, H.ITTS_F32, H.ITTS_F32)])
+def test_prefill_edges(T, bits, pd, kv):
+    say(f"[gpu] rows prefill T={T} bits={bits} pd={pd} kv={kv}")
+    W, g, M = _model(bits, pd)
+    pr = synth.make_prompt(W.cfg, 3, 20, seed=T)
+    prior = (np.arange(T - 26, dtype=np.int32) * 13) % (W.cfg["mel_vocab"] - 2)
+    cache, okv = g.kv_cache(400, kv), M.kv(400, kv_bf16=kv == H.ITTS_BF16)
+    # a longer prompt first: what it leaves in the buffers must not reach the next one
+    g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, np.zeros(T + 30, np.int32), cache)
+    a = g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, prior, cache)
+    b = M.prefill_after(okv, pr.text_tokens, pr.conds, pr.lang_id, prior)
+    # the bars of the decoder's other parity tests: 2e-4 with like caches, where bf16 rows that
+    # round the other way set the floor (3e-4 at full depth), 2e-5 with fp32 rows
+    tol = 2e-5 if kv == H.ITTS_F32 else 2e-3
+    assert np.abs(a - b).max() < tol * max(1.0, np.abs(b).max())
+    s1, s2 = g.step(cache, 11, len(prior) + 2), M.step(okv, 11, len(prior) + 2)  # on the rows just written
+    assert np.abs(s1 - s2).max() < tol * max(1.0, np.abs(s2).max())
+
+
+def test_wide_model_without_folds():
+    """d > 2048: the LayerNorms keep their row kernel."""
+    over = (("n_layer", 2), ("d_model", 2112), ("n_head", 33), ("d_ffn", 128), ("text_vocab", 50), ("mel_vocab", 130))
+    W, g, M = _model(8, H.ITTS_F16, over)
+    pr = synth.make_prompt(W.cfg, 3, 60, seed=3)
+    cache, okv = g.kv_cache(128, H.ITTS_F32), M.kv(128, kv_bf16=False)
+    a = g.prefill(pr.text_tokens, pr.conds, pr.lang_id, cache)
+    b = M.prefill_after(okv, pr.text_tokens, pr.conds, pr.lang_id)
+    assert np.abs(a - b).max() < 2e-5 * max(1.0, np.abs(b).max())
+
+
+def test_forward_logits_prompt_boundaries():
+    """Prompts that start and end inside query and key tiles, one shorter than a tile."""
+    W, g, M = _model(8, H.ITTS_F16)
+    prompts = [H.CodePrompt(p.text_tokens, p.conds, p.lang_id, (np.arange(k, dtype=np.int32) * 7) % 1000)
+               for p, k in ((synth.make_prompt(W.cfg, 3, n, seed=n), k) for n, k in ((5, 0), (30, 61), (2, 3), (40, 20)))]
+    got = g.forward_logits(prompts)
+    r = 0
+    for p in prompts:
+        emb = M.sequence_embedding(p.text_tokens, p.conds, p.lang_id, p.prior_codes)
+        ref = M.forward_rows(M.kv(200, kv_bf16=False), emb, 0)
+        assert np.abs(got[r:r + len(ref)] - ref).max() < 2e-5 * max(1.0, np.abs(ref).max())
+        r += len(ref)
+    assert r == len(got)
+
+
+# 32 x 64 tiles by four waves; by eight (K >= 4096, few tiles); 64 x 64 (K >= 4096, many tiles)
+@pytest.mark.parametrize("bits,pd", [(8, H.ITTS_F16), (4, H.ITTS_F32)])
+@pytest.mark.parametrize("M,N,K", [(49, 37, 192), (65, 130, 64), (100, 1026, 1280), (70, 132, 4160), (2000, 1090, 4096)])
+def test_product_vs_fp64(bits, pd, M, N, K):
+    say(f"[gpu] rows product M={M} N={N} K={K} bits={bits}")
+    _, g, _ = _model(8, H.ITTS_F16)
+    rng = np.random.default_rng(M + N + K)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    codes, s, b = H.quantize(w, bits, pd)
+    bias = rng.standard_normal(N).astype(np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = g.qlinear_forward(codes, s, b, bias, x, N, K, bits, pd)
+    Wd = ito.dequant(synth.QLinear(codes, s, b, bias, N, K), bits, pd).astype(np.float64)
+    ref = x.astype(np.float64) @ Wd.T + bias
+    # the tiled product's bar: 4e-6 of the sum of magnitudes (22-bit operands, fp32 sums)
+    bound = np.abs(x).astype(np.float64) @ np.abs(Wd).T + np.abs(bias)
+    assert np.all(np.abs(got - ref) <= 4e-6 * bound + 1e-7)
