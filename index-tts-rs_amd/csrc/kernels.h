@@ -154,6 +154,10 @@ struct TileFoldOut {
 
 struct GemmArgs {
   DevQL ql;
+  // few-row products: the codes in fragment order and the (scale, bias) words [K/64][ldn]
+  const uint4 *fcodes;
+  const void *fparams;
+  int ldn;
   SplitAct x;       // [M][K] (unused with fold.x)
   FoldIn fold;      // fold.x set: the input is LayerNorm(x) by the fold above
   TileFoldIn tfi;   // tfi.st set (tiled product, QKV or GELU epilogue): folded LayerNorm input
@@ -187,7 +191,9 @@ int rows_ldn(int N);
 size_t rows_scale_floats(int N, int K);
 size_t rows_bias_pieces(int N, int K);
 size_t rows_codes_bytes(int N, int K, int bits);
-hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, hipStream_t s);
+// ... (codes, scales, bias planes; params: the (scale, bias) words [K/64][rows_ldn(N)])
+hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, void *params,
+                       hipStream_t s);
 // LN (and a second one with w2; none without w) of M rows [M][d] as planes.
 hipError_t rows_ln(const float *x, const float *w, const float *b, const float *w2, const float *b2, int M, int d,
                    uint4 *out, hipStream_t s);

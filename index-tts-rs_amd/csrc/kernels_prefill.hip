@@ -804,8 +804,8 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
 // The 64-row tiles above spend most of a launch filling the ring for a few real rows.  Here
 // a block of kFewWaves waves takes 64 output columns (two 32-column MFMA tiles) over
 // kFewWaves K groups, one per wave, with no LDS staging: each lane loads its activation and code
-// fragments straight into registers (a lane's 16 codes of a column are one 16-byte load,
-// its 16 activations of a row two), in the K order the tiles above use.  Rows past M are
+// fragments straight into registers (a lane's 16 codes of a column are one 16-byte load
+// of the codes' copy in fragment order, its 16 activations of a row two), in the K order the tiles above use.  Rows past M are
 // zero fragments; in the 32 x 32 result a lane's rows 4h .. 4h+3 (h = lane >> 5) are the
 // only live ones.  The waves' partials are added in wave order in LDS; the K splits
 // (blocks) in split order by the last block of the column tile to arrive, as above.
@@ -893,24 +893,23 @@ __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN,
         xa[gi][1][kp][1] = pl[1];
       }
     }
-    // code fragments of columns n0 + 32 j + c (a column past N reads column N - 1, a group
-    // past G reads group 0)
+    // code fragments and parameters of columns n0 + 32 j + c, from the copies in fragment order
+    // (columns past N hold zeros; a group past G reads group 0)
     const int gl = live ? g : 0;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const int n = min(n0 + 32 * j + c, N - 1);
+      const uint8_t *cf = reinterpret_cast<const uint8_t *>(a.fcodes) + ((size_t)(2 * tn + j) * G + gl) * (BITS * 256) +
+                          lane * (BITS * 2);
 #pragma unroll
       for (int kp = 0; kp < 2; kp++) {
         if constexpr (BITS == 8) {
-          cq[gi][j][kp] =
-              *reinterpret_cast<const u32x4 *>(a.ql.codes + (size_t)n * K + (size_t)gl * 64 + 32 * kp + 16 * h);
+          cq[gi][j][kp] = *reinterpret_cast<const u32x4 *>(cf + kp * (BITS * 128));
         } else {
-          const uint2 v =
-              *reinterpret_cast<const uint2 *>(a.ql.codes + (size_t)n * (K / 2) + (size_t)gl * 32 + 16 * kp + 8 * h);
+          const uint2 v = *reinterpret_cast<const uint2 *>(cf + kp * (BITS * 128));
           cq[gi][j][kp] = u32x4{v.x, v.y, 0u, 0u};
         }
       }
-      pr[gi][j] = static_cast<const PRaw *>(a.ql.params)[(size_t)n * G + gl];
+      pr[gi][j] = static_cast<const PRaw *>(a.fparams)[(size_t)gl * a.ldn + n0 + 32 * j + c];
     }
     if constexpr (!FOLD) {
 #pragma unroll
@@ -1325,7 +1324,7 @@ hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt,
   if (a.ql.K % kGroup != 0 || a.M <= 0 || a.ql.N <= 0) return hipErrorInvalidValue;
   if (epi == kEpiGelu && a.ql.N % kGroup != 0) return hipErrorInvalidValue;
   if (a.fold.x) {  // the folded LayerNorm: few-row products with one group a wave only
-    if (a.M > kFewRows || (bits != 8 && bits != 4) || a.ql.K % 256 != 0 || a.ql.K > 256 * kFoldQ ||
+    if (a.M > kFewRows || !a.fcodes || (bits != 8 && bits != 4) || a.ql.K % 256 != 0 || a.ql.K > 256 * kFoldQ ||
         (epi != kEpiQKV && epi != kEpiGelu) || !a.fold.gamma || !a.fold.G || !a.fold.c)
       return hipErrorInvalidValue;
   }
@@ -1335,7 +1334,7 @@ hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt,
                    !a.tfo.o.gs || a.fold.x))
     return hipErrorInvalidValue;
   // (the tiled folds are written for the tiled product only)
-  if (a.M <= kFewRows && (bits == 8 || bits == 4) && !a.tfi.st && !a.tfo.st) {
+  if (a.M <= kFewRows && (bits == 8 || bits == 4) && !a.tfi.st && !a.tfo.st && a.fcodes) {
     // a group per wave while that keeps the splits within kFewMaxSplits (gw > kFewMaxGw
     // beyond that: the tiled GEMM)
     const int nN = (a.ql.N + 63) / 64, G = a.ql.K / kGroup;

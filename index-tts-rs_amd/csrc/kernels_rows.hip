@@ -91,10 +91,11 @@ __global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const flo
 }
 
 // ---- weights ----------------------------------------------------------------------------
-// scale [G][ldn] fp32 (columns past N zero) and b' = b + off s as fragment planes of G values
+// scale [G][ldn] fp32 and the (scale, bias) words transposed alike (columns past N zero), and b' =
+// b + off s as fragment planes of G values
 template <int PT>
 __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, int N, int G, int ldn, float off,
-                                                          float *scale, u32x4 *bw) {
+                                                          float *scale, u32x4 *bw, void *words) {
   const int nx = (G + 15) / 16;
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)ldn * nx * 2) return;
@@ -105,7 +106,12 @@ __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, in
     const int g = g8 * 8 + j;
     float2 sb = make_float2(0.0f, 0.0f);
     if (n < N && g < G) sb = load_param<PT>(params, (size_t)n * G + g);
-    if (g < G) scale[(size_t)g * ldn + n] = sb.x;
+    if (g < G) {
+      const size_t i = (size_t)g * ldn + n;
+      scale[i] = sb.x;
+      if constexpr (PT == kParamF32) static_cast<float2 *>(words)[i] = sb;
+      else static_cast<uint32_t *>(words)[i] = n < N ? static_cast<const uint32_t *>(params)[(size_t)n * G + g] : 0u;
+    }
     v[j] = fmaf(off, sb.x, sb.y);
   }
   u32x4 hi, lo;
@@ -731,7 +737,8 @@ size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64) * rows_ldn(N); 
 size_t rows_codes_bytes(int N, int K, int bits) { return (size_t)rows_ldn(N) * K * bits / 8; }
 size_t rows_bias_pieces(int N, int K) { return (size_t)(rows_ldn(N) / 32) * ((K / 64 + 15) / 16) * 128; }
 
-hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, hipStream_t s) {
+hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, void *params,
+                       hipStream_t s) {
   const long nc = (long)(rows_ldn(ql.N) / 32) * (ql.K / 64) * 128;
   const dim3 cg((unsigned)((nc + 255) / 256));
   uint8_t *co = reinterpret_cast<uint8_t *>(codes);
@@ -743,10 +750,10 @@ hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float
   const dim3 grid((unsigned)((n + 255) / 256));
   if (ptype == kParamF32)
     hipLaunchKernelGGL(rows_params_kernel<kParamF32>, grid, dim3(256), 0, s, ql.params, ql.N, G, ldn, off, scale,
-                       reinterpret_cast<u32x4 *>(bw));
+                       reinterpret_cast<u32x4 *>(bw), params);
   else
     hipLaunchKernelGGL(rows_params_kernel<kParamF16>, grid, dim3(256), 0, s, ql.params, ql.N, G, ldn, off, scale,
-                       reinterpret_cast<u32x4 *>(bw));
+                       reinterpret_cast<u32x4 *>(bw), params);
   return hipGetLastError();
 }
 

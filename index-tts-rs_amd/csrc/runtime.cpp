@@ -152,12 +152,15 @@ bool valid_config(const itts_config &c, std::string &why) {
 
 struct QLHost {
   DevBuf codes, params, bias;
-  DevBuf rcodes, rscale, rbias;  // the multi-row products' codes, scale table and bias planes
+  // the multi-row products' codes, scale table, bias planes and parameter words
+  DevBuf rcodes, rscale, rbias, rwords;
   hipError_t ready_rows(int bits, int ptype, hipStream_t s) {
     hipError_t e = rcodes.ensure(rows_codes_bytes(N, K, bits));
     if (e == hipSuccess) e = rscale.ensure(sizeof(float) * rows_scale_floats(N, K));
     if (e == hipSuccess) e = rbias.ensure(sizeof(uint4) * rows_bias_pieces(N, K));
-    if (e == hipSuccess) e = rows_params(dev(), bits, ptype, rcodes.as<uint4>(), rscale.as<float>(), rbias.as<uint4>(), s);
+    if (e == hipSuccess) e = rwords.ensure((ptype == kParamF32 ? 8 : 4) * rows_scale_floats(N, K));
+    if (e == hipSuccess)
+      e = rows_params(dev(), bits, ptype, rcodes.as<uint4>(), rscale.as<float>(), rbias.as<uint4>(), rwords.p, s);
     return e;
   }
   DevQL dev() const { return DevQL{codes.as<uint8_t>(), params.p, bias.as<float>(), N, K}; }
@@ -314,10 +317,13 @@ DevSampling to_dev_sampling(const itts_sampling &p, int n) {
   return d;
 }
 
-// GEMM arguments over M rows with the decoder's split-K workspace.
-GemmArgs gemm_args(const itts_gpt *g, const DevQL &ql, SplitAct x, int M) {
+// GEMM arguments over M rows of a weight with the decoder's split-K workspace.
+GemmArgs gemm_args(const itts_gpt *g, const QLHost &q, SplitAct x, int M) {
   GemmArgs ga{};
-  ga.ql = ql;
+  ga.ql = q.dev();
+  ga.fcodes = q.rcodes.as<uint4>();
+  ga.fparams = q.rwords.p;
+  ga.ldn = rows_ldn(q.N);
   ga.x = x;
   ga.M = M;
   ga.ws = g->gws.as<float>();
@@ -559,7 +565,7 @@ itts_status enqueue_prefill_stack(itts_gpt *g, itts_kv *kv, int T) {
   const int d = c.d_model, bits = c.quant_bits, pt = g->ptype();
   hipStream_t s = g->stream;
   float *X = g->px.as<float>(), *Q = g->pq.as<float>();
-  auto gemm = [&](const DevQL &ql, SplitAct x) { return gemm_args(g, ql, x, T); };
+  auto gemm = [&](size_t i, SplitAct x) { return gemm_args(g, g->qls[i], x, T); };
   if (T > kRowsMin) {
     if (itts_status st = rows_stack(g, kv, T, c.n_layer, nullptr, nullptr, {})) return st;
   }
@@ -567,22 +573,22 @@ itts_status enqueue_prefill_stack(itts_gpt *g, itts_kv *kv, int T) {
   for (int l = 0; T <= kRowsMin && l < c.n_layer; l++) {
     const DevLayer &L = g->layers[l];
     if (!sf.on || l == 0) HIP_TRY(launch_ln_rows(X, L.ln1_w, L.ln1_b, T, d, g->ph.out(), s));
-    GemmArgs ga = gemm(L.attn, g->ph.act());
+    GemmArgs ga = gemm(4 * (size_t)l, g->ph.act());
     if (sf.on && l > 0) ga.tfi = sf.qkv(l);
     ga.qkv = QkvDst{Q, kv->k_layer(l), kv->v_layer(l), kv->max_seq, 0, d};
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiQKV, kv->kvt, s));
     HIP_TRY(launch_attn_prefill(Q, T, 0, kv->k_layer(l), kv->v_layer(l), c.n_head, kv->max_seq, g->pa.out(),
                                 kv->kvt, s));
-    ga = gemm(L.proj, g->pa.act());
+    ga = gemm(4 * (size_t)l + 1, g->pa.act());
     ga.y = X;
     if (sf.on) ga.tfo = sf.out(g->ph, L.ln2_w);
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kv->kvt, s));
     if (!sf.on) HIP_TRY(launch_ln_rows(X, L.ln2_w, L.ln2_b, T, d, g->ph.out(), s));
-    ga = gemm(L.fc, g->ph.act());
+    ga = gemm(4 * (size_t)l + 2, g->ph.act());
     if (sf.on) ga.tfi = sf.fc(l);
     ga.xo = g->pf.out();
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiGelu, kv->kvt, s));
-    ga = gemm(L.mproj, g->pf.act());
+    ga = gemm(4 * (size_t)l + 3, g->pf.act());
     ga.y = X;
     if (sf.on && l + 1 < c.n_layer) ga.tfo = sf.out(g->ph, g->layers[l + 1].ln1_w);
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kv->kvt, s));
@@ -878,7 +884,7 @@ itts_status enqueue_step_batch(itts_gpt *g, int B, int max_seq, int kvt) {
   for (int l = 0; l < c.n_layer; l++) {
     const DevLayer &L = g->layers[l];
     const float *fo = fold ? g->fold.as<float>() + per * l : nullptr;
-    GemmArgs ga = gemm_args(g, L.attn, g->bh.act(), B);
+    GemmArgs ga = gemm_args(g, g->qls[4 * (size_t)l], g->bh.act(), B);
     if (fold)
       ga.fold = FoldIn{X, L.ln1_w, fo, fo + 3 * d};
     else
@@ -887,23 +893,23 @@ itts_status enqueue_step_batch(itts_gpt *g, int B, int max_seq, int kvt) {
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiQKV, kvt, s));
     HIP_TRY(launch_decode_batch_rows(g->bq.as<float>(), seqs, B, layer_elems * l, c.n_head, max_seq, g->ba.out(),
                                      kvt, s));
-    ga = gemm_args(g, L.proj, g->ba.act(), B);
+    ga = gemm_args(g, g->qls[4 * (size_t)l + 1], g->ba.act(), B);
     ga.y = X;
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kvt, s));
-    ga = gemm_args(g, L.fc, g->bh.act(), B);
+    ga = gemm_args(g, g->qls[4 * (size_t)l + 2], g->bh.act(), B);
     if (fold)
       ga.fold = FoldIn{X, L.ln2_w, fo + 6 * d, fo + 6 * d + c.d_ffn};
     else
       HIP_TRY(launch_ln_rows(X, L.ln2_w, L.ln2_b, B, d, g->bh.out(), s));
     ga.xo = g->bf.out();
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiGelu, kvt, s));
-    ga = gemm_args(g, L.mproj, g->bf.act(), B);
+    ga = gemm_args(g, g->qls[4 * (size_t)l + 3], g->bf.act(), B);
     ga.y = X;
     HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kvt, s));
   }
   HIP_TRY(launch_ln_rows(X, g->ln_f_w.as<float>(), g->ln_f_b.as<float>(), B, d, g->bh.out(), s, g->fn_w.as<float>(),
                          g->fn_b.as<float>()));
-  GemmArgs ga = gemm_args(g, g->head, g->bh.act(), B);
+  GemmArgs ga = gemm_args(g, g->qls[4 * (size_t)c.n_layer], g->bh.act(), B);
   ga.y = g->blog.as<float>();
   HIP_TRY(launch_gemm(ga, bits, pt, kEpiStore, kvt, s));
   HIP_TRY(launch_advance_batch(seqs, B, s));
@@ -2082,16 +2088,9 @@ itts_status itts_qlinear_forward(itts_gpt *gpt, const itts_qlinear *ql, int32_t 
     SplitBuf xs;
     HIP_TRY(xs.ensure(M, K));
     HIP_TRY(launch_split_rows(dx.as<float>(), M, K, xs.out(), gpt->stream));
-    GemmArgs a{};
-    a.ql = q.dev();
-    a.x = xs.act();
-    a.M = M;
+    if (M <= 8) HIP_TRY(q.ready_rows(bits, pt, gpt->stream));
+    GemmArgs a = gemm_args(gpt, q, xs.act(), M);
     a.y = dy.as<float>();
-    a.ws = gpt->gws.as<float>();
-    a.ws_floats = gpt->gws.bytes / sizeof(float);
-    a.cnt = gpt->gcnt.as<uint32_t>();
-    a.cnt_words = kGemmCounters;
-    a.n_cu = gpt->n_cu;
     HIP_TRY(launch_gemm(a, bits, pt, kEpiStore, kKvBf16, gpt->stream));
     HIP_TRY(hipStreamSynchronize(gpt->stream));
   }
