@@ -119,10 +119,6 @@ struct AttnProbe {
 // [n_head][M][64]): writes only the probabilities, for rows p.q0..M-1.
 hipError_t launch_attn_probe(const float *q, int M, const int *kstart, const void *kc, const void *vc, int n_head,
                              const AttnProbe &p, int kvt, hipStream_t s);
-// Causal attention of T rows at cache positions base..base+T-1, one 64-lane block per
-// (head, row) (short prompts); the output rows are written in the GEMM's split form.
-hipError_t launch_attn_prefill(const float *q, int T, int base, const void *kc, const void *vc,
-                               int n_head, int max_seq, const SplitOut &out, int kvt, hipStream_t s);
 // out[r] = log_softmax(logits[r])[codes[r]] for R rows of V logits.
 hipError_t launch_log_softmax_pick(const float *logits, int R, int V, const int *codes, float *out, hipStream_t s);
 
@@ -135,23 +131,6 @@ struct FoldIn {
   const float *x, *gamma, *G, *c;
 };
 
-// The same fold in the tiled product (any M): the input planes already hold gamma * x
-// (written by the residual product before it, TileFoldOut), st[m][K/64] holds the mean
-// and the sum of squared deviations of each 64-column group of row m of x, and the
-// epilogue applies rstd (sum - mean G[n]) + c[n] with the row's statistics combined from
-// its groups (equal-size groups: mean of the means, M2 = sum M2_g + 64 sum (mean_g - mean)^2).
-struct TileFoldIn {
-  const float2 *st;
-  const float *G, *c;
-};
-// Residual epilogue that also writes the next folded LayerNorm's input from the updated
-// rows x: gamma * x in split form (planes and group sums) and the group statistics of x.
-struct TileFoldOut {
-  SplitOut o;
-  const float *gamma;
-  float2 *st;       // [M][N/64]
-};
-
 struct GemmArgs {
   DevQL ql;
   // few-row products: the codes in fragment order and the (scale, bias) words [K/64][ldn]
@@ -160,8 +139,6 @@ struct GemmArgs {
   int ldn;
   SplitAct x;       // [M][K] (unused with fold.x)
   FoldIn fold;      // fold.x set: the input is LayerNorm(x) by the fold above
-  TileFoldIn tfi;   // tfi.st set (tiled product, QKV or GELU epilogue): folded LayerNorm input
-  TileFoldOut tfo;  // tfo.st set (tiled product, residual epilogue): write the next fold's input
   int M;
   float *y;         // [M][N] (store) or residual stream [M][N] (resid)
   SplitOut xo;      // gelu: the next GEMM's input [M][N] (N a multiple of 64)
@@ -217,7 +194,11 @@ struct RowsMm {
   float *q_out;
   void *kc, *vc;
   int max_seq, n_cu;
-  int nM, nN, gm;  // tile grid, set at the launch
+  float *ws;       // partial tiles and counters of products whose K is split over blocks (as in GemmArgs)
+  size_t ws_floats;
+  uint32_t *cnt;
+  int cnt_words;
+  int nM, nN, gm, S;  // tile grid and K split, set at the launch
 };
 hipError_t rows_mm(const RowsMm &a, int bits, int epi, int kvt, hipStream_t s);
 // Causal attention: row t attends to keys kstart[t] (or 0) .. t; order (optional) lists the

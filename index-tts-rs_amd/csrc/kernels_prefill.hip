@@ -1,4 +1,6 @@
-// Prefill GEMM for gfx950, the activation splitter and the standalone dequantiser.
+// GEMM over row-major split activations for gfx950 (batched decode steps: 9 sequences and more on
+// the tiles, up to 8 on the few-row product), the activation splitter and the standalone
+// dequantiser.
 //
 // The GEMM contracts M activation rows against the int8 (or int4) codes on the MFMA
 // units (v_mfma_f32_32x32x16_f16).  Codes are exact in fp16, so the matrix cores see the
@@ -365,70 +367,12 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
 
   if (copier)
     for (int i = 0; i < NS - 1 && i < ng; i++) issue(g0 + i, stage(i));
-  // Folded LayerNorm input: each row's mean and rstd from its groups' statistics.  A quad of
-  // worker lanes a row (64 rows per pass of the four worker waves), lane p of the quad
-  // holding groups p, p + 4, ... (K <= 2048: at most 8), the quad's sums formed by two DPP
-  // quad permutes.  On 64-row tiles the loads are issued here, before the K loop (nothing
-  // else of the workers' waits on the vector-memory counter), and reduced after it; 128-row
-  // tiles (no registers to spare) load after the loop.
-  constexpr bool kFoldIn = EPI == kEpiQKV || EPI == kEpiGelu;
-  constexpr int kFoldGpl = 8;  // groups a lane
-  constexpr bool kFoldEarly = kFoldIn && TM == 1;
-  __shared__ float2 fold_row[kFoldIn ? BM : 1];
-  const bool fin = kFoldIn && a.tfi.st != nullptr;
-  float2 fv[kFoldEarly ? kFoldGpl : 1];
-  auto fold_load = [&](int pass, float2 *v) __attribute__((always_inline)) {
-    const int m = min(m0 + pass * 64 + ((tid & 255) >> 2), M - 1), p = tid & 3;
-#pragma unroll
-    for (int i = 0; i < kFoldGpl; i++) {
-      const int g = p + 4 * i;
-      v[i] = g < G ? a.tfi.st[(size_t)m * G + g] : make_float2(0.0f, 0.0f);
-    }
-  };
-  auto fold_reduce = [&](int pass, const float2 *v) __attribute__((always_inline)) {
-    const int p = tid & 3;
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kFoldGpl; i++) sum += v[i].x;
-    sum += dpp_pair<0xB1>(sum);  // quad_perm [1,0,3,2]
-    sum += dpp_pair<0x4E>(sum);  // quad_perm [2,3,0,1]
-    const float mean = sum / (float)G;
-    float m2 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kFoldGpl; i++) {
-      const float dm = v[i].x - mean;
-      if (p + 4 * i < G) m2 += v[i].y + 64.0f * (dm * dm);
-    }
-    m2 += dpp_pair<0xB1>(m2);
-    m2 += dpp_pair<0x4E>(m2);
-    if (p == 0) fold_row[pass * 64 + ((tid & 255) >> 2)] = make_float2(mean, 1.0f / sqrtf(m2 / (float)K + 1e-5f));
-  };
-  if constexpr (kFoldEarly) {
-    if (fin && worker) fold_load(0, fv);
-  }
-  // The epilogue's column constants on 64 x 64 tiles (one 32-column MFMA tile a wave): the
-  // bias (or the folded LayerNorm's c) and the folded G of the lane's column, loaded here so
-  // the epilogue does not start with a memory round trip.  Addresses selected, not loads
-  // predicated (a load behind a branch would make the compiler wait for the fold loads).
+  // The bias of the lane's column on 64 x 64 tiles (one 32-column MFMA tile a wave), loaded here
+  // so the epilogue does not start with a memory round trip.
   constexpr bool kColEarly = PROD && TM == 1 && TN == 1;
-  float cb = 0.0f, cg = 0.0f;
+  float cb = 0.0f;
   if constexpr (kColEarly) {
-    if (worker) {
-      const int n = min(n0 + wn * 32 + (lane & 31), N - 1);
-      cb = gload((kFoldIn && fin ? a.tfi.c : a.ql.bias) + n);
-      if constexpr (kFoldIn) cg = gload((fin ? a.tfi.G : a.ql.bias) + n);
-    }
-  }
-  // ... and the residual fold-out's gamma: worker thread t takes columns 16 (t & 3) .. +15
-  // of the tile (its item in the epilogue below), the same for every row
-  constexpr bool kGamEarly = kColEarly && EPI == kEpiResid;
-  float gam0[kGamEarly ? 16 : 1];
-  if constexpr (kGamEarly) {
-    if (worker && a.tfo.st) {
-      const float *gp = a.tfo.gamma + n0 + (tid & 3) * 16;
-#pragma unroll
-      for (int c = 0; c < 16; c++) gam0[c] = gload(gp + c);
-    }
+    if (worker) cb = gload(a.ql.bias + min(n0 + wn * 32 + (lane & 31), N - 1));
   }
   int i = 0;
   for (; i + 1 < ng; i += 2) {
@@ -440,22 +384,6 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     if (worker && !PROD) apply(P0);
   } else {
     if (worker && !PROD) apply(P1);
-  }
-
-  if constexpr (kFoldIn) {
-    if (fin && worker) {
-      if constexpr (kFoldEarly) {
-        fold_reduce(0, fv);
-      } else {
-#pragma unroll
-        for (int pass = 0; pass < TM; pass++) {
-          float2 v[kFoldGpl];
-          fold_load(pass, v);
-          fold_reduce(pass, v);
-        }
-      }
-    }
-    if (fin) __syncthreads();  // rows reduced by one wave are read by the others
   }
 
   // Residual epilogues on 64-row tiles: the lane's old rows y, all loaded before any is
@@ -555,111 +483,6 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
 
   if (kResid && S == 1 && TM == 1 && worker) load_y();
 
-  if constexpr (EPI == kEpiResid) {
-    if (a.tfo.st) {
-      // The updated rows x staged in LDS, then per (row, 64-column group): the group's mean
-      // and sum of squared deviations of x, and gamma * x as the next GEMM's input (hi/lo
-      // planes and the group sum).
-      constexpr int LDT = BN + 1;
-      constexpr int GPR = BN / 64, ITEMS = BM * GPR, TPI = 256 / ITEMS, VPT = 64 / TPI;
-      static_assert(ITEMS * TPI == 256 && VPT % 8 == 0, "fold epilogue shape");
-      float *T = reinterpret_cast<float *>(lds);
-      // this thread's item (row rl, 64-column group grp, values c0 .. c0 + VPT - 1); its
-      // gamma values (16-byte aligned: the vector starts on 256 bytes and c0 is a multiple
-      // of 16) are loaded under the staging below on 64-row tiles, after it on 128-row
-      // tiles (whose registers the staged tile still holds)
-      const int item = tid / TPI, sub = tid % TPI;
-      const int rl = item / GPR, grp = item % GPR;
-      const int c0 = grp * 64 + sub * VPT;
-      // N is a multiple of 64: a group is wholly in or out
-      const bool live = worker && m0 + rl < M && n0 + c0 < N;
-      float4 gam[VPT / 4];
-      auto load_gamma = [&]() __attribute__((always_inline)) {
-        if constexpr (kGamEarly) {
-          static_assert(VPT == 16 && TPI == 4, "gamma loaded before the K loop for 16-column items");
-#pragma unroll
-          for (int c = 0; c < 4; c++) gam[c] = make_float4(gam0[4 * c], gam0[4 * c + 1], gam0[4 * c + 2], gam0[4 * c + 3]);
-        } else {
-#pragma unroll
-          for (int c = 0; c < VPT / 4; c++)
-            gam[c] = live ? reinterpret_cast<const float4 *>(a.tfo.gamma + n0 + c0)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-      };
-      if constexpr (TM == 1) load_gamma();
-      __syncthreads();
-      if (worker)
-#pragma unroll
-        for (int i2 = 0; i2 < TM; i2++)
-#pragma unroll
-          for (int j = 0; j < TN; j++) {
-            const int cl = wn * 32 * TN + j * 32 + (lane & 31), n = n0 + cl;
-            if (n >= N) continue;
-            const float bias = kColEarly ? cb : a.ql.bias[n];
-            const int rb = wm * 32 * TM + i2 * 32 + (lane >> 5) * 4;  // tile row of element 0
-            // values first (straight-line), then the stores predicated on the row
-            float outv[16];
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const float y = TM == 1 ? yv[i2][j][e]
-                                      : gload(a.y + (size_t)min(m0 + rb + (e >> 2) * 8 + (e & 3), M - 1) * N + n);
-              outv[e] = y + (acc[i2][j][e] + bias);
-              T[(rb + (e >> 2) * 8 + (e & 3)) * LDT + cl] = outv[e];
-            }
-#pragma unroll
-            for (int e = 0; e < 16; e++) asm volatile("" : "+v"(outv[e]));
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
-              if (m < M) gstore(a.y + (size_t)m * N + n, outv[e]);
-            }
-          }
-      __syncthreads();
-      if constexpr (TM != 1) load_gamma();
-      if (worker) {
-        const int m = m0 + rl, n = n0 + c0;
-        float xv[VPT];
-        float sum = 0.0f;
-#pragma unroll
-        for (int c = 0; c < VPT; c++) {
-          xv[c] = T[rl * LDT + c0 + c];
-          sum += xv[c];
-        }
-        sum = item_sum<TPI>(sum);
-        const float mean = sum / 64.0f;
-        float m2 = 0.0f, gsum = 0.0f;
-#pragma unroll
-        for (int c = 0; c < VPT; c += 8) {
-          uint32_t hw[4], lw[4];
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const float v0 = xv[c + e], v1 = xv[c + e + 1];
-            const float d0 = v0 - mean, d1 = v1 - mean;
-            m2 += d0 * d0;
-            m2 += d1 * d1;
-            const float4 gq = gam[(c + e) >> 2];
-            const float g0 = ((e & 2) ? gq.z : gq.x) * v0;
-            const float g1 = ((e & 2) ? gq.w : gq.y) * v1;
-            gsum += g0;
-            gsum += g1;
-            split_f16x2(g0, g1, hw[e >> 1], lw[e >> 1]);
-          }
-          if (live) {
-            gstore(reinterpret_cast<uint4 *>(a.tfo.o.hi + (size_t)m * N + n + c), make_uint4(hw[0], hw[1], hw[2], hw[3]));
-            gstore(reinterpret_cast<uint4 *>(a.tfo.o.lo + (size_t)m * N + n + c), make_uint4(lw[0], lw[1], lw[2], lw[3]));
-          }
-        }
-        m2 = item_sum<TPI>(m2);
-        gsum = item_sum<TPI>(gsum);
-        if (live && sub == 0) {
-          const size_t gi = (size_t)m * (N / kGroup) + (n0 + grp * 64) / kGroup;
-          gstore(a.tfo.o.gs + gi, gsum);
-          gstore(a.tfo.st + gi, make_float2(mean, m2));
-        }
-      }
-      return;
-    }
-  }
-
   if constexpr (EPI == kEpiGelu) {
     // GELU tile staged in LDS, then written as the next GEMM's input: hi/lo planes and
     // the per-64-column row sums
@@ -673,14 +496,11 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
       for (int j = 0; j < TN; j++) {
         const int cl = wn * 32 * TN + j * 32 + (lane & 31);
         const bool nl = n0 + cl < N;
-        const float bias = kColEarly ? cb : nl ? (fin ? a.tfi.c[n0 + cl] : a.ql.bias[n0 + cl]) : 0.0f;
-        const float gn = kColEarly ? (fin ? cg : 0.0f) : fin && nl ? a.tfi.G[n0 + cl] : 0.0f;
+        const float bias = kColEarly ? cb : nl ? a.ql.bias[n0 + cl] : 0.0f;
 #pragma unroll
         for (int e = 0; e < 16; e++) {
           const int rl = wm * 32 * TM + i2 * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          float v = acc[i2][j][e];
-          if (fin) v = fold_row[rl].y * (v - fold_row[rl].x * gn);
-          T[rl * LDT + cl] = gelu_tanh_exp(v + bias);
+          T[rl * LDT + cl] = gelu_tanh_exp(acc[i2][j][e] + bias);
         }
       }
     __syncthreads();
@@ -719,8 +539,7 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
       for (int j = 0; j < TN; j++) {
         const int n = n0 + wn * 32 * TN + j * 32 + (lane & 31);
         if (n >= N) continue;
-        const float bias = kColEarly ? cb : fin ? a.tfi.c[n] : a.ql.bias[n];
-        const float gn = kColEarly ? (fin ? cg : 0.0f) : fin ? a.tfi.G[n] : 0.0f;
+        const float bias = kColEarly ? cb : a.ql.bias[n];
         const int rb = wm * 32 * TM + i2 * 32 + (lane >> 5) * 4;  // tile row of element 0
         // 128-row tiles: the sub-tile's 16 old values loaded together (registers for all 64
         // of the lane's would spill)
@@ -736,10 +555,7 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
         float outv[16];
 #pragma unroll
         for (int e = 0; e < 16; e++) {
-          const int rl = rb + (e >> 2) * 8 + (e & 3);
-          float v = acc[i2][j][e];
-          if constexpr (kFoldIn) v = fin ? fold_row[rl].y * (v - fold_row[rl].x * gn) : v;
-          v += bias;
+          float v = acc[i2][j][e] + bias;
           if constexpr (kResid) v = (TM == 1 ? yv[i2][j][e] : ysub[e]) + v;
           outv[e] = v;
         }
@@ -1328,13 +1144,7 @@ hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt,
         (epi != kEpiQKV && epi != kEpiGelu) || !a.fold.gamma || !a.fold.G || !a.fold.c)
       return hipErrorInvalidValue;
   }
-  if (a.tfi.st && ((epi != kEpiQKV && epi != kEpiGelu) || a.ql.K > 32 * kGroup || !a.tfi.G || !a.tfi.c || a.fold.x))
-    return hipErrorInvalidValue;
-  if (a.tfo.st && (epi != kEpiResid || a.ql.N % kGroup != 0 || !a.tfo.gamma || !a.tfo.o.hi || !a.tfo.o.lo ||
-                   !a.tfo.o.gs || a.fold.x))
-    return hipErrorInvalidValue;
-  // (the tiled folds are written for the tiled product only)
-  if (a.M <= kFewRows && (bits == 8 || bits == 4) && !a.tfi.st && !a.tfo.st && a.fcodes) {
+  if (a.M <= kFewRows && (bits == 8 || bits == 4) && a.fcodes) {
     // a group per wave while that keeps the splits within kFewMaxSplits (gw > kFewMaxGw
     // beyond that: the tiled GEMM)
     const int nN = (a.ql.N + 63) / 64, G = a.ql.K / kGroup;

@@ -148,6 +148,7 @@ __global__ __launch_bounds__(256) void rows_codes_kernel(const uint8_t *codes, i
 // Block: one tile of BM = 32 TM rows x 64 columns by KS waves that split the K groups, their
 // partial tiles added through LDS (two halves of the waves at a time).  A wave keeps CH
 // groups of activation fragments, codes and scales in flight.
+constexpr int kMaxSplit = 6;  // blocks that may share a tile's K
 template <int TM_, int KS_, int CH_>
 struct RmCfg {
   static constexpr int TM = TM_, TN = 2, KS = KS_, CH = CH_;
@@ -192,12 +193,14 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r31 = lane & 31;
   const int kq = __builtin_amdgcn_readfirstlane(tid >> 6);
   // block -> tile: XCD x takes every gm-th row tile and every gn-th column tile
-  const int gn = 8 / a.gm, x = blockIdx.x & 7, jb = blockIdx.x >> 3, pn = (a.nN + gn - 1) / gn;
+  const int gn = 8 / a.gm, x = blockIdx.x & 7, pn = (a.nN + gn - 1) / gn, per = pn * ((a.nM + a.gm - 1) / a.gm);
+  const int jb = (blockIdx.x >> 3) % per, split = (blockIdx.x >> 3) / per;  // split: part of K (a.S of them)
   const int tm = jb / pn * a.gm + x % a.gm, tn = jb % pn * gn + x / a.gm;
   if (tm >= a.nM || tn >= a.nN) return;
   const int m0 = tm * BM, n0 = tn * BN;
   const int G = a.K / 64, nk = a.K / 16, nx = (G + 15) / 16, ns = nk + nx;
-  const int g0 = G * kq / KS, g1 = G * (kq + 1) / KS;
+  const int kk = split * KS + kq, KT = KS * a.S;
+  const int g0 = G * kk / KT, g1 = G * (kk + 1) / KT;
 
   // wave-uniform bases with 32-bit lane offsets (registers, not 64-bit addresses, are short here)
   const u32x4 *ab = reinterpret_cast<const u32x4 *>(a.x) + ((size_t)(m0 >> 5) * ns) * 128;
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
     }
   };
   // the bias term's steps first (their loads go out ahead of the rings')
-  const int x0 = nx * kq / KS, x1 = nx * (kq + 1) / KS;
+  const int x0 = nx * kk / KT, x1 = nx * (kk + 1) / KT;
   for (int kx = x0; kx < x1; kx++) {
     u32x4 xa[TM][2], xb[TN][2];
 #pragma unroll
@@ -434,6 +437,73 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] += cadd[e];
   };
+  // K over a.S blocks (residual products): each stores its partial tile through agent-scope
+  // accesses (coherent across the XCDs' L2s); the last to arrive (wrapping counter) adds the
+  // others' in split order, so the result does not depend on arrival.
+  __shared__ uint32_t last_flag;
+  float4 sum[EPI == kEpiResid ? IT : 1][2];
+  if constexpr (EPI == kEpiResid) {
+    if (a.S > 1) {
+      const int tile = tm * a.nN + tn;
+      uint64_t *ws = reinterpret_cast<uint64_t *>(a.ws + (size_t)tile * a.S * (BM * 64));
+      auto raw = [&](int q, float4(&o)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+          const float *p = red + (size_t)(q >> 3) * LD + (q & 7) * 8 + 4 * w;
+          float4 t = *reinterpret_cast<const float4 *>(p);
+#pragma unroll
+          for (int k = 1; k < KL; k++) {
+            const float4 u = *reinterpret_cast<const float4 *>(p + (size_t)k * BM * LD);
+            t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
+          }
+          o[w] = t;
+        }
+      };
+      // word w of item q: [split][w][q], consecutive lanes on consecutive words
+      constexpr int ITEMS_ = BM * 8;
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+        const int q = tid + i * NT;
+        if (q >= ITEMS_) break;
+        raw(q, sum[i]);
+        const float f[8] = {sum[i][0].x, sum[i][0].y, sum[i][0].z, sum[i][0].w,
+                            sum[i][1].x, sum[i][1].y, sum[i][1].z, sum[i][1].w};
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+          __hip_atomic_store(ws + ((size_t)split * 4 + w) * ITEMS_ + q,
+                             __builtin_bit_cast(uint64_t, make_float2(f[2 * w], f[2 * w + 1])), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) last_flag = atomicInc(a.cnt + tile, (uint32_t)(a.S - 1)) == (uint32_t)(a.S - 1) ? 1u : 0u;
+      __syncthreads();
+      if (!last_flag) return;
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+        const int q = tid + i * NT;
+        if (q >= ITEMS_) break;
+        float2 p[kMaxSplit][4];
+#pragma unroll
+        for (int s2 = 0; s2 < kMaxSplit; s2++)
+#pragma unroll
+          for (int w = 0; w < 4; w++)
+            p[s2][w] = s2 < a.S ? __builtin_bit_cast(float2, __hip_atomic_load(ws + ((size_t)s2 * 4 + w) * ITEMS_ + q,
+                                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                : make_float2(0.0f, 0.0f);
+        float2 t[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          t[w] = p[0][w];
+#pragma unroll
+          for (int s2 = 1; s2 < kMaxSplit; s2++)
+            if (s2 < a.S) t[w].x += p[s2][w].x, t[w].y += p[s2][w].y;
+        }
+        sum[i][0] = make_float4(t[0].x, t[0].y, t[1].x, t[1].y);
+        sum[i][1] = make_float4(t[2].x, t[2].y, t[3].x, t[3].y);
+      }
+    }
+  }
   constexpr int ITEMS = BM * 8;
   if constexpr (EPI == kEpiStore) {
     for (int q = tid; q < ITEMS; q += NT) {
@@ -458,7 +528,14 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       if (q >= ITEMS) break;  // whole waves
       const bool live = r < a.M;
       float v[8];
-      tile8(row, c * 8, v);
+      if (a.S > 1) {
+        const float4 t0 = sum[i][0], t1 = sum[i][1];
+        const float f[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = f[e] + cadd[e];
+      } else {
+        tile8(row, c * 8, v);
+      }
       float4 *o = reinterpret_cast<float4 *>(a.y + (size_t)min(r, a.M - 1) * a.N + n);
       const float4 p = old[i][0], t = old[i][1];
       const float yv[8] = {p.x, p.y, p.z, p.w, t.x, t.y, t.z, t.w};
@@ -690,26 +767,37 @@ hipError_t run(RowsMm a, hipStream_t s) {
   a.nM = (a.M + C::BM - 1) / C::BM;
   a.nN = (a.N + C::BN - 1) / C::BN;
   a.gm = xcd_rows(a.nM, a.nN, 4.0 * C::BM * a.K, (double)C::BN * a.K * BITS / 8);
-  const int gn = 8 / a.gm, blocks = 8 * ((a.nM + a.gm - 1) / a.gm) * ((a.nN + gn - 1) / gn);
+  if (a.S < 1 || EPI != kEpiResid || !a.ws || !a.cnt || a.nM * a.nN > a.cnt_words ||
+      (size_t)a.nM * a.nN * a.S * C::BM * 64 > a.ws_floats)
+    a.S = 1;
+  const int gn = 8 / a.gm, blocks = 8 * ((a.nM + a.gm - 1) / a.gm) * ((a.nN + gn - 1) / gn) * a.S;
   hipLaunchKernelGGL((rows_mm_kernel<BITS, EPI, KVT, C>), dim3(blocks), dim3(C::NT), C::LDS, s, a);
   return hipGetLastError();
 }
 
-// 32 x 64 tiles by four waves; by eight where K is long and the tiles few, 64 x 64 tiles where K is
-// long and the tiles many.  M x N x K in us, 32 x 64 by four / by eight / 64 x 64: 35 x 1280 x 1280
-// 7.2 / 7.5 / 10.1, 35 x 1280 x 5120 16.0 / 14.8 / 22.6, 235 x 1280 x 5120 17.0 / 15.9 / 23.5, 235 x
-// 5120 x 1280 13.5 / 18.9 / 16.4, 886 x 5120 x 1280 32.7 (355 TFLOP/s) / 52.5 / 34.4, 886 x 1280 x
-// 5120 34.5 / 44.3 / 42.3, 2188 x 5120 x 1280 72.5 / 122 / 72.4, 2188 x 1280 x 5120 69.7 / 88.4 / 62.5
-// (459 TFLOP/s, 918 of fp16 products).  (Two groups of codes in flight instead of one: 10-40 %
-// slower, fewer waves in flight.)
+// 32 x 64 tiles by four waves; 64 x 64 where K is long and the tiles many.  M x N x K in us, 32 x
+// 64 / 64 x 64: 35 x 1280 x 1280 7.2 / 10.1, 235 x 5120 x 1280 13.5 / 16.4, 886 x 5120 x 1280 32.7
+// (355 TFLOP/s) / 34.4, 886 x 1280 x 5120 34.5 / 42.3, 2188 x 5120 x 1280 72.5 / 72.4, 2188 x 1280 x
+// 5120 69.7 / 62.5 (459 TFLOP/s, 918 of fp16 products).  (Two groups in flight instead of one
+// gain nothing, eight waves on a tile lose wherever K is not split instead.)
 using RmSmall = RmCfg<1, 4, 1>;
-using RmLong = RmCfg<1, 8, 1>;
 using RmLarge = RmCfg<2, 4, 1>;
 
 template <int BITS, int EPI, int KVT>
-hipError_t pick(const RowsMm &a, hipStream_t s) {
+hipError_t pick(RowsMm a, hipStream_t s) {
   const long tn = (a.N + 63) / 64, t32 = (a.M + 31) / 32 * tn, t64 = (a.M + 63) / 64 * tn;
-  if (a.K >= 4096 && 4 * t32 <= 5L * a.n_cu) return run<BITS, EPI, KVT, RmLong>(a, s);
+  // A long K over S blocks a tile, where the tiles alone leave compute units idle: the S with the
+  // least blocks-per-unit / S, plus what storing and adding a partial costs (mlp c_proj, whole
+  // prefill in us, unsplit / split: 20 rows 1467 / 1198, 99 rows 1445 / 1256, 200 rows 1640 / 1538;
+  // from about two blocks a compute unit on the partials cost what the balance gains).
+  a.S = 1;
+  if (EPI == kEpiResid && a.K >= 4096 && t32 <= 2L * a.n_cu) {
+    double best = 1e30;
+    for (int S = 1; S <= kMaxSplit; S++) {
+      const double cost = (double)((t32 * S + a.n_cu - 1) / a.n_cu) / S + 0.07 * S;
+      if (cost < best) best = cost, a.S = S;
+    }
+  }
   if (a.K >= 4096 && t64 >= 2L * a.n_cu) return run<BITS, EPI, KVT, RmLarge>(a, s);
   return run<BITS, EPI, KVT, RmSmall>(a, s);
 }

@@ -195,11 +195,10 @@ struct itts_gpt {
   itts_decode_path path = ITTS_DECODE_AUTO;
   // decode workspace
   DevBuf x, q, a, f, logits;
-  // prefill workspace (grown on demand): residual stream and q (fp32), GEMM inputs in
-  // split form (LN output, attention output, GELU output), split-K partials and counters
+  // prefill workspace (grown on demand): residual stream and probed q (fp32), split-K partials
+  // and counters
   DevBuf px, pq, rows, conds;
   HostStage h_rows, h_conds;  // their pinned host staging
-  SplitBuf ph, pa, pf;
   // the folded LayerNorms' group statistics of the residual rows [M][d/64] (mean, M2)
   DevBuf pst;
   DevBuf gws, gcnt;
@@ -334,12 +333,6 @@ GemmArgs gemm_args(const itts_gpt *g, const QLHost &q, SplitAct x, int M) {
   return ga;
 }
 
-// Prompts of more than this many rows run on operands in fragment order (kernels_rows.hip), fewer
-// on the 64 x 64 tiles whose K is split over blocks (kernels_prefill.hip).  Whole prefill in us,
-// fragments / tiles: 20 rows 1423 / 1329, 35 rows 1392 / 1373, 64 rows 1406 / 1435, 99 rows 1405 /
-// 1544, 235 rows 1630 / 2005.
-constexpr int kRowsMin = 48;
-
 // Grows buf to the planes of M rows of K values, zero where nothing is written.
 hipError_t ensure_planes(itts_gpt *g, DevBuf &buf, int M, int K) {
   const size_t bytes = sizeof(uint4) * rows_planes_pieces(M, K);
@@ -358,6 +351,10 @@ RowsMm rows_args(const itts_gpt *g, const QLHost &q, const DevBuf &x, int M) {
   a.bw = q.rbias.as<uint4>();
   a.bias = q.bias.as<float>();
   a.ldn = rows_ldn(q.N);
+  a.ws = g->gws.as<float>();
+  a.ws_floats = g->gws.bytes / sizeof(float);
+  a.cnt = g->gcnt.as<uint32_t>();
+  a.cnt_words = kGemmCounters;
   a.M = M;
   a.N = q.N;
   a.K = q.K;
@@ -378,37 +375,8 @@ itts_status ensure_rows(itts_gpt *g, int M) {
   HIP_TRY(ensure_planes(g, g->ff, M, g->cfg.d_ffn));
   HIP_TRY(g->fq.ensure(sizeof(uint4) * rows_q_pieces(M, g->cfg.n_head)));
   HIP_TRY(g->fkv.ensure(sizeof(uint4) * rows_kv_pieces(M, g->cfg.n_head)));
-  if (M > kRowsMin) return ITTS_OK;
-  HIP_TRY(g->ph.ensure(M, d));
-  HIP_TRY(g->pq.ensure(sizeof(float) * (size_t)M * d));
-  HIP_TRY(g->pa.ensure(M, d));
-  HIP_TRY(g->pf.ensure(M, g->cfg.d_ffn));
   return ITTS_OK;
 }
-
-// LayerNorms of a short prompt's stack after layer 0's ln_1 folded into the products: each
-// residual product writes gamma * x of the next LayerNorm in split form with the group
-// statistics of x (TileFoldOut), and the QKV / c_fc product applies them (TileFoldIn).
-// Layer 0's ln_1 input comes from the embeddings and keeps its row kernel.  d <= 2048 (the
-// statistics' reduction holds at most 32 groups a row).
-struct StackFold {
-  bool on;
-  size_t per;
-  const float *fold;
-  float2 *st;
-  int d, F;
-  explicit StackFold(const itts_gpt *g) {
-    d = g->cfg.d_model;
-    F = g->cfg.d_ffn;
-    on = g->fold.p != nullptr && d % kGroup == 0 && d <= 32 * kGroup;
-    per = fold_floats(d, F);
-    fold = g->fold.as<float>();
-    st = g->pst.as<float2>();
-  }
-  TileFoldIn qkv(int l) const { return TileFoldIn{st, fold + per * l, fold + per * l + 3 * d}; }
-  TileFoldIn fc(int l) const { return TileFoldIn{st, fold + per * l + 6 * d, fold + per * l + 6 * d + F}; }
-  TileFoldOut out(const SplitBuf &b, const float *gamma) const { return TileFoldOut{b.out(), gamma, st}; }
-};
 
 itts_status validate_prefix(const itts_config &c, const int32_t *text, int32_t n_text,
                             const float *conds, int32_t n_cond, int32_t max_cond, int32_t lang,
@@ -564,38 +532,10 @@ itts_status enqueue_prefill_stack(itts_gpt *g, itts_kv *kv, int T) {
   const itts_config &c = g->cfg;
   const int d = c.d_model, bits = c.quant_bits, pt = g->ptype();
   hipStream_t s = g->stream;
-  float *X = g->px.as<float>(), *Q = g->pq.as<float>();
-  auto gemm = [&](size_t i, SplitAct x) { return gemm_args(g, g->qls[i], x, T); };
-  if (T > kRowsMin) {
-    if (itts_status st = rows_stack(g, kv, T, c.n_layer, nullptr, nullptr, {})) return st;
-  }
-  const StackFold sf(g);
-  for (int l = 0; T <= kRowsMin && l < c.n_layer; l++) {
-    const DevLayer &L = g->layers[l];
-    if (!sf.on || l == 0) HIP_TRY(launch_ln_rows(X, L.ln1_w, L.ln1_b, T, d, g->ph.out(), s));
-    GemmArgs ga = gemm(4 * (size_t)l, g->ph.act());
-    if (sf.on && l > 0) ga.tfi = sf.qkv(l);
-    ga.qkv = QkvDst{Q, kv->k_layer(l), kv->v_layer(l), kv->max_seq, 0, d};
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiQKV, kv->kvt, s));
-    HIP_TRY(launch_attn_prefill(Q, T, 0, kv->k_layer(l), kv->v_layer(l), c.n_head, kv->max_seq, g->pa.out(),
-                                kv->kvt, s));
-    ga = gemm(4 * (size_t)l + 1, g->pa.act());
-    ga.y = X;
-    if (sf.on) ga.tfo = sf.out(g->ph, L.ln2_w);
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kv->kvt, s));
-    if (!sf.on) HIP_TRY(launch_ln_rows(X, L.ln2_w, L.ln2_b, T, d, g->ph.out(), s));
-    ga = gemm(4 * (size_t)l + 2, g->ph.act());
-    if (sf.on) ga.tfi = sf.fc(l);
-    ga.xo = g->pf.out();
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiGelu, kv->kvt, s));
-    ga = gemm(4 * (size_t)l + 3, g->pf.act());
-    ga.y = X;
-    if (sf.on && l + 1 < c.n_layer) ga.tfo = sf.out(g->ph, g->layers[l + 1].ln1_w);
-    HIP_TRY(launch_gemm(ga, bits, pt, kEpiResid, kv->kvt, s));
-  }
+  if (itts_status st = rows_stack(g, kv, T, c.n_layer, nullptr, nullptr, {})) return st;
   GemvArgs ha{};
   ha.ql = g->head;
-  ha.x = X + (size_t)(T - 1) * d;
+  ha.x = g->px.as<float>() + (size_t)(T - 1) * d;
   ha.ln_w = g->ln_f_w.as<float>();
   ha.ln_b = g->ln_f_b.as<float>();
   ha.ln2_w = g->fn_w.as<float>();
@@ -2075,7 +2015,7 @@ itts_status itts_qlinear_forward(itts_gpt *gpt, const itts_qlinear *ql, int32_t 
     a.x = dx.as<float>();
     a.y = dy.as<float>();
     HIP_TRY(launch_gemv(a, bits, pt, kProNone, kEpiStore, kKvBf16, gpt->stream));
-  } else if (M > kRowsMin) {
+  } else if (M > 64) {
     DevBuf planes;
     HIP_TRY(ensure_planes(gpt, planes, M, K));
     HIP_TRY(q.ready_rows(bits, pt, gpt->stream));
