@@ -6,8 +6,10 @@
 // v_mfma_f32_32x32x16_f16 per K step, and folds each 64-group's scale into an fp32
 // accumulator: acc += s[g, n] P.  The groups' bias term, sum_g b'[n, g] sum_{k in g} x[m, k]
 // with b' = b + 128 s (or 8 s), is itself a product over G more K values: the activation
-// planes carry the group sums as further K steps, the weights' b' planes hold the other
-// operand (both hi/lo, three products).
+// planes carry an eighth of the groups' sums as further K steps (the sums of 64 values up to 16376
+// fit fp16's hi/lo range; what an eighth rounds of tiny activations is no more than the activations'
+// own rounding), the weights' b' planes hold the other operand (both hi/lo, three products).  b' is scaled by a power of two a column, its largest in [2^13, 2^14): unscaled, b'
+// of 1e-4 keeps 12 bits of fp32 parameters (replay, error against 64 bits 5e-7 instead of 6e-8).
 //
 // Activation planes ("rows"): per 32-row block, K / 16 steps, then ceil(G / 16) steps of group
 // sums.  Inside a 64-group the K order is permuted so that a lane's codes of two steps are one
@@ -31,10 +33,10 @@ __device__ __forceinline__ size_t rows_piece(int row, int c, int ns) {
   const int step = (c >> 3) * 4 + ((c >> 2) & 1) * 2 + (c & 1);
   return (((size_t)(row >> 5) * ns + step) * 2) * 64 + (size_t)(((c >> 1) & 1) * 32 + (row & 31));
 }
-// the group sum of group g: element of the extra steps
+// an eighth of group g's sum v: element of the extra steps
 __device__ __forceinline__ void put_group_sum(u32x4 *o, int row, int g, int nk, int ns, float v) {
   uint32_t h, l;
-  split_f16(v, h, l);
+  split_f16(v * 0.125f, h, l);
   uint16_t *p = reinterpret_cast<uint16_t *>(o + (((size_t)(row >> 5) * ns + nk + (g >> 4)) * 2) * 64 +
                                              (size_t)(((g >> 3) & 1) * 32 + (row & 31))) +
                 (g & 7);
@@ -92,7 +94,8 @@ __global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const flo
 
 // ---- weights ----------------------------------------------------------------------------
 // scale [G][ldn] fp32 and the (scale, bias) words transposed alike (columns past N zero), and b' =
-// b + off s as fragment planes of G values
+// b + off s as fragment planes of G values, times 2^-e a column; row G of scale holds 8 2^e (8: the
+// planes meet eighths of sums)
 template <int PT>
 __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, int N, int G, int ldn, float off,
                                                           float *scale, u32x4 *bw, void *words) {
@@ -100,7 +103,17 @@ __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, in
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)ldn * nx * 2) return;
   const int n = (int)(i % ldn), g8 = (int)(i / ldn);
-  float v[8];
+  float v[8], top = 0.0f;
+  for (int g = 0; g < G && n < N; g++) {
+    const float2 sb = load_param<PT>(params, (size_t)n * G + g);
+    top = fmaxf(top, fabsf(fmaf(off, sb.x, sb.y)));
+  }
+  int e = 0;
+  if (top > 0.0f && top < INFINITY) {
+    frexpf(top, &e);  // top in [2^(e-1), 2^e)
+    e = max(e - 14, -120);
+  }
+  if (g8 == 0) scale[(size_t)G * ldn + n] = ldexpf(8.0f, e);
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const int g = g8 * 8 + j;
@@ -112,7 +125,7 @@ __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, in
       if constexpr (PT == kParamF32) static_cast<float2 *>(words)[i] = sb;
       else static_cast<uint32_t *>(words)[i] = n < N ? static_cast<const uint32_t *>(params)[(size_t)n * G + g] : 0u;
     }
-    v[j] = fmaf(off, sb.x, sb.y);
+    v[j] = ldexpf(fmaf(off, sb.x, sb.y), -e);
   }
   u32x4 hi, lo;
   split8(v, hi, lo);
@@ -258,6 +271,9 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   };
   // the bias term's steps first (their loads go out ahead of the rings')
   const int x0 = nx * kk / KT, x1 = nx * (kk + 1) / KT;
+  float bs[TN];
+#pragma unroll
+  for (int j = 0; j < TN; j++) bs[j] = x0 < x1 ? (a.scale + (size_t)G * a.ldn + n0 + j * 32)[r31] : 1.0f;
   for (int kx = x0; kx < x1; kx++) {
     u32x4 xa[TM][2], xb[TN][2];
 #pragma unroll
@@ -284,6 +300,12 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
           acc[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, xa[i][p == 2]), __builtin_bit_cast(f16x8, xb[j][p == 1]),
                                   acc[i][j], 0, 0, 0);
   }
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] *= bs[j];
   if (x0 == x1 && g0 < g1) {
     load_rings();
   }
@@ -821,7 +843,7 @@ size_t rows_planes_pieces(int M, int K) { return (size_t)((M + 63) / 64 * 2) * (
 size_t rows_q_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * 4 * 128; }
 size_t rows_kv_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * flash_tile_pieces(2); }
 int rows_ldn(int N) { return (N + 63) / 64 * 64; }
-size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64) * rows_ldn(N); }
+size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64 + 1) * rows_ldn(N); }
 size_t rows_codes_bytes(int N, int K, int bits) { return (size_t)rows_ldn(N) * K * bits / 8; }
 size_t rows_bias_pieces(int N, int K) { return (size_t)(rows_ldn(N) / 32) * ((K / 64 + 15) / 16) * 128; }
 

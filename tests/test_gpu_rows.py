@@ -1,5 +1,4 @@
-"""The multi-row forward on operands in fragment order (prompts of more than 48 rows, replay,
-all-row forward): its tiles' edges against the oracle and, for the product alone, against
+"""The multi-row forward on operands in fragment order (prompts, replay, all-row forward): its tiles' edges against the oracle and, for the product alone, against
 float64."""
 import sys
 
@@ -30,7 +29,7 @@ def _model(bits, pd, over=()):
     return _models[key]
 
 
-# 49: the first row count of this path; tiles of 32 and 64 rows and of 32 and 64 keys
+# around tiles of 32 and 64 rows and of 32 and 64 keys
 @pytest.mark.parametrize("T", [48, 49, 63, 64, 65, 96, 97, 129, 320, 321])
 @pytest.mark.parametrize("bits,pd,kv", [(8, H.ITTS_F16, H.ITTS_F32), (8, H.ITTS_F32, H.ITTS_BF16),
                                         (4, H.ITTS_F16, H.ITTS_BF16), (4, H.ITTS_F32, H.ITTS_F32)])
@@ -78,7 +77,20 @@ def test_forward_logits_prompt_boundaries():
     assert r == len(got)
 
 
-# 32 x 64 tiles by four waves; by eight (K >= 4096, few tiles); 64 x 64 (K >= 4096, many tiles)
+def test_long_k_split_over_blocks():
+    """mlp c_proj with K >= 4096 and few tiles: K over several blocks, the counters reused."""
+    over = (("n_layer", 2), ("d_ffn", 4160))
+    W, g, M = _model(8, H.ITTS_F16, over)
+    for n in (2, 40, 120):
+        pr = synth.make_prompt(W.cfg, 3, n, seed=n)
+        cache, okv = g.kv_cache(256, H.ITTS_F32), M.kv(256, kv_bf16=False)
+        b = M.prefill_after(okv, pr.text_tokens, pr.conds, pr.lang_id)
+        for _ in range(2):
+            a = g.prefill(pr.text_tokens, pr.conds, pr.lang_id, cache)
+            assert np.abs(a - b).max() < 2e-5 * max(1.0, np.abs(b).max())
+
+
+# up to 64 rows the 64 x 64 LDS tiles, then 32 x 64 tiles and (K >= 4096, many tiles) 64 x 64
 @pytest.mark.parametrize("bits,pd", [(8, H.ITTS_F16), (4, H.ITTS_F32)])
 @pytest.mark.parametrize("M,N,K", [(49, 37, 192), (65, 130, 64), (100, 1026, 1280), (70, 132, 4160), (2000, 1090, 4096)])
 def test_product_vs_fp64(bits, pd, M, N, K):
@@ -95,3 +107,25 @@ def test_product_vs_fp64(bits, pd, M, N, K):
     # the tiled product's bar: 4e-6 of the sum of magnitudes (22-bit operands, fp32 sums)
     bound = np.abs(x).astype(np.float64) @ np.abs(Wd).T + np.abs(bias)
     assert np.all(np.abs(got - ref) <= 4e-6 * bound + 1e-7)
+
+
+# b + 128 s (b + 8 s) far below fp16's normal range, and past its largest value; groups on one side of zero
+@pytest.mark.parametrize("scale,offset", [(1e-5, 0.0), (1e-5, 90.0), (1e3, 0.0), (1e3, 90.0)])
+@pytest.mark.parametrize("bits", [8, 4])
+def test_product_range_of_f32_params(bits, scale, offset):
+    _, g, _ = _model(8, H.ITTS_F16)
+    M, N, K = 70, 130, 320
+    rng = np.random.default_rng(5)
+    codes, _, _ = H.quantize(rng.standard_normal((N, K)).astype(np.float32), bits, H.ITTS_F32)
+    top = 2.0 ** bits
+    s = (scale * rng.uniform(0.5, 1.5, (N, K // 64))).astype(np.float32)
+    b = (s * (rng.uniform(-0.55, -0.45, s.shape) * top + offset * top / 256)).astype(np.float32)
+    bias = np.zeros(N, np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = g.qlinear_forward(codes, s, b, bias, x, N, K, bits, H.ITTS_F32)
+    Wd = ito.dequant(synth.QLinear(codes, s, b, bias, N, K), bits, H.ITTS_F32).astype(np.float64)
+    ref = x.astype(np.float64) @ Wd.T
+    bound = np.abs(x).astype(np.float64) @ np.abs(Wd).T
+    # 22-bit operands and fp32 sums of the terms' magnitudes (codes and group sums, s times half the
+    # code range an element)
+    assert np.all(np.abs(got - ref) <= 4e-6 * (bound + scale * top / 2 * np.abs(x).sum(1, keepdims=True) / 8))
