@@ -1,4 +1,4 @@
-// Multi-row products and causal attention of the decoder (prefill of long prompts, replay,
+// Multi-row products and causal attention of the decoder (prefill, replay,
 // all-row forward) on operands kept in MFMA fragment order (frag.h).
 //
 // y[M][N] = x[M][K] Wdeq^T + bias contracts fp16 hi/lo activation fragments (~22 bits) with
@@ -800,7 +800,8 @@ hipError_t run(RowsMm a, hipStream_t s) {
 // 32 x 64 tiles by four waves; 64 x 64 where K is long and the tiles many.  M x N x K in us, 32 x
 // 64 / 64 x 64: 35 x 1280 x 1280 7.2 / 10.1, 235 x 5120 x 1280 13.5 / 16.4, 886 x 5120 x 1280 32.7
 // (355 TFLOP/s) / 34.4, 886 x 1280 x 5120 34.5 / 42.3, 2188 x 5120 x 1280 72.5 / 72.4, 2188 x 1280 x
-// 5120 69.7 / 62.5 (459 TFLOP/s, 918 of fp16 products).  (Two groups in flight instead of one
+// 5120 69.7 / 62.5 (459 TFLOP/s, 918 of fp16 products); 64 x 64 at K = 1280 too made prefills of 547
+// and 886 rows 2660 -> 2730 and 3590 -> 3735 us.  (Two groups in flight instead of one
 // gain nothing, eight waves on a tile lose wherever K is not split instead.)
 using RmSmall = RmCfg<1, 4, 1>;
 using RmLarge = RmCfg<2, 4, 1>;

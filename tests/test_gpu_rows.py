@@ -1,5 +1,5 @@
-"""The multi-row forward on operands in fragment order (prompts, replay, all-row forward): its tiles' edges against the oracle and, for the product alone, against
-float64."""
+"""The multi-row forward on operands in fragment order (prompts, replay, all-row forward):
+its tiles' edges against the oracle and, for the product alone, against float64."""
 import sys
 
 import numpy as np
