@@ -50,15 +50,18 @@ constexpr int kFreqDim = 256;
 struct Buf {
   float *p = nullptr;
   size_t n = 0;
+  // the shape whose table or zero rows the buffer holds ((0, 0): none); lost with the memory
+  std::pair<int, int> holds{0, 0};
   Buf() = default;
   Buf(const Buf &) = delete;
   Buf &operator=(const Buf &) = delete;
-  Buf(Buf &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr, o.n = 0; }
+  Buf(Buf &&o) noexcept : p(o.p), n(o.n), holds(o.holds) { o.p = nullptr, o.n = 0, o.holds = {0, 0}; }
   ~Buf() {
     if (p) (void)hipFree(p);
   }
   hipError_t ensure(size_t count) {
     if (count <= n) return hipSuccess;
+    holds = {0, 0};
     if (p) {
       hipError_t e = hipFree(p);
       p = nullptr;
@@ -97,9 +100,7 @@ struct itts_cfm {
   // long skip joins, the skips, merged and x_t inputs, x_res, WaveNet's padded input, Q, K / V
   Buf nP, attP, actP, curP, mP, xtP, xresP, hpP, qF, kvF;
   std::vector<Buf> skipP, skips;
-  int rope_T = 0;           // sequence length the rope table holds
-  int hp_B = 0, hp_T = 0;   // shape whose padding rows hpP holds as zeros
-  int n_cu = 0;             // compute units of the device (the launch rules' parameter)
+  int n_cu = 0;  // compute units of the device (the launch rules' parameter)
   // solve / API staging
   Buf x, xt, merged, catc, refm, sty, io_a, io_b;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -204,10 +205,10 @@ itts_status ensure_rows(itts_cfm *m, int B, int T) {
   CK(m->kvF.ensure(piece_floats(cfm_kv_pieces(B, T, c.n_heads))));
   const size_t hp = hp_pieces(c, T);
   CK(m->hpP.ensure(piece_floats(B * hp)));
-  if (m->hp_B != B || m->hp_T != T) {  // the convolution's padding rows, zero from here on
+  if (m->hpP.holds != std::make_pair(B, T)) {  // the convolution's padding rows, zero from here on
+    m->hpP.holds = {0, 0};
     CK(hipMemsetAsync(m->hpP.p, 0, sizeof(uint4) * B * hp, m->s));
-    m->hp_B = B;
-    m->hp_T = T;
+    m->hpP.holds = {B, T};
   }
   const bool few = R < kMfmaRows;
   if (few || unaligned_skip(c)) {
@@ -231,10 +232,11 @@ itts_status ensure_rows(itts_cfm *m, int B, int T) {
     CK(m->mP.ensure(piece_floats(cfm_frag_pieces(R, steps16(2 * c.in_ch + c.dim + c.style_dim)))));
     CK(m->xtP.ensure(piece_floats(cfm_frag_pieces(R, steps16(c.in_ch)))));
   }
-  if (m->rope_T != T) {
-    CK(m->rope.ensure((size_t)T * 64));
+  CK(m->rope.ensure((size_t)T * 64));
+  if (m->rope.holds != std::make_pair(1, T)) {
+    m->rope.holds = {0, 0};
     CK(cfm_rope_table(T, m->rope.p, m->s));
-    m->rope_T = T;
+    m->rope.holds = {1, T};
   }
   return ITTS_OK;
 }
