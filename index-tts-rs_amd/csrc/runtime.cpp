@@ -73,6 +73,11 @@ struct DevBuf {
     if (e == hipSuccess) bytes = n;
     return e;
   }
+  void drop() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  }
   template <class T>
   T *as() const {
     return static_cast<T *>(p);
@@ -338,7 +343,9 @@ hipError_t ensure_planes(itts_gpt *g, DevBuf &buf, int M, int K) {
   const size_t bytes = sizeof(uint4) * rows_planes_pieces(M, K);
   if (bytes <= buf.bytes) return hipSuccess;
   hipError_t e = buf.ensure(bytes);
-  if (e == hipSuccess) e = hipMemsetAsync(buf.p, 0, buf.bytes, g->stream);
+  if (e != hipSuccess) return e;
+  e = hipMemsetAsync(buf.p, 0, buf.bytes, g->stream);
+  if (e != hipSuccess) buf.drop();  // (its size says that it was cleared)
   return e;
 }
 

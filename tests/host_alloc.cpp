@@ -100,3 +100,26 @@ int main() {
   return 0;
 }
 #endif
+
+#ifdef RUNTIME
+namespace itts {
+size_t rows_planes_pieces(int M, int K) { return (size_t)M * K / 4; }
+}  // namespace itts
+
+int main() {
+  itts_gpt g;
+  for (int *f : {&fail_malloc, &fail_memset}) {
+    DevBuf b;
+    EXPECT(ensure_planes(&g, b, 32, 64) == hipSuccess && zero(b.p, b.bytes), "first planes");
+    *f = 1;
+    EXPECT(ensure_planes(&g, b, 96, 64) != hipSuccess, "a failure goes unnoticed");
+    *f = 0;
+    for (int M : {32, 96}) {
+      EXPECT(ensure_planes(&g, b, M, 64) == hipSuccess, "the next call fails");
+      EXPECT(b.bytes >= sizeof(uint4) * rows_planes_pieces(M, 64) && zero(b.p, b.bytes), "planes not zero at %d rows", M);
+    }
+  }
+  puts("ok");
+  return 0;
+}
+#endif

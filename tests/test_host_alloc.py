@@ -12,9 +12,9 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is needed to compile the library's host code")
-@pytest.mark.parametrize("part", ["CFM"])
+@pytest.mark.parametrize("part", ["CFM", "RUNTIME"])
 def test_failed_allocation_leaves_nothing_stale(tmp_path, part):
-    src = os.path.join(ROOT, "index-tts-rs_amd", "csrc", {"CFM": "cfm.cpp"}[part])
+    src = os.path.join(ROOT, "index-tts-rs_amd", "csrc", {"CFM": "cfm.cpp", "RUNTIME": "runtime.cpp"}[part])
     exe = str(tmp_path / part)
     # (the kernels' launchers stay undefined: nothing here reaches them)
     subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", f'-DSOURCE="{src}"',
