@@ -1,11 +1,14 @@
-// Operands of v_mfma_f32_32x32x16_f16 kept in memory in fragment order, and the attention
-// loop that runs on them (gfx950, wave64).
+// Operands of v_mfma_f32_32x32x16_{f16, bf16} kept in memory in fragment order, and the
+// attention loop that runs on them (gfx950, wave64).
 //
-// A matrix X [rows][K] that a product reads as an MFMA operand is stored as fp16 hi/lo
-// planes in blocks of 32 rows x 16 K: lane l of the operand holds row (l & 31), K values
+// A matrix X [rows][K] that a product reads as an MFMA operand is stored as planes of 16-bit
+// values in blocks of 32 rows x 16 K: lane l of the operand holds row (l & 31), K values
 // 8 (l >> 5) .. +7, so a block's plane is 64 pieces of 16 bytes in lane order (1 KiB) and
 // an operand load is one fully coalesced 16-byte load per lane straight into registers: no
 // LDS staging, no barrier, and any number of K steps in flight.
+//
+// Planes: fp16 hi/lo pairs (~22 bits, magnitudes below 131008, an absolute 2^-25 at the small
+// end), or bf16 triples, which hold an fp32 value's 24 bits over its whole range.
 #pragma once
 
 #include "common.h"
@@ -13,12 +16,15 @@
 namespace itts {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 #define ITTS_MFMA16 __builtin_amdgcn_mfma_f32_32x32x16_f16
+#define ITTS_MFMABF __builtin_amdgcn_mfma_f32_32x32x16_bf16
 
 // 16-byte piece of (row, 8-value chunk k8 of K), hi plane; the lo plane's is 64 pieces on.
 // nk: K steps of 16 that a row block holds.
@@ -36,6 +42,46 @@ __device__ __forceinline__ void split8(const float v[8], u32x4 &hi, u32x4 &lo) {
   }
 }
 
+// v = p[0] + p[1] + p[2] (each plane the rounding of what the planes before it leave).  An
+// infinity or NaN stays one in plane 0.
+__device__ __forceinline__ void split8_bf16(const float v[8], u32x4 (&p)[3]) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    f32x2e a = {v[2 * j], v[2 * j + 1]};
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const bf16x2v h = __builtin_convertvector(a, bf16x2v);
+      p[i][j] = __builtin_bit_cast(uint32_t, h);
+      a -= __builtin_convertvector(h, f32x2e);
+    }
+  }
+}
+
+// The two operand forms: planes of an activation operand, its split, one MFMA of two planes.
+struct F16Pairs {
+  typedef f16x8 V;
+  static constexpr int N = 2;
+  static __device__ __forceinline__ floatx16 mma(V a, V b, floatx16 c) { return ITTS_MFMA16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ void split(const float v[8], u32x4 (&p)[N]) { split8(v, p[0], p[1]); }
+};
+struct Bf16Triples {
+  typedef bf16x8 V;
+  static constexpr int N = 3;
+  static __device__ __forceinline__ floatx16 mma(V a, V b, floatx16 c) { return ITTS_MFMABF(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ void split(const float v[8], u32x4 (&p)[N]) { split8_bf16(v, p); }
+};
+// c + a b over operands of NA and T::N planes: the products of planes whose orders add up to
+// less than T::N (the others lie below the last plane's rounding).
+template <class T, int NA>
+__device__ __forceinline__ floatx16 mma_planes(const u32x4 (&a)[NA], const u32x4 (&b)[T::N], floatx16 c) {
+#pragma unroll
+  for (int i = 0; i < NA; i++)
+#pragma unroll
+    for (int j = 0; j < T::N - i; j++)
+      c = T::mma(__builtin_bit_cast(typename T::V, a[i]), __builtin_bit_cast(typename T::V, b[j]), c);
+  return c;
+}
+
 // Exchanges v with lane ^ 32 (one VALU swap, no LDS round trip).
 __device__ __forceinline__ float other_half(float v, int lane) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -50,9 +96,9 @@ __device__ __forceinline__ float other_half(float v, int lane) {
 // order: position 8 h + 4 j2 + b of a 16-key step is key 8 j2 + 4 h + b.
 //
 // A key tile holds 8 fragments (4 K steps of K rows over the 64 dims; 2 dim tiles x 2 key
-// steps of V^T) of NP planes each: kFlashFrags * NP KiB, contiguous.  NP = 1 where the lo
-// planes are all zero (bf16 rows: eight significant bits fit fp16 exactly, and below fp16's
-// normal range both forms stop at the same 2^-25).
+// steps of V^T) of NP planes each: kFlashFrags * NP KiB, contiguous.  Pairs have two planes;
+// triples three, or one where the rows are bf16 (the plane is the value itself, whatever its
+// magnitude, infinities and NaN with it).
 constexpr int kFlashFrags = 8;
 __host__ __device__ inline size_t flash_tile_pieces(int np) { return (size_t)kFlashFrags * np * 64; }
 // position of key t (mod 16) within V^T's 16-key step
@@ -77,10 +123,11 @@ __device__ __forceinline__ void flash_init(FlashState &st) {
 // that a score's exponential is 2^s.  mask(tile, S) sets scores of masked keys to -inf.  The
 // exponent reference m is raised only when some score passes it by more than 2^8: until then
 // probabilities up to 2^8 are carried, in the same relative precision, and the rescaling of
-// O is skipped.
-template <int NP, class Mask>
-__device__ __forceinline__ void flash_tiles(const u32x4 *kv, int t0, int t1, const f16x8 (&qh)[4],
-                                            const f16x8 (&ql)[4], Mask mask, FlashState &st) {
+// O is skipped.  (A masked key's V row still meets a probability of zero: if it is not finite,
+// the rows that share its tile become NaN too.)
+template <class T, int NP, class Mask>
+__device__ __forceinline__ void flash_tiles(const u32x4 *kv, int t0, int t1, const u32x4 (&q)[4][T::N], Mask mask,
+                                            FlashState &st) {
   if (t0 >= t1) return;
   u32x4 kf[4][NP], vf[4][NP];
   auto load_k = [&](int t) __attribute__((always_inline)) {
@@ -104,12 +151,7 @@ __device__ __forceinline__ void flash_tiles(const u32x4 *kv, int t0, int t1, con
 #pragma unroll
     for (int i = 0; i < 16; i++) S[i] = 0.0f;
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      const f16x8 kh = __builtin_bit_cast(f16x8, kf[kk][0]);
-      S = ITTS_MFMA16(kh, qh[kk], S, 0, 0, 0);
-      S = ITTS_MFMA16(kh, ql[kk], S, 0, 0, 0);
-      if constexpr (NP == 2) S = ITTS_MFMA16(__builtin_bit_cast(f16x8, kf[kk][1]), qh[kk], S, 0, 0, 0);
-    }
+    for (int kk = 0; kk < 4; kk++) S = mma_planes<T, NP>(kf[kk], q[kk], S);
     // the next tile's K into the registers just read (the last tile's again at the end)
     load_k(min(t + 1, t1 - 1));
     mask(t, S);
@@ -137,17 +179,10 @@ __device__ __forceinline__ void flash_tiles(const u32x4 *kv, int t0, int t1, con
     st.l += sum;
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
-      u32x4 h, l;
-      split8(p + 8 * kk, h, l);
-      const f16x8 ph = __builtin_bit_cast(f16x8, h), pl = __builtin_bit_cast(f16x8, l);
+      u32x4 pp[T::N];
+      T::split(p + 8 * kk, pp);
 #pragma unroll
-      for (int dt = 0; dt < 2; dt++) {
-        const f16x8 vh = __builtin_bit_cast(f16x8, vf[dt * 2 + kk][0]);
-        st.O[dt] = ITTS_MFMA16(vh, ph, st.O[dt], 0, 0, 0);
-        st.O[dt] = ITTS_MFMA16(vh, pl, st.O[dt], 0, 0, 0);
-        if constexpr (NP == 2)
-          st.O[dt] = ITTS_MFMA16(__builtin_bit_cast(f16x8, vf[dt * 2 + kk][1]), ph, st.O[dt], 0, 0, 0);
-      }
+      for (int dt = 0; dt < 2; dt++) st.O[dt] = mma_planes<T, NP>(vf[dt * 2 + kk], pp, st.O[dt]);
     }
     load_v(min(t + 1, t1 - 1));
   }

@@ -158,6 +158,10 @@ size_t gemm_ws_floats(int n_cu);
 constexpr int kGemmCounters = 4096;
 
 // ---- multi-row forwards on operands in fragment order (kernels_rows.hip) ----
+// kvt of rows_mm and rows_attn, beside KvType: fp32 rows whose attention operands are fp16 pairs
+// (magnitudes below 131008, 22 bits, an absolute 2^-25 at the small end; kKvF32 holds all of them
+// as they are).
+constexpr int kRowsPairs = 2;
 // Activation planes of M rows of K values (16-byte pieces; the group sums' last step must be
 // zero-filled once), the attention's Q and K / V fragments, and a weight's codes in fragment
 // order, scale table and bias planes (made once by rows_params).

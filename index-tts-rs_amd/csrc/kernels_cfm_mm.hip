@@ -558,12 +558,12 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(const u32x4 *qf, const u32
   const int bh = blockIdx.x, b = bh / H, head = bh % H;
   const int Tt = (T + 63) / 64 * 2, nt = (T + 31) / 32;
   const int qt = blockIdx.y * WQ + wq;
-  f16x8 qh[4], ql[4];
+  u32x4 q[4][2];
   const u32x4 *qp = qf + (((size_t)bh * Tt + min(qt, Tt - 1)) * 4) * 128 + lane;
 #pragma unroll
   for (int kk = 0; kk < 4; kk++) {
-    qh[kk] = __builtin_bit_cast(f16x8, qp[kk * 128]);
-    ql[kk] = __builtin_bit_cast(f16x8, qp[kk * 128 + 64]);
+    q[kk][0] = qp[kk * 128];
+    q[kk][1] = qp[kk * 128 + 64];
   }
   FlashState st;
   flash_init(st);
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(const u32x4 *qf, const u32
         if (t * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3) >= T) S[i] = -INFINITY;
     }
   };
-  flash_tiles<2>(kvf + (size_t)bh * Tt * flash_tile_pieces(2) + lane, t0, t1, qh, ql, mask, st);
+  flash_tiles<F16Pairs, 2>(kvf + (size_t)bh * Tt * flash_tile_pieces(2) + lane, t0, t1, q, mask, st);
   flash_merge<WK>(st, buf + wq * WK * 2112, g, lane);
   const int t = qt * 32 + (lane & 31);
   if (g != 0 || t >= T) return;

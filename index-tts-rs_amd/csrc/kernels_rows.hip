@@ -197,6 +197,20 @@ __device__ __forceinline__ f16x8 codes_f16(uint32_t w0, uint32_t w1) {
   return __builtin_bit_cast(f16x8, r);
 }
 
+// The attention's operands by the rows' type: q and the probabilities in T's planes, K and V in
+// NP.  bf16 rows are their own single plane, so nothing of q, K, V or the probabilities is
+// rounded and no magnitude is out of range; fp32 rows the same in three planes, or as pairs.
+template <int KVT>
+struct AttnPlanes {
+  typedef Bf16Triples T;
+  static constexpr int NP = KVT == kKvBf16 ? 1 : 3;
+};
+template <>
+struct AttnPlanes<kRowsPairs> {
+  typedef F16Pairs T;
+  static constexpr int NP = 2;
+};
+
 template <int BITS, int EPI, int KVT, class C>
 __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(RowsMm a) {
   constexpr int TM = C::TM, TN = C::TN, KS = C::KS, KL = C::KL, BM = C::BM, BN = C::BN, LD = C::LD, NT = C::NT;
@@ -616,7 +630,8 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   } else {
     // the 64 columns are one head of q, k or v: the attention's fragments (q scaled by
     // log2(e) / 8; rows past M, up to whole tiles of 64 keys, zero), and the cache rows
-    constexpr int NP = KVT == kKvBf16 ? 1 : 2;
+    using P = AttnPlanes<KVT>;
+    constexpr int NQ = P::T::N, NP = P::NP;
     const int d = a.N / 3, which = n0 / d, head = (n0 - which * d) / 64, Tt = (a.M + 63) / 64 * 2;
     auto round_kv = [&](float v[8]) __attribute__((always_inline)) {
       if constexpr (KVT == kKvBf16) {
@@ -638,12 +653,12 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) v[e] = t < a.M ? v[e] * (0.125f * 1.4426950408889634f) : 0.0f;
-        u32x4 hi, lo;
-        split8(v, hi, lo);
-        u32x4 *dst = reinterpret_cast<u32x4 *>(a.qf) + (((size_t)head * Tt + (t >> 5)) * 4 + (c >> 1)) * 128 +
+        u32x4 p[NQ];
+        P::T::split(v, p);
+        u32x4 *dst = reinterpret_cast<u32x4 *>(a.qf) + (((size_t)head * Tt + (t >> 5)) * 4 + (c >> 1)) * (NQ * 64) +
                      (c & 1) * 32 + (t & 31);
-        dst[0] = hi;
-        dst[64] = lo;
+#pragma unroll
+        for (int i = 0; i < NQ; i++) dst[i * 64] = p[i];
         continue;
       }
       round_kv(v);
@@ -665,11 +680,11 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       if (which == 1 && t < Tt * 32) {
 #pragma unroll
         for (int e = 0; e < 8; e++) v[e] = t < a.M ? v[e] : 0.0f;
-        u32x4 hi, lo;
-        split8(v, hi, lo);
+        u32x4 p[NQ];
+        P::T::split(v, p);
         u32x4 *dst = kvf + (size_t)(t >> 5) * flash_tile_pieces(NP) + (c >> 1) * NP * 64 + (c & 1) * 32 + (t & 31);
-        dst[0] = hi;
-        if constexpr (NP == 2) dst[64] = lo;
+#pragma unroll
+        for (int i = 0; i < NP; i++) dst[i * 64] = p[i];
       }
     }
     if (which == 2) {
@@ -692,12 +707,12 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
         round_kv(v);
 #pragma unroll
         for (int j = 0; j < 8; j++) v[j] = m0 + rb + (j >> 2) * 8 + (j & 3) < a.M ? v[j] : 0.0f;
-        u32x4 hi, lo;
-        split8(v, hi, lo);
+        u32x4 p[NQ];
+        P::T::split(v, p);
         u32x4 *dst = kvf + (size_t)(t >> 5) * flash_tile_pieces(NP) +
                      (4 + (e >> 5) * 2 + ((t >> 4) & 1)) * NP * 64 + (k8 & 1) * 32 + (e & 31);
-        dst[0] = hi;
-        if constexpr (NP == 2) dst[64] = lo;
+#pragma unroll
+        for (int i = 0; i < NP; i++) dst[i * 64] = p[i];
       }
     }
   }
@@ -706,7 +721,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
 // ---- causal attention -------------------------------------------------------------------
 // Block: 32 query rows of one head, its four waves on a quarter of the key tiles each.  Row t
 // attends to keys kstart[t] (or 0) .. t; order lists the query tiles, most keys first.
-template <int NP>
+template <int KVT>
 __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, const u32x4 *kvf, int M, const int *kstart,
                                                            const int *order, u32x4 *out) {
   __shared__ float buf[4 * 2112];
@@ -715,13 +730,14 @@ __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, cons
   const int qt = order ? order[blockIdx.y] : (int)(gridDim.y - 1 - blockIdx.y);
   const int t = qt * 32 + (lane & 31), tc = min(t, M - 1);
   const int ks = kstart ? kstart[tc] : 0;
-  f16x8 qh[4], ql[4];
-  const u32x4 *qp = qf + (((size_t)head * Tt + qt) * 4) * 128 + lane;
+  using P = AttnPlanes<KVT>;
+  constexpr int NQ = P::T::N, NP = P::NP;
+  u32x4 q[4][NQ];
+  const u32x4 *qp = qf + (((size_t)head * Tt + qt) * 4) * (NQ * 64) + lane;
 #pragma unroll
-  for (int kk = 0; kk < 4; kk++) {
-    qh[kk] = __builtin_bit_cast(f16x8, qp[kk * 128]);
-    ql[kk] = __builtin_bit_cast(f16x8, qp[kk * 128 + 64]);
-  }
+  for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+    for (int i = 0; i < NQ; i++) q[kk][i] = qp[(kk * NQ + i) * 64];
   FlashState st;
   flash_init(st);
   const int tb = kstart ? kstart[qt * 32] / 32 : 0, nt = qt + 1 - tb;
@@ -736,7 +752,7 @@ __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, cons
       }
     }
   };
-  flash_tiles<NP>(kvf + (size_t)head * Tt * flash_tile_pieces(NP) + lane, t0, t1, qh, ql, mask, st);
+  flash_tiles<typename P::T, NP>(kvf + (size_t)head * Tt * flash_tile_pieces(NP) + lane, t0, t1, q, mask, st);
   flash_merge<4>(st, buf, g, lane);
   if (g != 0) return;
   const float inv = 1.0f / st.l;
@@ -833,7 +849,8 @@ hipError_t dispatch(const RowsMm &a, int epi, int kvt, hipStream_t s) {
     case kEpiGelu: return a.N % 64 == 0 && a.o ? pick<BITS, kEpiGelu, 0>(a, s) : hipErrorInvalidValue;
     case kEpiQKV:
       if (a.N % 192 != 0 || !a.qf || !a.kvf) return hipErrorInvalidValue;
-      return kvt == kKvBf16 ? pick<BITS, kEpiQKV, kKvBf16>(a, s) : pick<BITS, kEpiQKV, kKvF32>(a, s);
+      if (kvt == kKvBf16) return pick<BITS, kEpiQKV, kKvBf16>(a, s);
+      return kvt == kKvF32 ? pick<BITS, kEpiQKV, kKvF32>(a, s) : pick<BITS, kEpiQKV, kRowsPairs>(a, s);
   }
   return hipErrorInvalidValue;
 }
@@ -841,8 +858,8 @@ hipError_t dispatch(const RowsMm &a, int epi, int kvt, hipStream_t s) {
 }  // namespace
 
 size_t rows_planes_pieces(int M, int K) { return (size_t)((M + 63) / 64 * 2) * (K / 16 + (K / 64 + 15) / 16) * 128; }
-size_t rows_q_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * 4 * 128; }
-size_t rows_kv_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * flash_tile_pieces(2); }
+size_t rows_q_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * 4 * 192; }
+size_t rows_kv_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * flash_tile_pieces(3); }
 int rows_ldn(int N) { return (N + 63) / 64 * 64; }
 size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64 + 1) * rows_ldn(N); }
 size_t rows_codes_bytes(int N, int K, int bits) { return (size_t)rows_ldn(N) * K * bits / 8; }
@@ -886,10 +903,8 @@ hipError_t rows_attn(const uint4 *qf, const uint4 *kvf, int M, int H, const int 
   if (M < 1 || H < 1) return hipErrorInvalidValue;
   const dim3 grid(H, (M + 31) / 32);
   const u32x4 *q = reinterpret_cast<const u32x4 *>(qf), *kv = reinterpret_cast<const u32x4 *>(kvf);
-  if (kvt == kKvBf16)
-    hipLaunchKernelGGL(rows_attn_kernel<1>, grid, dim3(256), 0, s, q, kv, M, kstart, order, reinterpret_cast<u32x4 *>(out));
-  else
-    hipLaunchKernelGGL(rows_attn_kernel<2>, grid, dim3(256), 0, s, q, kv, M, kstart, order, reinterpret_cast<u32x4 *>(out));
+  auto *fn = kvt == kKvBf16 ? rows_attn_kernel<kKvBf16> : kvt == kKvF32 ? rows_attn_kernel<kKvF32> : rows_attn_kernel<kRowsPairs>;
+  hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, q, kv, M, kstart, order, reinterpret_cast<u32x4 *>(out));
   return hipGetLastError();
 }
 

@@ -459,6 +459,11 @@ struct ProbeSpec {
   float *out;
 };
 
+// Up to this many rows a prompt's attention over an fp32 cache holds q, K, V and the probabilities
+// in all their bits (six products a tile); longer ones, and replays, as fp16 pairs (three).  Six
+// throughout: 235 rows 1645 -> 1685 us, 886 rows 3600 -> 3785, replay of 1400 codes 6360 -> 6830.
+constexpr int kExactAttnRows = 384;
+
 // Runs n_layers blocks over the M rows in gpt->px on operands in fragment order.  Row
 // r attends to keys kstart[r] (or 0) .. r; K/V rows go to kv's cache (prefill) or, for the
 // layers that are probed, to the fp32 scratch rk / rv.  ln_1 (after layer 0) and ln_2 are
@@ -467,7 +472,8 @@ struct ProbeSpec {
 itts_status rows_stack(itts_gpt *g, itts_kv *kv, int M, int n_layers, const int *kstart, const int *order,
                        const std::vector<ProbeSpec> &probes) {
   const itts_config &c = g->cfg;
-  const int d = c.d_model, F = c.d_ffn, bits = c.quant_bits, kvt = kv ? kv->kvt : kKvF32;
+  const int d = c.d_model, F = c.d_ffn, bits = c.quant_bits;
+  const int kvt = kv && (kv->kvt == kKvBf16 || M <= kExactAttnRows) ? kv->kvt : kRowsPairs;
   hipStream_t s = g->stream;
   float *X = g->px.as<float>();
   const bool folded = g->fold.p != nullptr && d <= 32 * kGroup;  // (a row's group statistics in registers)

@@ -62,6 +62,51 @@ def test_wide_model_without_folds():
     assert np.abs(a - b).max() < 2e-5 * max(1.0, np.abs(b).max())
 
 
+def _one_block(**over):
+    return dict(synth.TINY_CONFIG, n_layer=1, param_dtype=H.ITTS_F32, mel_pos_len=600, **over)
+
+
+@pytest.mark.parametrize("kv", [H.ITTS_BF16, H.ITTS_F32])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_nonfinite_conditioning_reaches_the_logits(kv, bad):
+    """A row that is not finite makes its K and V NaN, and with them every later row's attention;
+    one block of two heads, so that nothing else can carry it there."""
+    say(f"[gpu] prefill with a {bad} conditioning row, kv {kv}")
+    for seed in range(8):
+        W = synth.make_weights(_one_block(), seed=seed, init="rich")
+        g = H.Gpt(W)
+        for T in (24, 100, 450):
+            pr = synth.make_prompt(W.cfg, 3, 15, seed=seed)
+            pr.conds[1, 7] = bad
+            cache = g.kv_cache(512, kv)
+            prior = (np.arange(T - 21, dtype=np.int32) * 13) % (W.cfg["mel_vocab"] - 2)
+            assert np.isnan(g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, prior, cache)).all(), (seed, T)
+            assert np.isnan(g.step(cache, 5, T - 19)).all(), (seed, T)
+        g.close()
+
+
+@pytest.mark.parametrize("kv,T", [(H.ITTS_BF16, 40), (H.ITTS_BF16, 300), (H.ITTS_BF16, 500), (H.ITTS_F32, 40), (H.ITTS_F32, 384)])
+@pytest.mark.parametrize("e", [14, 20])
+def test_attention_of_scaled_q_and_k(kv, T, e):
+    """q times 2^-e and K times 2^e are the same attention, to the bit: all of it is fp32 (or bf16
+    rows) over its whole range."""
+    say(f"[gpu] prefill T={T} kv {kv}, q and K scaled by 2^{e}")
+    W = synth.make_weights(_one_block(), seed=3, init="rich")
+    d = W.cfg["d_model"]
+    got = []
+    for scale in (1.0, 2.0**e):
+        for L in W.layers:
+            for a in (L.c_attn.scales, L.c_attn.biases, L.c_attn.bias):
+                a[:d] *= np.float32(1.0 / scale)
+                a[d:2 * d] *= np.float32(scale)
+        g = H.Gpt(W)
+        pr = synth.make_prompt(W.cfg, 3, 15, seed=1)
+        prior = (np.arange(T - 21, dtype=np.int32) * 13) % (W.cfg["mel_vocab"] - 2)
+        got.append(g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, prior, g.kv_cache(512, kv)))
+        g.close()
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]), float(np.abs(got[0] - got[1]).max())
+
+
 def test_forward_logits_prompt_boundaries():
     """Prompts that start and end inside query and key tiles, one shorter than a tile."""
     W, g, M = _model(8, H.ITTS_F16)
