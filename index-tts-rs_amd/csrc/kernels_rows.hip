@@ -5,15 +5,15 @@
 // the codes, exact in fp16 as q - 128 (8-bit) or q - 8 (4-bit), two products on
 // v_mfma_f32_32x32x16_f16 per K step, and folds each 64-group's scale into an fp32
 // accumulator: acc += s[g, n] P.  The groups' bias term, sum_g b'[n, g] sum_{k in g} x[m, k]
-// with b' = b + 128 s (or 8 s), is itself a product over G more K values: the activation
-// planes carry an eighth of the groups' sums as further K steps (the sums of 64 values up to 16376
-// fit fp16's hi/lo range; what an eighth rounds of tiny activations is no more than the activations'
-// own rounding), the weights' b' planes hold the other operand (both hi/lo, three products).  b' is scaled by a power of two a column, its largest in [2^13, 2^14): unscaled, b'
-// of 1e-4 keeps 12 bits of fp32 parameters (replay, error against 64 bits 5e-7 instead of 6e-8).
+// with b' = b + 128 s (or 8 s), is itself a product over G more K values, of bf16 triples: the
+// activation planes carry the groups' sums as further K steps, the weights' b' planes hold the
+// other operand.  Triples keep both as the fp32 values they are, over fp32's range: as fp16
+// pairs, sums past 8188 an element lost bits and sums past 16376 overflowed.
 //
-// Activation planes ("rows"): per 32-row block, K / 16 steps, then ceil(G / 16) steps of group
-// sums.  Inside a 64-group the K order is permuted so that a lane's codes of two steps are one
-// contiguous read: chunk c8 (8 values) is half (c8 >> 1) & 1 of step 2 (c8 >> 2) + (c8 & 1).
+// Activation planes ("rows"): per 32-row block, K / 16 steps of fp16 pairs, then ceil(G / 16)
+// steps of group sums.  Inside a 64-group the K order is permuted so that a lane's codes of two
+// steps are one contiguous read: chunk c8 (8 values) is half (c8 >> 1) & 1 of step 2 (c8 >> 2) +
+// (c8 & 1).
 // The codes are held a second time in that order (per 32 columns and group, two 32-value
 // halves of 64 lanes x 16 codes): a fragment load is then one coalesced run, where the
 // row-major codes touch 32 rows (886 x 5120 x 1280: 32.7 against 46.7 us).
@@ -28,20 +28,27 @@ namespace {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-// piece of (row, chunk c of K): hi plane; lo 64 pieces on.  ns: steps a row block holds.
-__device__ __forceinline__ size_t rows_piece(int row, int c, int ns) {
+// pieces of a row block: nk steps of K, nx of group sums
+__host__ __device__ inline size_t rows_block(int nk, int nx) { return (size_t)nk * 128 + (size_t)nx * 192; }
+__device__ __forceinline__ size_t rows_block_of(int d) { return rows_block(d / 16, (d / 64 + 15) / 16); }
+// piece of (row, chunk c of K): hi plane; lo 64 pieces on.  rb: rows_block of the planes.
+__device__ __forceinline__ size_t rows_piece(int row, int c, size_t rb) {
   const int step = (c >> 3) * 4 + ((c >> 2) & 1) * 2 + (c & 1);
-  return (((size_t)(row >> 5) * ns + step) * 2) * 64 + (size_t)(((c >> 1) & 1) * 32 + (row & 31));
+  return (row >> 5) * rb + (size_t)(step * 128 + ((c >> 1) & 1) * 32 + (row & 31));
 }
-// an eighth of group g's sum v: element of the extra steps
-__device__ __forceinline__ void put_group_sum(u32x4 *o, int row, int g, int nk, int ns, float v) {
-  uint32_t h, l;
-  split_f16(v * 0.125f, h, l);
-  uint16_t *p = reinterpret_cast<uint16_t *>(o + (((size_t)(row >> 5) * ns + nk + (g >> 4)) * 2) * 64 +
-                                             (size_t)(((g >> 3) & 1) * 32 + (row & 31))) +
-                (g & 7);
-  p[0] = (uint16_t)h;
-  p[64 * 8] = (uint16_t)l;
+// piece of (row, chunk g8 of groups) of rb pieces a block whose group steps start at piece at; plane 0 of three
+__device__ __forceinline__ size_t group_piece(int row, int g8, size_t rb, int at) {
+  return (row >> 5) * rb + (size_t)(at + (g8 >> 1) * 192 + (g8 & 1) * 32 + (row & 31));
+}
+// group g's sum v: element of the group steps
+__device__ __forceinline__ void put_group_sum(u32x4 *o, int row, int g, int nk, size_t rb, float v) {
+  __bf16 *p = reinterpret_cast<__bf16 *>(o + group_piece(row, g >> 3, rb, nk * 128)) + (g & 7);
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    const __bf16 h = (__bf16)v;
+    p[i * 64 * 8] = h;
+    v -= (float)h;
+  }
 }
 
 __device__ __forceinline__ float sum8(float v) {  // over eight consecutive lanes
@@ -53,7 +60,8 @@ __device__ __forceinline__ float sum8(float v) {  // over eight consecutive lane
 // LayerNorm of rows (a second one with w2; none without w) as planes and group sums; one wave a row.
 __global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const float *w, const float *b, const float *w2,
                                                        const float *b2, int d, u32x4 *out) {
-  const int row = blockIdx.x, lane = threadIdx.x, nc = d / 8, nk = d / 16, ns = nk + (d / 64 + 15) / 16;
+  const int row = blockIdx.x, lane = threadIdx.x, nc = d / 8, nk = d / 16;
+  const size_t rb = rows_block_of(d);
   const float *xr = x + (size_t)row * d;
   // mean and 1 / std over f(element) (the row is read again for each pass, from the caches)
   auto stats = [&](auto f, float &mean, float &rstd) __attribute__((always_inline)) {
@@ -85,17 +93,16 @@ __global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const flo
     if (c >= nc) continue;
     u32x4 hi, lo;
     split8(v, hi, lo);
-    const size_t p = rows_piece(row, c, ns);
+    const size_t p = rows_piece(row, c, rb);
     out[p] = hi;
     out[p + 64] = lo;
-    if ((c & 7) == 0) put_group_sum(out, row, c >> 3, nk, ns, g);
+    if ((c & 7) == 0) put_group_sum(out, row, c >> 3, nk, rb, g);
   }
 }
 
 // ---- weights ----------------------------------------------------------------------------
 // scale [G][ldn] fp32 and the (scale, bias) words transposed alike (columns past N zero), and b' =
-// b + off s as fragment planes of G values, times 2^-e a column; row G of scale holds 8 2^e (8: the
-// planes meet eighths of sums)
+// b + off s as the group steps' planes
 template <int PT>
 __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, int N, int G, int ldn, float off,
                                                           float *scale, u32x4 *bw, void *words) {
@@ -103,17 +110,7 @@ __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, in
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)ldn * nx * 2) return;
   const int n = (int)(i % ldn), g8 = (int)(i / ldn);
-  float v[8], top = 0.0f;
-  for (int g = 0; g < G && n < N; g++) {
-    const float2 sb = load_param<PT>(params, (size_t)n * G + g);
-    top = fmaxf(top, fabsf(fmaf(off, sb.x, sb.y)));
-  }
-  int e = 0;
-  if (top > 0.0f && top < INFINITY) {
-    frexpf(top, &e);  // top in [2^(e-1), 2^e)
-    e = max(e - 14, -120);
-  }
-  if (g8 == 0) scale[(size_t)G * ldn + n] = ldexpf(8.0f, e);
+  float v[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const int g = g8 * 8 + j;
@@ -125,13 +122,13 @@ __global__ __launch_bounds__(256) void rows_params_kernel(const void *params, in
       if constexpr (PT == kParamF32) static_cast<float2 *>(words)[i] = sb;
       else static_cast<uint32_t *>(words)[i] = n < N ? static_cast<const uint32_t *>(params)[(size_t)n * G + g] : 0u;
     }
-    v[j] = ldexpf(fmaf(off, sb.x, sb.y), -e);
+    v[j] = fmaf(off, sb.x, sb.y);
   }
-  u32x4 hi, lo;
-  split8(v, hi, lo);
-  const size_t p = frag_piece(n, g8, nx);
-  bw[p] = hi;
-  bw[p + 64] = lo;
+  u32x4 pl[3];
+  split8_bf16(v, pl);
+  const size_t p = group_piece(n, g8, rows_block(0, nx), 0);
+#pragma unroll
+  for (int k = 0; k < 3; k++) bw[p + k * 64] = pl[k];
 }
 
 // codes in fragment order: lane's 16 codes (BITS * 2 bytes) of (32 columns, group, half), zero past N
@@ -225,12 +222,12 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   const int tm = jb / pn * a.gm + x % a.gm, tn = jb % pn * gn + x / a.gm;
   if (tm >= a.nM || tn >= a.nN) return;
   const int m0 = tm * BM, n0 = tn * BN;
-  const int G = a.K / 64, nk = a.K / 16, nx = (G + 15) / 16, ns = nk + nx;
+  const int G = a.K / 64, nk = a.K / 16, nx = (G + 15) / 16, rb = (int)rows_block(nk, nx);
   const int kk = split * KS + kq, KT = KS * a.S;
   const int g0 = G * kk / KT, g1 = G * (kk + 1) / KT;
 
   // wave-uniform bases with 32-bit lane offsets (registers, not 64-bit addresses, are short here)
-  const u32x4 *ab = reinterpret_cast<const u32x4 *>(a.x) + ((size_t)(m0 >> 5) * ns) * 128;
+  const u32x4 *ab = reinterpret_cast<const u32x4 *>(a.x) + (size_t)(m0 >> 5) * rb;
   const uint8_t *cb = reinterpret_cast<const uint8_t *>(a.codes) + (size_t)(n0 >> 5) * G * (BITS * 256);
 
   floatx16 acc[TM][TN];
@@ -250,7 +247,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   auto load_a = [&](int g, int s4, u32x4(&f)[TM][2]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      const u32x4 *p = ab + ((size_t)i * ns + min(g, g1 - 1) * 4 + s4) * 128;
+      const u32x4 *p = ab + (size_t)i * rb + (min(g, g1 - 1) * 4 + s4) * 128;
       f[i][0] = p[lane];
       f[i][1] = p[lane + 64];
     }
@@ -285,41 +282,28 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
   };
   // the bias term's steps first (their loads go out ahead of the rings')
   const int x0 = nx * kk / KT, x1 = nx * (kk + 1) / KT;
-  float bs[TN];
-#pragma unroll
-  for (int j = 0; j < TN; j++) bs[j] = x0 < x1 ? (a.scale + (size_t)G * a.ldn + n0 + j * 32)[r31] : 1.0f;
   for (int kx = x0; kx < x1; kx++) {
-    u32x4 xa[TM][2], xb[TN][2];
+    u32x4 xa[TM][3], xb[TN][3];
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      const u32x4 *p = ab + ((size_t)i * ns + nk + kx) * 128;
-      xa[i][0] = p[lane];
-      xa[i][1] = p[lane + 64];
+      const u32x4 *p = ab + (size_t)i * rb + nk * 128 + kx * 192;
+#pragma unroll
+      for (int q = 0; q < 3; q++) xa[i][q] = p[lane + 64 * q];
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      const u32x4 *p = reinterpret_cast<const u32x4 *>(a.bw) + ((size_t)((n0 >> 5) + j) * nx + kx) * 128;
-      xb[j][0] = p[lane];
-      xb[j][1] = p[lane + 64];
+      const u32x4 *p = reinterpret_cast<const u32x4 *>(a.bw) + ((size_t)((n0 >> 5) + j) * nx + kx) * 192;
+#pragma unroll
+      for (int q = 0; q < 3; q++) xb[j][q] = p[lane + 64 * q];
     }
     if (kx == x0 && g0 < g1) {
       load_rings();
     }
 #pragma unroll
-    for (int p = 0; p < 3; p++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-          acc[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, xa[i][p == 2]), __builtin_bit_cast(f16x8, xb[j][p == 1]),
-                                  acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; j++) acc[i][j] = mma_planes<Bf16Triples, 3>(xa[i], xb[j], acc[i][j]);
   }
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] *= bs[j];
   if (x0 == x1 && g0 < g1) {
     load_rings();
   }
@@ -594,15 +578,16 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       m2 = sum8(m2);
       gs = sum8(gs);
       if (!live) continue;
-      const int onk = a.N / 16, ons = onk + (a.N / 64 + 15) / 16;
+      const int onk = a.N / 16;
+      const size_t orb = rows_block_of(a.N);
       u32x4 hi, lo;
       split8(y, hi, lo);
       u32x4 *out = reinterpret_cast<u32x4 *>(a.o);
-      const size_t pc = rows_piece(r, n >> 3, ons);
+      const size_t pc = rows_piece(r, n >> 3, orb);
       out[pc] = hi;
       out[pc + 64] = lo;
       if (c == 0) {
-        put_group_sum(out, r, n >> 6, onk, ons, gs);
+        put_group_sum(out, r, n >> 6, onk, orb, gs);
         a.so[(size_t)r * (a.N / 64) + (n >> 6)] = make_float2(mean, m2);
       }
     }
@@ -618,14 +603,15 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       }
       gs = sum8(gs);
       if (r >= a.M) continue;
-      const int onk = a.N / 16, ons = onk + (a.N / 64 + 15) / 16;
+      const int onk = a.N / 16;
+      const size_t orb = rows_block_of(a.N);
       u32x4 hi, lo;
       split8(v, hi, lo);
       u32x4 *out = reinterpret_cast<u32x4 *>(a.o);
-      const size_t pc = rows_piece(r, n >> 3, ons);
+      const size_t pc = rows_piece(r, n >> 3, orb);
       out[pc] = hi;
       out[pc + 64] = lo;
-      if (c == 0) put_group_sum(out, r, n >> 6, onk, ons, gs);
+      if (c == 0) put_group_sum(out, r, n >> 6, onk, orb, gs);
     }
   } else {
     // the 64 columns are one head of q, k or v: the attention's fragments (q scaled by
@@ -756,7 +742,8 @@ __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, cons
   flash_merge<4>(st, buf, g, lane);
   if (g != 0) return;
   const float inv = 1.0f / st.l;
-  const int nk = d / 16, ns = nk + (d / 64 + 15) / 16;
+  const int nk = d / 16;
+  const size_t rb = rows_block_of(d);
   float gs = 0.0f;
 #pragma unroll
   for (int dt = 0; dt < 2; dt++)
@@ -779,11 +766,11 @@ __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, cons
         hi[j] = hw;
         lo[j] = lw;
       }
-      u32x2 *p = reinterpret_cast<u32x2 *>(out + rows_piece(t, head * 8 + dt * 4 + a8, ns)) + (lane >> 5);
+      u32x2 *p = reinterpret_cast<u32x2 *>(out + rows_piece(t, head * 8 + dt * 4 + a8, rb)) + (lane >> 5);
       p[0] = hi;
       p[128] = lo;
     }
-  if (lane < 32) put_group_sum(out, t, head, nk, ns, gs);
+  if (lane < 32) put_group_sum(out, t, head, nk, rb, gs);
 }
 
 // (row parts of the XCDs: the split with the fewest operand bytes read by each)
@@ -857,13 +844,13 @@ hipError_t dispatch(const RowsMm &a, int epi, int kvt, hipStream_t s) {
 
 }  // namespace
 
-size_t rows_planes_pieces(int M, int K) { return (size_t)((M + 63) / 64 * 2) * (K / 16 + (K / 64 + 15) / 16) * 128; }
+size_t rows_planes_pieces(int M, int K) { return (M + 63) / 64 * 2 * rows_block(K / 16, (K / 64 + 15) / 16); }
 size_t rows_q_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * 4 * 192; }
 size_t rows_kv_pieces(int M, int H) { return (size_t)H * ((M + 63) / 64 * 2) * flash_tile_pieces(3); }
 int rows_ldn(int N) { return (N + 63) / 64 * 64; }
-size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64 + 1) * rows_ldn(N); }
+size_t rows_scale_floats(int N, int K) { return (size_t)(K / 64) * rows_ldn(N); }
 size_t rows_codes_bytes(int N, int K, int bits) { return (size_t)rows_ldn(N) * K * bits / 8; }
-size_t rows_bias_pieces(int N, int K) { return (size_t)(rows_ldn(N) / 32) * ((K / 64 + 15) / 16) * 128; }
+size_t rows_bias_pieces(int N, int K) { return rows_ldn(N) / 32 * rows_block(0, (K / 64 + 15) / 16); }
 
 hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float *scale, uint4 *bw, void *params,
                        hipStream_t s) {

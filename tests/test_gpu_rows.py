@@ -174,3 +174,22 @@ def test_product_range_of_f32_params(bits, scale, offset):
     # 22-bit operands and fp32 sums of the terms' magnitudes (codes and group sums, s times half the
     # code range an element)
     assert np.all(np.abs(got - ref) <= 4e-6 * (bound + scale * top / 2 * np.abs(x).sum(1, keepdims=True) / 8))
+
+
+# activations of one sign: a group's sum is 64 of them, far past the range of an element
+@pytest.mark.parametrize("big", [1.0, 1e4, 6e4])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M", [5, 40, 70, 600])
+def test_product_of_one_signed_activations(bits, big, M):
+    say(f"[gpu] product of activations around {big}, M={M} bits={bits}")
+    _, g, _ = _model(8, H.ITTS_F16)
+    N, K = 130, 1280
+    rng = np.random.default_rng(M)
+    codes, s, b = H.quantize((rng.standard_normal((N, K)) * 0.02).astype(np.float32), bits, H.ITTS_F32)
+    x = (big * rng.uniform(0.9, 1.1, (M, K))).astype(np.float32)
+    got = g.qlinear_forward(codes, s, b, np.zeros(N, np.float32), x, N, K, bits, H.ITTS_F32)
+    Wd = ito.dequant(synth.QLinear(codes, s, b, np.zeros(N, np.float32), N, K), bits, H.ITTS_F32).astype(np.float64)
+    bound = np.abs(x).astype(np.float64) @ np.abs(Wd).T
+    # the products' bar (22-bit operands, fp32 sums), whatever the magnitude: below 65504 both
+    # planes of an activation are in range
+    assert np.all(np.abs(got - x.astype(np.float64) @ Wd.T) <= 4e-6 * bound)
