@@ -57,47 +57,104 @@ __device__ __forceinline__ float sum8(float v) {  // over eight consecutive lane
   return v + dpp_pair<0x141>(v);
 }
 
-// LayerNorm of rows (a second one with w2; none without w) as planes and group sums; one wave a row.
+// LayerNorm of M rows (a second one with w2; none without w) as planes and group sums.  Half a
+// wave a row (lane c of it: chunks c, c + 32, ..); the row in NC chunks of registers, loaded with
+// its parameters in one memory round trip, or any d with NC = 0 (read again for each pass).
+// Bound by latency: 886 x 1280 6.1 us (7.3 with a quarter of a wave a row, 12 with a row a
+// wave, read again for each pass).
+template <int NC>
 __global__ __launch_bounds__(64) void ln_planes_kernel(const float *x, const float *w, const float *b, const float *w2,
-                                                       const float *b2, int d, u32x4 *out) {
-  const int row = blockIdx.x, lane = threadIdx.x, nc = d / 8, nk = d / 16;
+                                                       const float *b2, int M, int d, u32x4 *out) {
+  constexpr int ND = NC ? NC : 1;
+  const int lane = threadIdx.x, c = lane & 31, row = blockIdx.x * 2 + (lane >> 5);
+  const int nc = d / 8, nk = d / 16, nj = (nc + 31) / 32;
   const size_t rb = rows_block_of(d);
-  const float *xr = x + (size_t)row * d;
-  // mean and 1 / std over f(element) (the row is read again for each pass, from the caches)
-  auto stats = [&](auto f, float &mean, float &rstd) __attribute__((always_inline)) {
-    float s = 0.0f;
-    for (int i = lane; i < d; i += 64) s += f(i);
-    mean = wave64_sum_dpp(s) / (float)d;
-    float q = 0.0f;
-    for (int i = lane; i < d; i += 64) {
-      const float e = f(i) - mean;
-      q += e * e;
-    }
-    rstd = 1.0f / sqrtf(wave64_sum_dpp(q) / (float)d + 1e-5f);
+  const float *xr = x + (size_t)min(row, M - 1) * d;
+  float v[ND][8], g[ND][8], h[ND][8];  // the row and its LayerNorm's parameters
+  auto load8 = [&](const float *p, float (&o)[8]) __attribute__((always_inline)) {
+    const float4 a = reinterpret_cast<const float4 *>(p)[0], e = reinterpret_cast<const float4 *>(p)[1];
+    o[0] = a.x, o[1] = a.y, o[2] = a.z, o[3] = a.w, o[4] = e.x, o[5] = e.y, o[6] = e.z, o[7] = e.w;
+  };
+  auto params = [&](const float *gw, const float *gb, int k, int i) __attribute__((always_inline)) {
+    load8(gw + k * 8, g[i]);
+    load8(gb + k * 8, h[i]);
   };
   float m1 = 0.0f, r1 = 1.0f, m2 = 0.0f, r2 = 1.0f;
-  auto f1 = [&](int i) __attribute__((always_inline)) { return w ? (xr[i] - m1) * r1 * w[i] + b[i] : xr[i]; };
-  if (w) stats([&](int i) __attribute__((always_inline)) { return xr[i]; }, m1, r1);
-  if (w2) stats(f1, m2, r2);
-  for (int c = lane; c < (nc + 63) / 64 * 64; c += 64) {
-    float v[8], g = 0.0f;
+  int done = 0;  // LayerNorms applied to v
+  auto norm = [&](float (&y)[8], int i, float m, float r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int i = min(c, nc - 1) * 8 + j;
-      float y = f1(i);
-      if (w2) y = (y - m2) * r2 * w2[i] + b2[i];
-      v[j] = y;
-      g += y;
+    for (int e = 0; e < 8; e++) y[e] = (y[e] - m) * r * g[i][e] + h[i][e];
+  };
+  // f(chunk, register index, live) over the lane's chunks; chunks past the row repeat its last one
+  auto each = [&](auto f) __attribute__((always_inline)) {
+    if constexpr (NC > 0) {
+#pragma unroll
+      for (int j = 0; j < NC; j++) f(min(c + 32 * j, nc - 1), j, c + 32 * j < nc);
+    } else {
+      for (int j = 0; j < nj; j++) {
+        const int k = min(c + 32 * j, nc - 1);
+        load8(xr + k * 8, v[0]);
+        if (done > 0) {
+          params(w, b, k, 0);
+          norm(v[0], 0, m1, r1);
+        }
+        if (done > 1) {
+          params(w2, b2, k, 0);
+          norm(v[0], 0, m2, r2);
+        }
+        f(k, 0, c + 32 * j < nc);
+      }
     }
-    g = sum8(g);
-    if (c >= nc) continue;
+  };
+  auto stats = [&](float &mean, float &rstd) __attribute__((always_inline)) {
+    float s = 0.0f, q = 0.0f;
+    each([&](int, int i, bool live) __attribute__((always_inline)) {
+      const float t = ((v[i][0] + v[i][1]) + (v[i][2] + v[i][3])) + ((v[i][4] + v[i][5]) + (v[i][6] + v[i][7]));
+      s += live ? t : 0.0f;
+    });
+    mean = half32_sum(s) / (float)d;
+    each([&](int, int i, bool live) __attribute__((always_inline)) {
+      float t = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) t += (v[i][e] - mean) * (v[i][e] - mean);
+      q += live ? t : 0.0f;
+    });
+    rstd = 1.0f / sqrtf(half32_sum(q) / (float)d + 1e-5f);
+  };
+  if constexpr (NC > 0) {
+    each([&](int k, int i, bool) __attribute__((always_inline)) {
+      load8(xr + k * 8, v[i]);
+      if (w) params(w, b, k, i);
+    });
+  }
+  if (w) {
+    stats(m1, r1);
+    if constexpr (NC > 0) {
+      each([&](int k, int i, bool) __attribute__((always_inline)) {
+        norm(v[i], i, m1, r1);
+        if (w2) params(w2, b2, k, i);
+      });
+    }
+    done = 1;
+  }
+  if (w2) {
+    stats(m2, r2);
+    if constexpr (NC > 0) {
+      each([&](int, int i, bool) __attribute__((always_inline)) { norm(v[i], i, m2, r2); });
+    }
+    done = 2;
+  }
+  each([&](int k, int i, bool live) __attribute__((always_inline)) {
+    const float t = ((v[i][0] + v[i][1]) + (v[i][2] + v[i][3])) + ((v[i][4] + v[i][5]) + (v[i][6] + v[i][7]));
+    const float gs = sum8(t);
+    if (!live || row >= M) return;
     u32x4 hi, lo;
-    split8(v, hi, lo);
-    const size_t p = rows_piece(row, c, rb);
+    split8(v[i], hi, lo);
+    const size_t p = rows_piece(row, k, rb);
     out[p] = hi;
     out[p + 64] = lo;
-    if ((c & 7) == 0) put_group_sum(out, row, c >> 3, nk, rb, g);
-  }
+    if ((k & 7) == 0) put_group_sum(out, row, k >> 3, nk, rb, gs);
+  });
 }
 
 // ---- weights ----------------------------------------------------------------------------
@@ -874,7 +931,8 @@ hipError_t rows_params(const DevQL &ql, int bits, int ptype, uint4 *codes, float
 
 hipError_t rows_ln(const float *x, const float *w, const float *b, const float *w2, const float *b2, int M, int d,
                    uint4 *out, hipStream_t s) {
-  hipLaunchKernelGGL(ln_planes_kernel, dim3(M), dim3(64), 0, s, x, w, b, w2, b2, d, reinterpret_cast<u32x4 *>(out));
+  auto *fn = d <= 512 ? ln_planes_kernel<2> : d <= 1280 ? ln_planes_kernel<5> : d <= 2048 ? ln_planes_kernel<8> : ln_planes_kernel<0>;
+  hipLaunchKernelGGL(fn, dim3((M + 1) / 2), dim3(64), 0, s, x, w, b, w2, b2, M, d, reinterpret_cast<u32x4 *>(out));
   return hipGetLastError();
 }
 

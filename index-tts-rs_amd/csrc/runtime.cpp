@@ -464,6 +464,14 @@ struct ProbeSpec {
 // throughout: 235 rows 1645 -> 1685 us, 886 rows 3600 -> 3785, replay of 1400 codes 6360 -> 6830.
 constexpr int kExactAttnRows = 384;
 
+// Above this many rows the LayerNorms run before the products' operands are formed, not folded
+// into them: the fold wants gamma x itself within the planes' range and multiplies what a row's
+// mean, far above its deviation, cancels (mean 100, deviation 1: the last row's error 4 times as
+// large).  The products lose their folds' work, so that the row kernels cost little there (fold /
+// row kernels, prefill in us: 25 rows 1200 / 1344, 235 rows 1650 / 1737, 512 rows 2400 / 2440, 547
+// rows 2685 / 2745, 886 rows 3665 / 3720, 1236 rows 4920 / 4960).
+constexpr int kFoldRows = 512;
+
 // Runs n_layers blocks over the M rows in gpt->px on operands in fragment order.  Row
 // r attends to keys kstart[r] (or 0) .. r; K/V rows go to kv's cache (prefill) or, for the
 // layers that are probed, to the fp32 scratch rk / rv.  ln_1 (after layer 0) and ln_2 are
@@ -476,7 +484,7 @@ itts_status rows_stack(itts_gpt *g, itts_kv *kv, int M, int n_layers, const int 
   const int kvt = kv && (kv->kvt == kKvBf16 || M <= kExactAttnRows) ? kv->kvt : kRowsPairs;
   hipStream_t s = g->stream;
   float *X = g->px.as<float>();
-  const bool folded = g->fold.p != nullptr && d <= 32 * kGroup;  // (a row's group statistics in registers)
+  const bool folded = g->fold.p != nullptr && d <= 32 * kGroup && M <= kFoldRows;  // (a row's group statistics in registers)
   const size_t per = fold_floats(d, F);
   float2 *st = g->pst.as<float2>();
   for (int l = 0; l < n_layers; l++) {

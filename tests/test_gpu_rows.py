@@ -8,6 +8,7 @@ import pytest
 import ito
 import itts_hip as H
 from itts_hip import synth
+from test_oracle_independent import numpy_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -193,3 +194,44 @@ def test_product_of_one_signed_activations(bits, big, M):
     # the products' bar (22-bit operands, fp32 sums), whatever the magnitude: below 65504 both
     # planes of an activation are in range
     assert np.all(np.abs(got - x.astype(np.float64) @ Wd.T) <= 4e-6 * bound)
+
+
+@pytest.mark.parametrize("mean,outlier", [(0.0, 0.0), (100.0, 0.0), (0.0, 2e5)])
+def test_long_prompt_of_uncentred_rows(mean, outlier):
+    """Rows of a large mean, and one channel past the operand planes' range, at more than 512 rows:
+    no further from float64 than the oracle's own fp32 rounding takes the oracle (twice its root
+    mean square; the rounding of the residual rows, which both share, makes most of it)."""
+    say(f"[gpu] 600 rows of mean {mean}, outlier channel {outlier}")
+    W = synth.make_weights(dict(synth.SMALL_CONFIG, param_dtype=H.ITTS_F32), seed=23, init="rich")
+    pr = synth.make_prompt(W.cfg, 3, 25, seed=1)
+    for tab in (W.mel_emb, W.text_emb, W.lang_emb, pr.conds):
+        tab += np.float32(mean)
+        tab[:, 5] += np.float32(outlier)
+    g, M = H.Gpt(W), ito.Model(W)
+    prior = (np.arange(569, dtype=np.int32) * 13) % (W.cfg["mel_vocab"] - 2)
+    emb = M.sequence_embedding(pr.text_tokens, pr.conds, pr.lang_id, prior)
+    exact = numpy_forward(W, emb)
+    rms = lambda a: float(np.sqrt(((a - exact) ** 2).mean()))  # noqa: E731
+    bar = 2 * rms(M.forward_rows(M.kv(600, kv_bf16=False), emb, 0)) + 1e-7 * float(np.abs(exact).max())
+    got = g.forward_logits([H.CodePrompt(pr.text_tokens, pr.conds, pr.lang_id, prior)])
+    assert len(got) == len(emb) == 600 and rms(got) < bar, (rms(got), bar)
+    last = g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, prior, g.kv_cache(600, H.ITTS_F32))
+    err = np.abs(last - exact[-1]).max()
+    assert err < 6 * bar, (float(err), bar)  # six standard deviations, of a thousand logits
+    g.close()
+
+
+@pytest.mark.parametrize("n_head", [1, 8, 9, 20, 21, 32, 33])
+def test_layernorm_widths(n_head):
+    """The row kernel's register widths and its last one, which reads rows again: one row, two, and
+    an odd count, one LayerNorm and two (the all-row head)."""
+    cfg = dict(synth.TINY_CONFIG, n_layer=1, d_model=64 * n_head, n_head=n_head, d_ffn=128, text_vocab=50, mel_vocab=130)
+    W = synth.make_weights(cfg, seed=n_head, init="rich")
+    g, M = H.Gpt(W), ito.Model(W)
+    for n in (2, 3, 4):
+        pr = synth.make_prompt(cfg, 0, n, seed=n)
+        emb = M.sequence_embedding(pr.text_tokens, pr.conds, pr.lang_id, [])
+        ref = M.forward_rows(M.kv(64, kv_bf16=False), emb, 0)
+        got = g.forward_logits([H.CodePrompt(pr.text_tokens, pr.conds, pr.lang_id, None)])
+        assert got.shape == ref.shape and np.abs(got - ref).max() < 2e-5 * max(1.0, np.abs(ref).max())
+    g.close()
