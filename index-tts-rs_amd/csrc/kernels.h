@@ -133,7 +133,8 @@ struct FoldIn {
 
 struct GemmArgs {
   DevQL ql;
-  // few-row products: the codes in fragment order and the (scale, bias) words [K/64][ldn]
+  // few-row products: the codes in fragment order and the (scale, bias) words [K/64][ldn] (null:
+  // kEpiStore reads ql's, the others take the tiles)
   const uint4 *fcodes;
   const void *fparams;
   int ldn;

@@ -620,8 +620,8 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
 // The 64-row tiles above spend most of a launch filling the ring for a few real rows.  Here
 // a block of kFewWaves waves takes 64 output columns (two 32-column MFMA tiles) over
 // kFewWaves K groups, one per wave, with no LDS staging: each lane loads its activation and code
-// fragments straight into registers (a lane's 16 codes of a column are one 16-byte load
-// of the codes' copy in fragment order, its 16 activations of a row two), in the K order the tiles above use.  Rows past M are
+// fragments straight into registers (a lane's 16 codes of a column are one 16-byte load,
+// its 16 activations of a row two), in the K order the tiles above use.  Rows past M are
 // zero fragments; in the 32 x 32 result a lane's rows 4h .. 4h+3 (h = lane >> 5) are the
 // only live ones.  The waves' partials are added in wave order in LDS; the K splits
 // (blocks) in split order by the last block of the column tile to arrive, as above.
@@ -640,7 +640,10 @@ constexpr int kFewEPT = 512 / (64 * kFewWaves);  // of a tile's 8 x 64 results, 
 // rstd of row w (biased variance, eps 1e-5, over K/256 float4s a lane in registers) beside
 // the product; the epilogue takes rstd (sum - mean G[n]) + c[n].
 constexpr int kFoldQ = 8;  // float4s a lane of a row's statistics: K <= 2048
-template <int BITS, int PT, int EPI, int KVT, bool FOLD>
+// FRAG: codes and parameters from the weight's copies in fragment order; without it from the
+// row-major ones (a product of its own, whose weight is used once: the copies would cost more
+// than they save).
+template <int BITS, int PT, int EPI, int KVT, bool FOLD, bool FRAG = true>
 __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN, int S, int gw) {
   __shared__ float red[kFewWaves][512];
   __shared__ float gel[kFewRows][65];
@@ -709,23 +712,27 @@ __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN,
         xa[gi][1][kp][1] = pl[1];
       }
     }
-    // code fragments and parameters of columns n0 + 32 j + c, from the copies in fragment order
-    // (columns past N hold zeros; a group past G reads group 0)
+    // code fragments and parameters of columns n0 + 32 j + c (columns past N: the copies hold
+    // zeros, of the rows column N - 1 is read; a group past G reads group 0)
     const int gl = live ? g : 0;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const uint8_t *cf = reinterpret_cast<const uint8_t *>(a.fcodes) + ((size_t)(2 * tn + j) * G + gl) * (BITS * 256) +
-                          lane * (BITS * 2);
+      const int n = min(n0 + 32 * j + c, N - 1);
+      const uint8_t *cf = FRAG ? reinterpret_cast<const uint8_t *>(a.fcodes) +
+                                     ((size_t)(2 * tn + j) * G + gl) * (BITS * 256) + lane * (BITS * 2)
+                               : a.ql.codes + (size_t)n * (K / 8 * BITS) + gl * (BITS * 8) + h * (BITS * 2);
+      constexpr int KP = FRAG ? BITS * 128 : BITS * 4;
 #pragma unroll
       for (int kp = 0; kp < 2; kp++) {
         if constexpr (BITS == 8) {
-          cq[gi][j][kp] = *reinterpret_cast<const u32x4 *>(cf + kp * (BITS * 128));
+          cq[gi][j][kp] = *reinterpret_cast<const u32x4 *>(cf + kp * KP);
         } else {
-          const uint2 v = *reinterpret_cast<const uint2 *>(cf + kp * (BITS * 128));
+          const uint2 v = *reinterpret_cast<const uint2 *>(cf + kp * KP);
           cq[gi][j][kp] = u32x4{v.x, v.y, 0u, 0u};
         }
       }
-      pr[gi][j] = static_cast<const PRaw *>(a.fparams)[(size_t)gl * a.ldn + n0 + 32 * j + c];
+      pr[gi][j] = FRAG ? static_cast<const PRaw *>(a.fparams)[(size_t)gl * a.ldn + n0 + 32 * j + c]
+                       : static_cast<const PRaw *>(a.ql.params)[(size_t)n * G + gl];
     }
     if constexpr (!FOLD) {
 #pragma unroll
@@ -1093,9 +1100,9 @@ hipError_t gemm_dispatch(const GemmArgs &a, const Plan &p, int epi, int kvt, hip
   }
 }
 
-template <int BITS, int PT, int EPI, int KVT, bool FOLD = false>
+template <int BITS, int PT, int EPI, int KVT, bool FOLD = false, bool FRAG = true>
 hipError_t few_launch(const GemmArgs &a, int nN, int S, int gw, hipStream_t s) {
-  hipLaunchKernelGGL((few_kernel<BITS, PT, EPI, KVT, FOLD>), dim3(nN * S), dim3(64 * kFewWaves), 0, s, a, nN, S,
+  hipLaunchKernelGGL((few_kernel<BITS, PT, EPI, KVT, FOLD, FRAG>), dim3(nN * S), dim3(64 * kFewWaves), 0, s, a, nN, S,
                      gw);
   return hipGetLastError();
 }
@@ -1104,7 +1111,8 @@ template <int BITS, int PT>
 hipError_t few_dispatch(const GemmArgs &a, int nN, int S, int gw, int epi, int kvt, hipStream_t s) {
   switch (epi) {
     case kEpiStore:
-      return few_launch<BITS, PT, kEpiStore, 0>(a, nN, S, gw, s);
+      return a.fcodes ? few_launch<BITS, PT, kEpiStore, 0>(a, nN, S, gw, s)
+                      : few_launch<BITS, PT, kEpiStore, 0, false, false>(a, nN, S, gw, s);
     case kEpiResid:
       return few_launch<BITS, PT, kEpiResid, 0>(a, nN, S, gw, s);
     case kEpiGelu:
@@ -1144,7 +1152,7 @@ hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt,
         (epi != kEpiQKV && epi != kEpiGelu) || !a.fold.gamma || !a.fold.G || !a.fold.c)
       return hipErrorInvalidValue;
   }
-  if (a.M <= kFewRows && (bits == 8 || bits == 4) && a.fcodes) {
+  if (a.M <= kFewRows && (bits == 8 || bits == 4) && (a.fcodes || epi == kEpiStore)) {
     // a group per wave while that keeps the splits within kFewMaxSplits (gw > kFewMaxGw
     // beyond that: the tiled GEMM)
     const int nN = (a.ql.N + 63) / 64, G = a.ql.K / kGroup;

@@ -155,18 +155,30 @@ bool valid_config(const itts_config &c, std::string &why) {
 // Handles
 // ------------------------------------------------------------------------------------
 
+size_t round256(size_t n) { return (n + 255) / 256 * 256; }
+
 struct QLHost {
   DevBuf codes, params, bias;
-  // the multi-row products' codes, scale table, bias planes and parameter words
-  DevBuf rcodes, rscale, rbias, rwords;
-  hipError_t ready_rows(int bits, int ptype, hipStream_t s) {
-    hipError_t e = rcodes.ensure(rows_codes_bytes(N, K, bits));
-    if (e == hipSuccess) e = rscale.ensure(sizeof(float) * rows_scale_floats(N, K));
-    if (e == hipSuccess) e = rbias.ensure(sizeof(uint4) * rows_bias_pieces(N, K));
-    if (e == hipSuccess) e = rwords.ensure((ptype == kParamF32 ? 8 : 4) * rows_scale_floats(N, K));
-    if (e == hipSuccess)
-      e = rows_params(dev(), bits, ptype, rcodes.as<uint4>(), rscale.as<float>(), rbias.as<uint4>(), rwords.p, s);
-    return e;
+  // the multi-row products' codes, scale table, bias planes and parameter words, in memory that the
+  // decoder keeps for all its weights (one allocation: four a weight took half of create's time)
+  uint4 *rcodes = nullptr, *rbias = nullptr;
+  float *rscale = nullptr;
+  void *rwords = nullptr;
+  static size_t rows_bytes(int N, int K, int bits, int ptype) {
+    return round256(rows_codes_bytes(N, K, bits)) + round256(sizeof(float) * rows_scale_floats(N, K)) +
+           round256(sizeof(uint4) * rows_bias_pieces(N, K)) +
+           round256((ptype == kParamF32 ? 8 : 4) * rows_scale_floats(N, K));
+  }
+  // mem: rows_bytes bytes
+  hipError_t ready_rows(char *mem, int bits, int ptype, hipStream_t s) {
+    rcodes = reinterpret_cast<uint4 *>(mem);
+    mem += round256(rows_codes_bytes(N, K, bits));
+    rscale = reinterpret_cast<float *>(mem);
+    mem += round256(sizeof(float) * rows_scale_floats(N, K));
+    rbias = reinterpret_cast<uint4 *>(mem);
+    mem += round256(sizeof(uint4) * rows_bias_pieces(N, K));
+    rwords = mem;
+    return rows_params(dev(), bits, ptype, rcodes, rscale, rbias, rwords, s);
   }
   DevQL dev() const { return DevQL{codes.as<uint8_t>(), params.p, bias.as<float>(), N, K}; }
   int N = 0, K = 0;
@@ -187,6 +199,8 @@ struct itts_gpt {
   DevBuf text_emb, lang_emb, mel_emb, mel_pos, text_pos;
   std::vector<DevBuf> ln;  // ln1_w, ln1_b, ln2_w, ln2_b per layer, then ln_f, final_norm
   std::vector<QLHost> qls; // 4 per layer, then mel_head
+  DevBuf rows_mem;         // their copies in fragment order
+  DevBuf ql_rows;          // the same of itts_qlinear_forward's weight (the last one's)
   std::vector<DevLayer> layers;
   DevBuf ln_f_w, ln_f_b, fn_w, fn_b;
   DevQL head{};
@@ -325,8 +339,8 @@ DevSampling to_dev_sampling(const itts_sampling &p, int n) {
 GemmArgs gemm_args(const itts_gpt *g, const QLHost &q, SplitAct x, int M) {
   GemmArgs ga{};
   ga.ql = q.dev();
-  ga.fcodes = q.rcodes.as<uint4>();
-  ga.fparams = q.rwords.p;
+  ga.fcodes = q.rcodes;
+  ga.fparams = q.rwords;
   ga.ldn = rows_ldn(q.N);
   ga.x = x;
   ga.M = M;
@@ -353,9 +367,9 @@ hipError_t ensure_planes(itts_gpt *g, DevBuf &buf, int M, int K) {
 RowsMm rows_args(const itts_gpt *g, const QLHost &q, const DevBuf &x, int M) {
   RowsMm a{};
   a.x = x.as<uint4>();
-  a.codes = q.rcodes.as<uint4>();
-  a.scale = q.rscale.as<float>();
-  a.bw = q.rbias.as<uint4>();
+  a.codes = q.rcodes;
+  a.scale = q.rscale;
+  a.bw = q.rbias;
   a.bias = q.bias.as<float>();
   a.ldn = rows_ldn(q.N);
   a.ws = g->gws.as<float>();
@@ -1146,9 +1160,16 @@ itts_status itts_gpt_create(const itts_weights *w, itts_gpt **out) {
       if (hipStreamSynchronize(g->stream) != hipSuccess)
         return fail(set_error(ITTS_E_DEVICE, "LayerNorm fold failed"));
     }
-    for (QLHost &q : g->qls)
-      if (q.ready_rows(bits, g->ptype(), g->stream) != hipSuccess)
-        return fail(set_error(ITTS_E_DEVICE, "laying out the multi-row products' weights failed"));
+    size_t need = 0;
+    for (const QLHost &q : g->qls) need += QLHost::rows_bytes(q.N, q.K, bits, g->ptype());
+    hipError_t e = g->rows_mem.ensure(need);
+    size_t at = 0;
+    for (QLHost &q : g->qls) {
+      if (e == hipSuccess) e = q.ready_rows(g->rows_mem.as<char>() + at, bits, g->ptype(), g->stream);
+      at += QLHost::rows_bytes(q.N, q.K, bits, g->ptype());
+    }
+    if (e != hipSuccess)
+      return fail(set_error(ITTS_E_DEVICE, "laying out the multi-row products' weights failed"));
     if (sampler_stage_init(dev) != hipSuccess)
       return fail(set_error(ITTS_E_DEVICE, "sampler staging area lookup failed"));
   }
@@ -2036,10 +2057,13 @@ itts_status itts_qlinear_forward(itts_gpt *gpt, const itts_qlinear *ql, int32_t 
     a.x = dx.as<float>();
     a.y = dy.as<float>();
     HIP_TRY(launch_gemv(a, bits, pt, kProNone, kEpiStore, kKvBf16, gpt->stream));
-  } else if (M > 64) {
+  } else if (M > 512) {
+    // (the copies in fragment order are made for this one product: below, that costs more than
+    // it gains; K 5120, N 1280, in all: 65 rows 419 us against 457, 235 rows equal)
     DevBuf planes;
     HIP_TRY(ensure_planes(gpt, planes, M, K));
-    HIP_TRY(q.ready_rows(bits, pt, gpt->stream));
+    HIP_TRY(gpt->ql_rows.ensure(QLHost::rows_bytes(N, K, bits, pt)));
+    HIP_TRY(q.ready_rows(gpt->ql_rows.as<char>(), bits, pt, gpt->stream));
     HIP_TRY(rows_ln(dx.as<float>(), nullptr, nullptr, nullptr, nullptr, M, K, planes.as<uint4>(), gpt->stream));
     RowsMm a = rows_args(gpt, q, planes, M);
     a.y = dy.as<float>();
@@ -2049,7 +2073,6 @@ itts_status itts_qlinear_forward(itts_gpt *gpt, const itts_qlinear *ql, int32_t 
     SplitBuf xs;
     HIP_TRY(xs.ensure(M, K));
     HIP_TRY(launch_split_rows(dx.as<float>(), M, K, xs.out(), gpt->stream));
-    if (M <= 8) HIP_TRY(q.ready_rows(bits, pt, gpt->stream));
     GemmArgs a = gemm_args(gpt, q, xs.act(), M);
     a.y = dy.as<float>();
     HIP_TRY(launch_gemm(a, bits, pt, kEpiStore, kKvBf16, gpt->stream));

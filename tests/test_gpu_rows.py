@@ -136,9 +136,12 @@ def test_long_k_split_over_blocks():
             assert np.abs(a - b).max() < 2e-5 * max(1.0, np.abs(b).max())
 
 
-# up to 64 rows the 64 x 64 LDS tiles, then 32 x 64 tiles and (K >= 4096, many tiles) 64 x 64
+# qlinear_forward: up to 8 rows the few-row product on row-major codes, up to 512 the 64 x 64 LDS
+# tiles, then 32 x 64 tiles and (K >= 4096, many tiles) 64 x 64 on operands in fragment order
 @pytest.mark.parametrize("bits,pd", [(8, H.ITTS_F16), (4, H.ITTS_F32)])
-@pytest.mark.parametrize("M,N,K", [(49, 37, 192), (65, 130, 64), (100, 1026, 1280), (70, 132, 4160), (2000, 1090, 4096)])
+@pytest.mark.parametrize("M,N,K", [(2, 37, 192), (8, 130, 1280), (49, 37, 192), (65, 130, 64), (100, 1026, 1280), (70, 132, 4160),
+                                   (512, 130, 64), (513, 130, 64), (545, 37, 192), (530, 132, 4160), (577, 1026, 1280),
+                                   (2000, 1090, 4096)])
 def test_product_vs_fp64(bits, pd, M, N, K):
     say(f"[gpu] rows product M={M} N={N} K={K} bits={bits}")
     _, g, _ = _model(8, H.ITTS_F16)
