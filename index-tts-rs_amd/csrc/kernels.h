@@ -43,9 +43,9 @@ struct BatchSeq {
 };
 
 // Where the QKV epilogue scatters: q -> q_out[M][d]; k, v -> this layer's cache
-// [n_head][max_seq][64] at rows pos0.. .  With seqs set (batched decode), row m belongs
-// to sequence m: its K/V row goes to seqs[m]'s cache at offset layer_off (elements) and
-// position ctl->valid_len, and nothing is written for a finished sequence.
+// [n_head][max_seq][64] at row pos0 (the GEMV).  launch_gemm's rows are those of a batched step:
+// row m belongs to sequence m, its K/V row goes to seqs[m]'s cache at offset layer_off (elements)
+// and position ctl->valid_len, and nothing is written for a finished sequence.
 struct QkvDst {
   float *q_out;
   void *k_cache;

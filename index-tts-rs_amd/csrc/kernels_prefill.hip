@@ -11,8 +11,8 @@
 // 4-bit codes enter as the fp16 values 16 + q (bit pattern 0x4C00 | q << 6), so the group
 // term uses b - 16 s in place of b.
 //
-// Block: 512 threads, 2 x 2 worker waves of (32 TM) x (32 TN) outputs, tile (64 TM) x
-// (64 TN), and four copier waves.  The K loop runs over 64-wide groups through an NS-stage
+// Block: 512 threads, 2 x 2 worker waves of 32 x 32 outputs, tile 64 x 64, and four copier
+// waves.  The K loop runs over 64-wide groups through an NS-stage
 // ring of LDS buffers filled by global->LDS DMA (no registers) that only the copiers issue,
 // so the copies overlap the workers' MFMAs; each stage holds the hi/lo activation tile, the
 // code tile, the group sums and the (scale, bias) pairs.  Activation and code rows are XOR
@@ -34,9 +34,10 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void *lds_ptr;
 
-template <int BITS, int PT, int TM, int TN>
+constexpr int BM = 64, BN = 64;  // a block's tile
+
+template <int BITS, int PT>
 struct Shape {
-  static constexpr int BM = 64 * TM, BN = 64 * TN;
   static constexpr int RB = BITS * 8;                          // code bytes per row per group
   static constexpr int A_BYTES = BM * 128;                     // one fp16 plane: 64 values a row
   static constexpr int B_BYTES = BN * RB;
@@ -59,15 +60,10 @@ struct Shape {
 __device__ __forceinline__ int swz_act(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int swz_codes(int bits, int r) { return bits == 8 ? (r >> 2) & 3 : (r >> 3) & 1; }
 
-// Sum over the TPI consecutive lanes of an item: nothing (1) or a DPP quad (4).
-template <int TPI>
-__device__ __forceinline__ float item_sum(float v) {
-  static_assert(TPI == 1 || TPI == 4, "item width");
-  if constexpr (TPI == 4) {
-    v += dpp_pair<0xB1>(v);  // quad_perm [1,0,3,2]
-    v += dpp_pair<0x4E>(v);  // quad_perm [2,3,0,1]
-  }
-  return v;
+// Sum over a quad of consecutive lanes.
+__device__ __forceinline__ float quad_sum(float v) {
+  v += dpp_pair<0xB1>(v);        // quad_perm [1,0,3,2]
+  return v + dpp_pair<0x4E>(v);  // quad_perm [2,3,0,1]
 }
 
 // two consecutive 8-bit codes (bits sh..sh+15 of w) -> packed fp16 pair (exact)
@@ -114,32 +110,28 @@ __device__ __forceinline__ void gstore(T *p, T v) {
 __device__ __forceinline__ void gstore(uint4 *p, uint4 v) {
   *(__attribute__((address_space(1))) u32x4 *)p = u32x4{v.x, v.y, v.z, v.w};
 }
-typedef float f32x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void gstore(float2 *p, float2 v) {
-  *(__attribute__((address_space(1))) f32x2v *)p = f32x2v{v.x, v.y};
-}
 
 struct Tile {
   int tn, tm, ks;
 };
 
-// PROD: 512 threads, waves 4-7 issue every copy and waves 0-3 only compute, so that the
-// copies (bound by the CU's vector-memory path) overlap the MFMA and VALU work instead of
-// running in series with it inside each wave.
-template <int BITS, int PT, int EPI, int KVT, int TM, int TN, int NS, bool PROD>
-__global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void gemm_kernel(GemmArgs a, int mode, int nN, int mt, int S, int gps) {
-  using Sh = Shape<BITS, PT, TM, TN>;
-  constexpr int BM = Sh::BM, BN = Sh::BN, PW = Sh::PW;
+// Waves 4-7 issue every copy and waves 0-3 only compute, so that the copies (bound by the CU's
+// vector-memory path) overlap the MFMA and VALU work instead of running in series with it inside
+// each wave.
+template <int BITS, int PT, int EPI, int KVT, int NS>
+__global__ __launch_bounds__(512, 4) void gemm_kernel(GemmArgs a, int mode, int nN, int mt, int S, int gps) {
+  using Sh = Shape<BITS, PT>;
+  constexpr int PW = Sh::PW;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   __shared__ uint32_t last_flag;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // copier: issues the copies; worker: computes (both, without PROD).  Wave-uniform.
-  const bool copier = !PROD || wave_all >= 4, worker = !PROD || wave_all < 4;
+  // copier: issues the copies; worker: computes.  Wave-uniform.
+  const bool copier = wave_all >= 4, worker = wave_all < 4;
   // the workers' MFMA and VALU instructions issue ahead of the copiers' (235-row prefill
   // 2.41 against 2.45 ms; the copiers raised instead: 2.46 ms)
-  if (PROD && worker) __builtin_amdgcn_s_setprio(3);
+  if (worker) __builtin_amdgcn_s_setprio(3);
   const int wave = wave_all & 3;
   const int wm = wave >> 1, wn = wave & 1;
   const int K = a.ql.K, N = a.ql.N, M = a.M, G = K / kGroup;
@@ -211,23 +203,13 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     }
   };
 
-  floatx16 acc[TM][TN], P0[TM][TN], P1[TM][TN];
-  float2 sbp[TN];
-  floatx4 gsp[TM][4];
+  floatx16 acc, P0, P1;
 #pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
 
-  auto mma = [&](const char *st, floatx16(&P)[TM][TN]) __attribute__((always_inline)) {
+  auto mma = [&](const char *st, floatx16 &P) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) P[i][j][e] = 0.0f;
+    for (int e = 0; e < 16; e++) P[e] = 0.0f;
     // K order inside a group: lane half h = lane >> 5 of MFMA step kk = 2 kp + s takes the 8
     // values 32 kp + 16 h + 8 s .. +7 (the same permutation for activations and codes, so
     // the contraction is unchanged); a lane's codes for both steps of a pair are then one
@@ -235,110 +217,61 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
 #pragma unroll
     for (int kp = 0; kp < 2; kp++) {
       const int h = lane >> 5;
-      f16x8 bq[2][TN];
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int nr = wn * 32 * TN + j * 32 + (lane & 31);
-        if constexpr (BITS == 8) {
-          const u32x4 q =
-              *reinterpret_cast<const u32x4 *>(st + Sh::OFF_B + nr * 64 + (((2 * kp + h) ^ swz_codes(8, nr)) << 4));
-          const u32x4 b0 = {f16_pair_u8(q[0], 0), f16_pair_u8(q[0], 16), f16_pair_u8(q[1], 0), f16_pair_u8(q[1], 16)};
-          const u32x4 b1 = {f16_pair_u8(q[2], 0), f16_pair_u8(q[2], 16), f16_pair_u8(q[3], 0), f16_pair_u8(q[3], 16)};
-          bq[0][j] = __builtin_bit_cast(f16x8, b0);
-          bq[1][j] = __builtin_bit_cast(f16x8, b1);
-        } else {
-          const uint2 q =
-              *reinterpret_cast<const uint2 *>(st + Sh::OFF_B + nr * 32 + ((kp ^ swz_codes(4, nr)) << 4) + h * 8);
-          const u32x4 b0 = {f16_pair_u4(q.x, 0), f16_pair_u4(q.x, 8), f16_pair_u4(q.x, 16), f16_pair_u4(q.x, 24)};
-          const u32x4 b1 = {f16_pair_u4(q.y, 0), f16_pair_u4(q.y, 8), f16_pair_u4(q.y, 16), f16_pair_u4(q.y, 24)};
-          bq[0][j] = __builtin_bit_cast(f16x8, b0);
-          bq[1][j] = __builtin_bit_cast(f16x8, b1);
-        }
+      f16x8 bq[2];
+      const int nr = wn * 32 + (lane & 31);
+      if constexpr (BITS == 8) {
+        const u32x4 q =
+            *reinterpret_cast<const u32x4 *>(st + Sh::OFF_B + nr * 64 + (((2 * kp + h) ^ swz_codes(8, nr)) << 4));
+        const u32x4 b0 = {f16_pair_u8(q[0], 0), f16_pair_u8(q[0], 16), f16_pair_u8(q[1], 0), f16_pair_u8(q[1], 16)};
+        const u32x4 b1 = {f16_pair_u8(q[2], 0), f16_pair_u8(q[2], 16), f16_pair_u8(q[3], 0), f16_pair_u8(q[3], 16)};
+        bq[0] = __builtin_bit_cast(f16x8, b0);
+        bq[1] = __builtin_bit_cast(f16x8, b1);
+      } else {
+        const uint2 q =
+            *reinterpret_cast<const uint2 *>(st + Sh::OFF_B + nr * 32 + ((kp ^ swz_codes(4, nr)) << 4) + h * 8);
+        const u32x4 b0 = {f16_pair_u4(q.x, 0), f16_pair_u4(q.x, 8), f16_pair_u4(q.x, 16), f16_pair_u4(q.x, 24)};
+        const u32x4 b1 = {f16_pair_u4(q.y, 0), f16_pair_u4(q.y, 8), f16_pair_u4(q.y, 16), f16_pair_u4(q.y, 24)};
+        bq[0] = __builtin_bit_cast(f16x8, b0);
+        bq[1] = __builtin_bit_cast(f16x8, b1);
       }
 #pragma unroll
       for (int sub = 0; sub < 2; sub++) {
-        f16x8 ah[TM], al[TM];
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-          const int row = wm * 32 * TM + i * 32 + (lane & 31);
-          const int c = 4 * kp + 2 * h + sub;
-          const int off = row * 128 + ((c ^ swz_act(row)) << 4);
-          ah[i] = *reinterpret_cast<const f16x8 *>(st + off);
-          al[i] = *reinterpret_cast<const f16x8 *>(st + Sh::OFF_LO + off);
-        }
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-          for (int j = 0; j < TN; j++) {
-            P[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bq[sub][j], P[i][j], 0, 0, 0);
-            P[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bq[sub][j], P[i][j], 0, 0, 0);
-          }
+        const int row = wm * 32 + (lane & 31);
+        const int c = 4 * kp + 2 * h + sub;
+        const int off = row * 128 + ((c ^ swz_act(row)) << 4);
+        const f16x8 ah = *reinterpret_cast<const f16x8 *>(st + off);
+        const f16x8 al = *reinterpret_cast<const f16x8 *>(st + Sh::OFF_LO + off);
+        P = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bq[sub], P, 0, 0, 0);
+        P = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bq[sub], P, 0, 0, 0);
       }
     }
   };
 
-  // (scale, bias) of this wave's columns, for the group in st
-  auto read_params = [&](const char *st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-      const int nr = wn * 32 * TN + j * 32 + (lane & 31);
-      float2 sb;
-      if constexpr (PT == kParamF32) {
-        sb = *reinterpret_cast<const float2 *>(st + Sh::OFF_P + nr * 8);
-      } else {
-        const uint32_t w = *reinterpret_cast<const uint32_t *>(st + Sh::OFF_P + nr * 4);
-        sb = make_float2(half_bits_to_float(w & 0xffffu), half_bits_to_float(w >> 16));
-      }
-      if constexpr (BITS == 4) sb.y = sb.y - 16.0f * sb.x;
-      sbp[j] = sb;
+  // The group's affine straight from the stage in LDS: (scale, bias) of the lane's column and the
+  // group sums of its rows.
+  auto apply = [&](const char *st, const floatx16 &P) __attribute__((always_inline)) {
+    const int nr = wn * 32 + (lane & 31), rb = wm * 32 + (lane >> 5) * 4;
+    float2 sb;
+    if constexpr (PT == kParamF32) {
+      sb = *reinterpret_cast<const float2 *>(st + Sh::OFF_P + nr * 8);
+    } else {
+      const uint32_t w = *reinterpret_cast<const uint32_t *>(st + Sh::OFF_P + nr * 4);
+      sb = make_float2(half_bits_to_float(w & 0xffffu), half_bits_to_float(w >> 16));
     }
-  };
-  // ... and the group sums of its rows
-  auto read_group = [&](const char *st) __attribute__((always_inline)) {
-    read_params(st);
+    if constexpr (BITS == 4) sb.y = sb.y - 16.0f * sb.x;
+    floatx4 g[4];
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int rb = wm * 32 * TM + i * 32 + (lane >> 5) * 4;
+    for (int q = 0; q < 4; q++) g[q] = *reinterpret_cast<const floatx4 *>(st + Sh::OFF_G + (rb + q * 8) * 4);
 #pragma unroll
-      for (int q = 0; q < 4; q++) gsp[i][q] = *reinterpret_cast<const floatx4 *>(st + Sh::OFF_G + (rb + q * 8) * 4);
-    }
-  };
-
-  auto apply = [&](const floatx16(&P)[TM][TN]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-          acc[i][j][e] = fmaf(sbp[j].x, P[i][j][e], fmaf(sbp[j].y, gsp[i][e >> 2][e & 3], acc[i][j][e]));
-  };
-
-  // The fold straight from the stage in LDS: the group sums of one M
-  // sub-tile at a time are held in registers, so the fold adds 16 registers to the
-  // partial tile instead of 32.
-  auto apply_from = [&](const char *st, const floatx16(&P)[TM][TN]) __attribute__((always_inline)) {
-    read_params(st);
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int rb = wm * 32 * TM + i * 32 + (lane >> 5) * 4;
-      floatx4 g[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) g[q] = *reinterpret_cast<const floatx4 *>(st + Sh::OFF_G + (rb + q * 8) * 4);
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-          acc[i][j][e] = fmaf(sbp[j].x, P[i][j][e], fmaf(sbp[j].y, g[e >> 2][e & 3], acc[i][j][e]));
-    }
+    for (int e = 0; e < 16; e++) acc[e] = fmaf(sb.x, P[e], fmaf(sb.y, g[e >> 2][e & 3], acc[e]));
   };
 
   auto stage = [&](int i) __attribute__((always_inline)) { return lds + (i % NS) * Sh::STAGE; };
 
   // group i: wait for its copies, start the copies NS-1 groups ahead into the buffer that
-  // group i-1 used, contract, then fold group i-1's partial (its params were read into
-  // registers while the buffer was still valid)
-  auto step = [&](int i, floatx16(&Pc)[TM][TN], const floatx16(&Pp)[TM][TN]) __attribute__((always_inline)) {
+  // group i-1 used, contract and apply its affine at once (one partial tile is live; the other
+  // wave on the SIMD covers the MFMA latency)
+  auto step = [&](int i, floatx16 &P) __attribute__((always_inline)) {
     if (copier) {
       const int ahead = min(NS - 2, ng - 1 - i);
       if (ahead <= 0) {
@@ -352,62 +285,38 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     __syncthreads();
     if (copier && i + NS - 1 < ng) issue(g0 + i + NS - 1, stage(i + NS - 1));
     if (worker) {
-      if constexpr (PROD) {
-        // at two waves per SIMD the group's affine is applied at once, so
-        // only one partial tile is live (the other wave on the SIMD covers the MFMA latency)
-        mma(stage(i), Pc);
-        apply_from(stage(i), Pc);
-      } else {
-        mma(stage(i), Pc);
-        if (i > 0) apply(Pp);
-        read_group(stage(i));
-      }
+      mma(stage(i), P);
+      apply(stage(i), P);
     }
   };
 
   if (copier)
     for (int i = 0; i < NS - 1 && i < ng; i++) issue(g0 + i, stage(i));
-  // The bias of the lane's column on 64 x 64 tiles (one 32-column MFMA tile a wave), loaded here
-  // so the epilogue does not start with a memory round trip.
-  constexpr bool kColEarly = PROD && TM == 1 && TN == 1;
-  float cb = 0.0f;
-  if constexpr (kColEarly) {
-    if (worker) cb = gload(a.ql.bias + min(n0 + wn * 32 + (lane & 31), N - 1));
-  }
+  // The bias of the lane's column, loaded here so the epilogue does not start with a memory round
+  // trip.
+  float bias = 0.0f;
+  if (worker) bias = gload(a.ql.bias + min(n0 + wn * 32 + (lane & 31), N - 1));
   int i = 0;
   for (; i + 1 < ng; i += 2) {
-    step(i, P0, P1);
-    step(i + 1, P1, P0);
+    step(i, P0);
+    step(i + 1, P1);
   }
-  if (i < ng) {
-    step(i, P0, P1);
-    if (worker && !PROD) apply(P0);
-  } else {
-    if (worker && !PROD) apply(P1);
-  }
+  if (i < ng) step(i, P0);
 
-  // Residual epilogues on 64-row tiles: the lane's old rows y, all loaded before any is
-  // used.  Read and written element by element, each load waited behind the previous
-  // element's store (the compiler cannot move a load of y above a store to y): 16 round
-  // trips a lane.
+  const int nc = n0 + wn * 32 + (lane & 31), rb = wm * 32 + (lane >> 5) * 4;  // the lane's column, tile row of element 0
+  // Residual epilogues: the lane's old rows y, all loaded before any is used.  Read and written
+  // element by element, each load waited behind the previous element's store (the compiler cannot
+  // move a load of y above a store to y): 16 round trips a lane.
   constexpr bool kResid = EPI == kEpiResid;
-  float yv[kResid ? TM : 1][kResid ? TN : 1][kResid ? 16 : 1];
+  float yv[kResid ? 16 : 1];
   auto load_y = [&]() __attribute__((always_inline)) {
     if constexpr (kResid) {
+      // indexes clamped rather than loads predicated: one straight run of loads, which
+      // the compiler's wait counting follows exactly (behind branches it waits for every
+      // access in flight, the stores of earlier elements included)
 #pragma unroll
-      for (int i2 = 0; i2 < TM; i2++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-          // indexes clamped rather than loads predicated: one straight run of loads, which
-          // the compiler's wait counting follows exactly (behind branches it waits for every
-          // access in flight, the stores of earlier elements included)
-          const int n = min(n0 + wn * 32 * TN + j * 32 + (lane & 31), N - 1);
-#pragma unroll
-          for (int e = 0; e < 16; e++) {
-            const int m = min(m0 + wm * 32 * TM + i2 * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3), M - 1);
-            yv[i2][j][e] = gload<float>(a.y + (size_t)m * N + n);
-          }
-        }
+      for (int e = 0; e < 16; e++)
+        yv[e] = gload<float>(a.y + (size_t)min(m0 + rb + (e >> 2) * 8 + (e & 3), M - 1) * N + min(nc, N - 1));
     }
   };
 
@@ -421,67 +330,55 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     constexpr int TILE = BM * BN;
     uint64_t *wsb = reinterpret_cast<uint64_t *>(a.ws + (size_t)tile * S * TILE);
     uint64_t *mine = wsb + (size_t)t.ks * (TILE / 2);
-    // register pair h of sub-tile i2 holds rows from `dead` on only when every one of its
-    // rows is past M (few-row tiles): those pairs are neither stored nor summed
-    auto dead = [&](int i2, int h) {
-      return m0 + wm * 32 * TM + i2 * 32 + (h >> 1) * 8 + ((2 * h) & 3) >= M;
-    };
+    // register pair h holds rows from `dead` on only when every one of its rows is past M (few-row
+    // tiles): those pairs are neither stored nor summed
+    auto dead = [&](int h) { return m0 + wm * 32 + (h >> 1) * 8 + ((2 * h) & 3) >= M; };
     if (worker) {
 #pragma unroll
-      for (int i2 = 0; i2 < TM; i2++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-          for (int h = 0; h < 8; h++) {
-            if (dead(i2, h)) continue;
-            const float2 v = make_float2(acc[i2][j][2 * h], acc[i2][j][2 * h + 1]);
-            __hip_atomic_store(mine + ((((wave * TM + i2) * TN + j) * 8 + h) * 64 + lane),
-                               __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
+      for (int h = 0; h < 8; h++) {
+        if (dead(h)) continue;
+        const float2 v = make_float2(acc[2 * h], acc[2 * h + 1]);
+        __hip_atomic_store(mine + ((wave * 8 + h) * 64 + lane), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) last_flag = atomicInc(a.cnt + tile, (uint32_t)(S - 1)) == (uint32_t)(S - 1) ? 1u : 0u;
     __syncthreads();
     if (!last_flag) return;
-    // (the old rows' loads go out ahead of the partials', their latencies overlapping; on
-    // 128-row tiles, whose registers are full here, after them)
-    if (kResid && TM == 1 && worker) load_y();
+    // (the old rows' loads go out ahead of the partials', their latencies overlapping)
+    if (kResid && worker) load_y();
     // splits added in split order (the block's own partial from registers)
     if (worker) {
+      const size_t base = (size_t)(wave * 8) * 64 + lane;
+      floatx16 sum;
+      for (int s2 = 0; s2 < S; s2++) {
+        floatx16 v;
+        if (s2 == t.ks) {
+          v = acc;
+        } else {
 #pragma unroll
-      for (int i2 = 0; i2 < TM; i2++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-          const size_t base = (size_t)(((wave * TM + i2) * TN + j) * 8) * 64 + lane;
-          floatx16 sum;
-          for (int s2 = 0; s2 < S; s2++) {
-            floatx16 v;
-            if (s2 == t.ks) {
-              v = acc[i2][j];
-            } else {
-#pragma unroll
-              for (int h = 0; h < 8; h++) {
-                if (dead(i2, h)) {
-                  v[2 * h] = 0.0f;
-                  v[2 * h + 1] = 0.0f;
-                  continue;
-                }
-                const float2 w = __builtin_bit_cast(
-                    float2, __hip_atomic_load(wsb + (size_t)s2 * (TILE / 2) + base + h * 64, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT));
-                v[2 * h] = w.x;
-                v[2 * h + 1] = w.y;
-              }
+          for (int h = 0; h < 8; h++) {
+            if (dead(h)) {
+              v[2 * h] = 0.0f;
+              v[2 * h + 1] = 0.0f;
+              continue;
             }
-            sum = s2 == 0 ? v : sum + v;
+            const float2 w = __builtin_bit_cast(
+                float2, __hip_atomic_load(wsb + (size_t)s2 * (TILE / 2) + base + h * 64, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT));
+            v[2 * h] = w.x;
+            v[2 * h + 1] = w.y;
           }
-          acc[i2][j] = sum;
         }
+        sum = s2 == 0 ? v : sum + v;
+      }
+      acc = sum;
     }
   }
 
-  if (kResid && S == 1 && TM == 1 && worker) load_y();
+  if (kResid && S == 1 && worker) load_y();
 
   if constexpr (EPI == kEpiGelu) {
     // GELU tile staged in LDS, then written as the next GEMM's input: hi/lo planes and
@@ -489,27 +386,15 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
     constexpr int LDT = BN + 1;
     float *T = reinterpret_cast<float *>(lds);
     __syncthreads();
-    if (worker)
-#pragma unroll
-    for (int i2 = 0; i2 < TM; i2++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int cl = wn * 32 * TN + j * 32 + (lane & 31);
-        const bool nl = n0 + cl < N;
-        const float bias = kColEarly ? cb : nl ? a.ql.bias[n0 + cl] : 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-          const int rl = wm * 32 * TM + i2 * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          T[rl * LDT + cl] = gelu_tanh_exp(acc[i2][j][e] + bias);
-        }
-      }
-    __syncthreads();
-    constexpr int GPR = BN / 64, ITEMS = BM * GPR, TPI = 256 / ITEMS, VPT = 64 / TPI;
-    static_assert(ITEMS * TPI == 256 && VPT % 8 == 0, "gelu epilogue shape");
     if (worker) {
-      const int item = tid / TPI, sub = tid % TPI;
-      const int rl = item / GPR, grp = item % GPR;
-      const int c0 = grp * 64 + sub * VPT;
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        T[(rb + (e >> 2) * 8 + (e & 3)) * LDT + wn * 32 + (lane & 31)] = gelu_tanh_exp(acc[e] + bias);
+    }
+    __syncthreads();
+    if (worker) {  // a quad of threads a row, 16 columns each
+      constexpr int VPT = 16;
+      const int rl = tid >> 2, c0 = (tid & 3) * VPT;
       const int m = m0 + rl, n = n0 + c0;
       float sum = 0.0f;
       const bool live = m < M && n < N;
@@ -528,91 +413,66 @@ __global__ __launch_bounds__(PROD ? 512 : 256, (PROD && TM == 1) ? 4 : 1) void g
           gstore(reinterpret_cast<uint4 *>(a.xo.lo + (size_t)m * N + n + c), make_uint4(lw[0], lw[1], lw[2], lw[3]));
         }
       }
-      sum = item_sum<TPI>(sum);
-      if (live && sub == 0) gstore(a.xo.gs + (size_t)m * (N / kGroup) + n / kGroup, sum);
+      sum = quad_sum(sum);
+      if (live && (tid & 3) == 0) gstore(a.xo.gs + (size_t)m * (N / kGroup) + n / kGroup, sum);
     }
     return;
-  } else if (worker) {
+  } else if (worker && nc < N) {
+    const int n = nc;
+    // The values first, in straight-line code (the waits on its loads come
+    // here, once), then the stores, each predicated on its row: behind a predicate the
+    // compiler's wait counting waits for every access in flight, earlier stores too.
+    float outv[16];
 #pragma unroll
-    for (int i2 = 0; i2 < TM; i2++)
+    for (int e = 0; e < 16; e++) {
+      float v = acc[e] + bias;
+      if constexpr (kResid) v = yv[e] + v;
+      outv[e] = v;
+    }
+    // (an empty asm over the values keeps the compiler from sinking their arithmetic,
+    // and the waits on its operands, into the predicated stores)
 #pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int n = n0 + wn * 32 * TN + j * 32 + (lane & 31);
-        if (n >= N) continue;
-        const float bias = kColEarly ? cb : a.ql.bias[n];
-        const int rb = wm * 32 * TM + i2 * 32 + (lane >> 5) * 4;  // tile row of element 0
-        // 128-row tiles: the sub-tile's 16 old values loaded together (registers for all 64
-        // of the lane's would spill)
-        float ysub[kResid && TM != 1 ? 16 : 1];
-        if constexpr (kResid && TM != 1) {
+    for (int e = 0; e < 16; e++) asm volatile("" : "+v"(outv[e]));
+    // stores through the global address space (generic stores also count against the
+    // LDS counter)
+    if constexpr (EPI == kEpiStore || EPI == kEpiResid) {
 #pragma unroll
-          for (int e = 0; e < 16; e++)
-            ysub[e] = gload(a.y + (size_t)min(m0 + rb + (e >> 2) * 8 + (e & 3), M - 1) * N + n);
-        }
-        // The sub-tile's values first, in straight-line code (the waits on its loads come
-        // here, once), then the stores, each predicated on its row: behind a predicate the
-        // compiler's wait counting waits for every access in flight, earlier stores too.
-        float outv[16];
+      for (int e = 0; e < 16; e++) {
+        const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
+        if (m < M) gstore(a.y + (size_t)m * N + n, outv[e]);
+      }
+    } else {
+      const int d = a.qkv.d_model;
+      if (n < d) {
 #pragma unroll
         for (int e = 0; e < 16; e++) {
-          float v = acc[i2][j][e] + bias;
-          if constexpr (kResid) v = (TM == 1 ? yv[i2][j][e] : ysub[e]) + v;
-          outv[e] = v;
+          const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
+          if (m < M) gstore(a.qkv.q_out + (size_t)m * d + n, outv[e]);
         }
-        // (an empty asm over the values keeps the compiler from sinking their arithmetic,
-        // and the waits on its operands, into the predicated stores)
-#pragma unroll
-        for (int e = 0; e < 16; e++) asm volatile("" : "+v"(outv[e]));
-        // stores through the global address space (generic stores also count against the
-        // LDS counter)
-        if constexpr (EPI == kEpiStore || EPI == kEpiResid) {
-#pragma unroll
-          for (int e = 0; e < 16; e++) {
-            const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
-            if (m < M) gstore(a.y + (size_t)m * N + n, outv[e]);
-          }
-        } else {
-          const int d = a.qkv.d_model;
-          if (n < d) {
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
-              if (m < M) gstore(a.qkv.q_out + (size_t)m * d + n, outv[e]);
-            }
+      } else {
+        const bool is_k = n < 2 * d;
+        const int idx = is_k ? n - d : n - 2 * d;
+        const int h = idx >> 6, e2 = idx & 63;
+        auto put = [&](void *cache, int pos, float v) __attribute__((always_inline)) {
+          const size_t ci = ((size_t)h * a.qkv.max_seq + pos) * kHeadDim + e2;
+          if constexpr (KVT == kKvBf16) {
+            gstore(static_cast<uint16_t *>(cache) + ci, (uint16_t)float_to_bf16_bits(v));
           } else {
-            const bool is_k = n < 2 * d;
-            const int idx = is_k ? n - d : n - 2 * d;
-            const int h = idx >> 6, e2 = idx & 63;
-            auto put = [&](void *cache, int pos, float v) __attribute__((always_inline)) {
-              const size_t ci = ((size_t)h * a.qkv.max_seq + pos) * kHeadDim + e2;
-              if constexpr (KVT == kKvBf16) {
-                gstore(static_cast<uint16_t *>(cache) + ci, (uint16_t)float_to_bf16_bits(v));
-              } else {
-                gstore(static_cast<float *>(cache) + ci, v);
-              }
-            };
-            if (!a.qkv.seqs) {
-              void *cache = is_k ? a.qkv.k_cache : a.qkv.v_cache;
-#pragma unroll
-              for (int e = 0; e < 16; e++) {
-                const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
-                if (m < M) put(cache, a.qkv.pos0 + m, outv[e]);
-              }
-            } else {  // batched decode: row m is sequence m
-#pragma unroll
-              for (int e = 0; e < 16; e++) {
-                const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
-                if (m >= M) continue;
-                const BatchSeq *sq = a.qkv.seqs + m;
-                DecodeCtl *ctl = gload(&sq->ctl);
-                if (gload<int32_t>(&ctl->done)) continue;
-                put(static_cast<char *>(gload(is_k ? &sq->k : &sq->v)) + a.qkv.layer_off * (KVT == kKvBf16 ? 2 : 4),
-                    gload<int32_t>(&ctl->valid_len), outv[e]);
-              }
-            }
+            gstore(static_cast<float *>(cache) + ci, v);
           }
+        };
+#pragma unroll
+        for (int e = 0; e < 16; e++) {  // row m is sequence m
+          const int m = m0 + rb + (e >> 2) * 8 + (e & 3);
+          if (m >= M) continue;
+          const BatchSeq *sq = a.qkv.seqs + m;
+          DecodeCtl *ctl = gload(&sq->ctl);
+          if (gload<int32_t>(&ctl->done)) continue;
+          put(static_cast<char *>(gload(is_k ? &sq->k : &sq->v)) + a.qkv.layer_off * (KVT == kKvBf16 ? 2 : 4),
+              gload<int32_t>(&ctl->valid_len), outv[e]);
         }
       }
+    }
   }
 }
 
@@ -665,8 +525,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN,
     ep_b[q] = FOLD ? a.fold.c[n] : a.ql.bias[n];
     ep_g[q] = FOLD ? a.fold.G[n] : 0.0f;
     ep_y[q] = EPI == kEpiResid && m < M ? a.y[(size_t)m * N + n] : 0.0f;
-    if constexpr (EPI == kEpiQKV)
-      if (a.qkv.seqs) ep_sq[q] = a.qkv.seqs[min(m, M - 1)];
+    if constexpr (EPI == kEpiQKV) ep_sq[q] = a.qkv.seqs[min(m, M - 1)];
   }
   // this wave's groups: ks * 4 gw + 4 i + wave, i < gw (none past G)
   floatx4 acc[2] = {floatx4{0.0f, 0.0f, 0.0f, 0.0f}, floatx4{0.0f, 0.0f, 0.0f, 0.0f}};
@@ -821,17 +680,16 @@ __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN,
       for (int e = 0; e < 4; e++) acc[j][e] = fmaf(sb.x, P[j][e], fmaf(sb.y, gsr[gi][e], acc[j][e]));
     }
   }
-  // a batched QKV row's cache position and state (the sequence's control block)
+  // a QKV row's cache position and state (the sequence's control block)
   int ep_pos[kFewEPT], ep_done[kFewEPT];
 #pragma unroll
   for (int q = 0; q < kFewEPT; q++) {
     ep_pos[q] = 0;
     ep_done[q] = 0;
-    if constexpr (EPI == kEpiQKV)
-      if (a.qkv.seqs) {
-        ep_pos[q] = ep_sq[q].ctl->valid_len;
-        ep_done[q] = ep_sq[q].ctl->done;
-      }
+    if constexpr (EPI == kEpiQKV) {
+      ep_pos[q] = ep_sq[q].ctl->valid_len;
+      ep_done[q] = ep_sq[q].ctl->done;
+    }
   }
   if constexpr (FOLD) {
     {  // rows past M have zero statistics' inputs (mean 0); their results are not stored
@@ -943,15 +801,10 @@ __global__ __launch_bounds__(64 * kFewWaves) void few_kernel(GemmArgs a, int nN,
         } else {
           const int idx = n < 2 * d ? n - d : n - 2 * d;
           const int hh = idx >> 6, e2 = idx & 63;
-          void *cache = n < 2 * d ? a.qkv.k_cache : a.qkv.v_cache;
-          int pos = a.qkv.pos0 + m;
-          if (a.qkv.seqs) {  // batched decode: row m is sequence m
-            if (ep_done[q]) continue;
-            pos = ep_pos[q];
-            cache = static_cast<char *>(n < 2 * d ? ep_sq[q].k : ep_sq[q].v) +
-                    a.qkv.layer_off * (KVT == kKvBf16 ? 2 : 4);
-          }
-          const size_t ci = ((size_t)hh * a.qkv.max_seq + pos) * kHeadDim + e2;
+          if (ep_done[q]) continue;  // row m is sequence m
+          void *cache = static_cast<char *>(n < 2 * d ? ep_sq[q].k : ep_sq[q].v) +
+                        a.qkv.layer_off * (KVT == kKvBf16 ? 2 : 4);
+          const size_t ci = ((size_t)hh * a.qkv.max_seq + ep_pos[q]) * kHeadDim + e2;
           if constexpr (KVT == kKvBf16) {
             static_cast<uint16_t *>(cache)[ci] = (uint16_t)float_to_bf16_bits(val);
           } else {
@@ -1004,24 +857,22 @@ constexpr int kStages = 3;
 
 struct Plan {
   int mode, nN, mt, S, gps, blocks;
-  size_t lds;
 };
 
-template <int BITS, int PT, int TM, int TN>
+template <int BITS, int PT>
 constexpr size_t lds_bytes() {
-  return (size_t)kStages * Shape<BITS, PT, TM, TN>::STAGE;
+  return (size_t)kStages * Shape<BITS, PT>::STAGE;
 }
 
-Plan make_plan(const GemmArgs &a, int bits, int ptype) {
+Plan make_plan(const GemmArgs &a) {
   Plan p{};
-  const int BM = 64, BN = 64;
-  const int G = a.ql.K / kGroup;
+    const int G = a.ql.K / kGroup;
   p.nN = (a.ql.N + BN - 1) / BN;
   p.mt = (a.M + BM - 1) / BM;
   const int tiles = p.nN * p.mt;
   const int slots = std::max(1, a.n_cu) * 2;
   // Split count with the lowest modelled time; partial tiles must fit the workspace.
-  // Small tiles (copier waves, two blocks per CU), in microseconds, fitted to MI355X timings
+  // In microseconds, fitted to MI355X timings
   // of the decoder's four GEMM shapes at 8, 99, 163 and 235 rows: ~0.95 us per split (the
   // last block of a tile adds every partial), and per K group of a block ~0.42 us while the
   // blocks fit one per CU, rising with the blocks per CU.
@@ -1044,23 +895,20 @@ Plan make_plan(const GemmArgs &a, int bits, int ptype) {
   p.gps = (G + p.S - 1) / p.S;
   p.mode = p.mt <= 4 ? 1 : 0;
   p.blocks = p.mode == 1 ? ((p.nN * p.S + 7) / 8) * 8 * p.mt : tiles * p.S;
-  (void)bits;
-  (void)ptype;
   return p;
 }
 
-template <int BITS, int PT, int EPI, int KVT, int TM, int TN>
-hipError_t set_cfg_attr() {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kernel<BITS, PT, EPI, KVT, TM, TN, kStages, true>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes<BITS, PT, TM, TN>());
+template <int BITS, int PT, int EPI, int KVT>
+hipError_t set_attr() {
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kernel<BITS, PT, EPI, KVT, kStages>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes<BITS, PT>());
 }
 
-template <int BITS, int PT, int EPI, int KVT, int TM, int TN>
-hipError_t launch_cfg(const GemmArgs &a, const Plan &p, hipStream_t s) {
-  constexpr bool prod = true;
-  auto *fn = gemm_kernel<BITS, PT, EPI, KVT, TM, TN, kStages, prod>;
-  constexpr size_t lds = lds_bytes<BITS, PT, TM, TN>();
-  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(prod ? 512 : 256), lds, s, a, p.mode, p.nN, p.mt, p.S, p.gps);
+template <int BITS, int PT, int EPI, int KVT>
+hipError_t launch_epi(const GemmArgs &a, const Plan &p, hipStream_t s) {
+  auto *fn = gemm_kernel<BITS, PT, EPI, KVT, kStages>;
+  constexpr size_t lds = lds_bytes<BITS, PT>();
+  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(512), lds, s, a, p.mode, p.nN, p.mt, p.S, p.gps);
   return hipGetLastError();
 }
 
@@ -1070,17 +918,12 @@ hipError_t init_bits() {
   auto chk = [&](hipError_t x) {
     if (e == hipSuccess) e = x;
   };
-  chk(set_cfg_attr<BITS, PT, kEpiStore, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiResid, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiGelu, 0, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvBf16, 1, 1>());
-  chk(set_cfg_attr<BITS, PT, kEpiQKV, kKvF32, 1, 1>());
+  chk(set_attr<BITS, PT, kEpiStore, 0>());
+  chk(set_attr<BITS, PT, kEpiResid, 0>());
+  chk(set_attr<BITS, PT, kEpiGelu, 0>());
+  chk(set_attr<BITS, PT, kEpiQKV, kKvBf16>());
+  chk(set_attr<BITS, PT, kEpiQKV, kKvF32>());
   return e;
-}
-
-template <int BITS, int PT, int EPI, int KVT>
-hipError_t launch_epi(const GemmArgs &a, const Plan &p, hipStream_t s) {
-  return launch_cfg<BITS, PT, EPI, KVT, 1, 1>(a, p, s);
 }
 
 template <int BITS, int PT>
@@ -1147,6 +990,7 @@ size_t gemm_ws_floats(int n_cu) {
 hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt, hipStream_t s) {
   if (a.ql.K % kGroup != 0 || a.M <= 0 || a.ql.N <= 0) return hipErrorInvalidValue;
   if (epi == kEpiGelu && a.ql.N % kGroup != 0) return hipErrorInvalidValue;
+  if (epi == kEpiQKV && !a.qkv.seqs) return hipErrorInvalidValue;
   if (a.fold.x) {  // the folded LayerNorm: few-row products with one group a wave only
     if (a.M > kFewRows || !a.fcodes || (bits != 8 && bits != 4) || a.ql.K % 256 != 0 || a.ql.K > 256 * kFoldQ ||
         (epi != kEpiQKV && epi != kEpiGelu) || !a.fold.gamma || !a.fold.G || !a.fold.c)
@@ -1168,7 +1012,7 @@ hipError_t launch_gemm(const GemmArgs &a, int bits, int ptype, int epi, int kvt,
                                 : few_dispatch<4, kParamF32>(a, nN, S, gw, epi, kvt, s);
     }
   }
-  const Plan p = make_plan(a, bits, ptype);
+  const Plan p = make_plan(a);
   if (p.S > 1 && (a.ws == nullptr || a.cnt == nullptr)) return hipErrorInvalidValue;
   if (bits == 8) {
     return ptype == kParamF16 ? gemm_dispatch<8, kParamF16>(a, p, epi, kvt, s)
