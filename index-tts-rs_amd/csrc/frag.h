@@ -11,6 +11,8 @@
 // end), or bf16 triples, which hold an fp32 value's 24 bits over its whole range.
 #pragma once
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace itts {
@@ -86,6 +88,74 @@ __device__ __forceinline__ floatx16 mma_planes(const u32x4 (&a)[NA], const u32x4
 __device__ __forceinline__ float other_half(float v, int lane) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(lane < 32 ? r[1] : r[0]);
+}
+
+// ---- a product block's partial tiles ------------------------------------------------------
+// Row parts (of 8 = rows x columns) the XCDs divide the tile grid into: the split whose XCDs
+// read the fewest operand bytes.  A part whose operands fit its L2 reads them once; a larger
+// one reads, for every ~64 tiles in flight, the row tiles and the column tiles they span.
+// (4650 x 1024 x 2560: 78 us at 2 x 4, 84 at 8 x 1; 2066 x 512 x 512: 10.6 at 4 x 2, 12.6 at
+// 1 x 8, which the plain tile order amounts to.)
+inline int xcd_rows(int nM, int nN, double a_tile, double w_tile) {
+  int best = 1;
+  double least = 1e300;
+  for (int gm = 1; gm <= 8; gm *= 2) {
+    const int gn = 8 / gm, pm = (nM + gm - 1) / gm, pn = (nN + gn - 1) / gn;
+    double bytes = pm * a_tile + pn * w_tile;
+    if (bytes > 3e6)
+      bytes = std::max(bytes, pm * pn / 64.0 * (std::max(1.0, 64.0 / pn) * a_tile + std::min(pn, 64) * w_tile));
+    if (bytes < least) least = bytes, best = gm;
+  }
+  return best;
+}
+
+// The TM x TN MFMA tiles of wave kq of KS that split K go to LDS (red: KL tiles of BM rows, LD
+// floats apart): with KS > KL the upper half of the waves first, then the lower half adds its own
+// to what it finds, so that half the tiles' LDS does.  h = lane >> 5, r31 = lane & 31.
+template <int TM, int TN, int KS, int KL, int BM, int LD>
+__device__ __forceinline__ void parts_to_lds(float *red, const floatx16 (&acc)[TM][TN], int kq, int h, int r31) {
+  auto part = [&](int k) __attribute__((always_inline)) { return red + (size_t)k * BM * LD; };
+  auto place = [&](int i, int j, int e) __attribute__((always_inline)) {
+    return (i * 32 + (e >> 2) * 8 + h * 4 + (e & 3)) * LD + j * 32 + r31;
+  };
+  if constexpr (KS > KL) {
+    if (kq >= KL) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) part(kq - KL)[place(i, j, e)] = acc[i][j][e];
+    }
+    __syncthreads();
+  }
+  if (kq < KL) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          float *t = part(kq) + place(i, j, e);
+          *t = KS > KL ? acc[i][j][e] + *t : acc[i][j][e];
+        }
+  }
+  __syncthreads();
+}
+
+// Eight columns of a tile row, the parts added in order.
+template <int KL, int BM, int LD>
+__device__ __forceinline__ void parts_row8(const float *red, int row, int col, float v[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    float4 s = *reinterpret_cast<const float4 *>(red + (size_t)row * LD + col + 4 * q);
+#pragma unroll
+    for (int k = 1; k < KL; k++) {
+      const float4 p = *reinterpret_cast<const float4 *>(red + ((size_t)k * BM + row) * LD + col + 4 * q);
+      s.x += p.x, s.y += p.y, s.z += p.z, s.w += p.w;
+    }
+    v[4 * q] = s.x, v[4 * q + 1] = s.y, v[4 * q + 2] = s.z, v[4 * q + 3] = s.w;
+  }
 }
 
 // ---- attention over key tiles of 32, one wave for 32 queries ----------------------------

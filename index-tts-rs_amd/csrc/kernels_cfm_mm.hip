@@ -7,8 +7,6 @@
 // into registers.  The epilogues stage the fp32 tile in LDS and write whole pieces: bias and
 // residual, the SwiGLU, WaveNet's gate and residual / skip sums, and the attention's operands
 // with rope applied.
-#include <algorithm>
-
 #include "frag.h"
 #include "kernels.h"
 
@@ -154,16 +152,17 @@ __global__ __launch_bounds__(64) void norm_frag_kernel(const float *x, int R, in
 
 // ---- the product ------------------------------------------------------------------------
 // A wave forms a (32 TM) x (32 TN) tile, three products each MFMA tile, from fragments loaded
-// AH K steps ahead of their use.  Block: WM x WN wave tiles, each by KS waves that take a part
-// of K (their partial tiles added in wave order).  The fp32 tile goes through LDS; a thread
+// AH K steps ahead of their use.  Block: one such tile by KS waves that take a part of K (their
+// partial tiles added in wave order).  The fp32 tile goes through LDS; a thread
 // then takes (row, 8 columns) items.
-template <int TM_, int TN_, int WM_, int WN_, int KS_, int AH_>
+template <int TM_, int TN_, int KS_, int AH_>
 struct MmCfg {
-  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, KS = KS_, AH = AH_;
-  static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, LD = BN + 4, NT = 64 * WM * WN * KS;
+  static constexpr int TM = TM_, TN = TN_, KS = KS_, AH = AH_;
+  static constexpr int BM = 32 * TM, BN = 32 * TN, LD = BN + 4, NT = 64 * KS;
   static constexpr int KL = KS > 2 ? KS / 2 : KS;  // partial tiles held in LDS
   static constexpr size_t LDS = sizeof(float) * KL * BM * LD;
   static_assert(BN % 64 == 0, "column groups of 64");
+  static_assert(128 % BN == 0 && 128 % BM == 0, "whole tiles in the planes' 128-row blocks");
 };
 
 template <class C, int EPI>
@@ -171,8 +170,7 @@ __global__ __launch_bounds__(C::NT, 2) void mm_kernel(CfmMm a) {
   constexpr int TM = C::TM, TN = C::TN, KS = C::KS, BM = C::BM, BN = C::BN, LD = C::LD, NT = C::NT, AH = C::AH;
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r31 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kq = wave % KS, wn = wave / KS % C::WN, wm = wave / (KS * C::WN);
+  const int kq = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Block -> tile.  Blocks go to the 8 XCDs round-robin, and each XCD reads what its tiles need
   // through its own L2: XCD x takes every gm-th row tile from x % gm and every gn-th column
   // tile from x / gm, so that the operands cross the fabric gn and gm times, not 8 times each.
@@ -186,10 +184,10 @@ __global__ __launch_bounds__(C::NT, 2) void mm_kernel(CfmMm a) {
   const u32x4 *wp[TN], *ap[TM], *ap2[TM];
 #pragma unroll
   for (int i = 0; i < TN; i++)
-    wp[i] = reinterpret_cast<const u32x4 *>(a.w) + ((size_t)((n0 >> 5) + wn * TN + i) * a.nk) * 128 + lane;
+    wp[i] = reinterpret_cast<const u32x4 *>(a.w) + ((size_t)((n0 >> 5) + i) * a.nk) * 128 + lane;
 #pragma unroll
   for (int i = 0; i < TM; i++) {
-    const int row = z * a.zr + m0 + (wm * TM + i) * 32 + r31, rp = h * 32 + (row & 31);
+    const int row = z * a.zr + m0 + i * 32 + r31, rp = h * 32 + (row & 31);
     ap[i] = reinterpret_cast<const u32x4 *>(a.a) + z * a.sa + ((size_t)(row >> 5) * a.kt_a) * 128 + rp;
     ap2[i] = a.a2 ? reinterpret_cast<const u32x4 *>(a.a2) + ((size_t)(row >> 5) * a.kt_a2) * 128 + rp : ap[i];
   }
@@ -203,7 +201,7 @@ __global__ __launch_bounds__(C::NT, 2) void mm_kernel(CfmMm a) {
       const u32x4 *p;
       if constexpr (EPI == kMmGate || EPI == kMmConv) {  // a convolution's taps: tap j reads row m + j of a padded operand
         const int tap = kc / a.taps_kt, ktd = kc - tap * a.taps_kt;
-        const int row = m0 + (wm * TM + i) * 32 + r31 + tap;
+        const int row = m0 + i * 32 + r31 + tap;
         p = reinterpret_cast<const u32x4 *>(a.a) + z * a.sa + ((size_t)(row >> 5) * a.kt_a + ktd) * 128 + h * 32 +
             (row & 31);
       } else {
@@ -280,47 +278,11 @@ __global__ __launch_bounds__(C::NT, 2) void mm_kernel(CfmMm a) {
       if (kt + s < k1) mma(f[s]);
   }
 
-  // the tile to LDS: with four parts of K the upper two add theirs to the lower two's first, so
-  // that two tiles of LDS do (four blocks of 64 x 64 to a compute unit, not two)
-  auto part = [&](int k) __attribute__((always_inline)) { return red + (size_t)k * BM * LD; };
-  auto place = [&](int i, int j, int e) __attribute__((always_inline)) {
-    return ((wm * TM + i) * 32 + (e >> 2) * 8 + h * 4 + (e & 3)) * LD + (wn * TN + j) * 32 + r31;
-  };
+  // (with four parts of K two tiles of LDS do: four blocks of 64 x 64 to a compute unit, not two)
   constexpr int KL = C::KL;
-  if constexpr (KS > KL) {
-    if (kq >= KL) {
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-          for (int e = 0; e < 16; e++) part(kq - KL)[place(i, j, e)] = acc[i][j][e];
-    }
-    __syncthreads();
-  }
-  if (kq < KL) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-          float *t = part(kq) + place(i, j, e);
-          *t = KS > KL ? acc[i][j][e] + *t : acc[i][j][e];
-        }
-  }
-  __syncthreads();
+  parts_to_lds<TM, TN, KS, KL, BM, LD>(red, acc, kq, h, r31);
   auto tile8 = [&](int row, int col, float v[8]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      float4 s = *reinterpret_cast<const float4 *>(red + (size_t)row * LD + col + 4 * q);
-#pragma unroll
-      for (int k = 1; k < KL; k++) {
-        const float4 p = *reinterpret_cast<const float4 *>(red + ((size_t)k * BM + row) * LD + col + 4 * q);
-        s.x += p.x, s.y += p.y, s.z += p.z, s.w += p.w;
-      }
-      v[4 * q] = s.x, v[4 * q + 1] = s.y, v[4 * q + 2] = s.z, v[4 * q + 3] = s.w;
-    }
+    parts_row8<KL, BM, LD>(red, row, col, v);
   };
   auto add8 = [&](const float *p, float v[8]) __attribute__((always_inline)) {
     const float4 x = *reinterpret_cast<const float4 *>(p), y = *reinterpret_cast<const float4 *>(p + 4);
@@ -613,23 +575,6 @@ int mm_cols(const CfmMm &a) {  // columns of the product (interleaved halves cou
   return EPI == kMmSwiglu || EPI == kMmGate ? (a.N + 31) / 32 * 64 : a.N;
 }
 
-// Row parts (of 8 = rows x columns) the XCDs divide the tile grid into: the split whose XCDs
-// read the fewest operand bytes.  A part whose operands fit its L2 reads them once; a larger
-// one reads, for every ~64 tiles in flight, the row tiles and the column tiles they span.
-// (4650 x 1024 x 2560: 78 us at 2 x 4, 84 at 8 x 1; 2066 x 512 x 512: 10.6 at 4 x 2, 12.6 at
-// 1 x 8, which the plain tile order amounts to.)
-int xcd_rows(int nM, int nN, double a_tile, double w_tile) {
-  int best = 1;
-  double least = 1e300;
-  for (int gm = 1; gm <= 8; gm *= 2) {
-    const int gn = 8 / gm, pm = (nM + gm - 1) / gm, pn = (nN + gn - 1) / gn;
-    double bytes = pm * a_tile + pn * w_tile;
-    if (bytes > 3e6) bytes = std::max(bytes, pm * pn / 64.0 * (std::max(1.0, 64.0 / pn) * a_tile + std::min(pn, 64) * w_tile));
-    if (bytes < least) least = bytes, best = gm;
-  }
-  return best;
-}
-
 template <class C, int EPI>
 hipError_t mm_run(CfmMm a, int batch, hipStream_t s) {
   a.nM = (a.M + C::BM - 1) / C::BM;
@@ -654,9 +599,9 @@ hipError_t mm_set() {
 // 6.8 / 5.1 / 4.9, 2066 x 512 x 512 10.0 / 8.8 / 9.9, 2066 x 512 x 1536 20.0 / 19.8 / 21.8, 2066 x
 // 1536 x 512 17.5 / 19.2 / 19.5, 2066 x 3072 x 512 29.2 / 32.9 / 33.8, 4650 x 1024 x 2560 78.7
 // (310 TFLOP/s, 930 of fp16 products) / 100 / 106; 128-row and 128-column tiles lose throughout.
-using MmLarge = MmCfg<2, 2, 1, 1, 4, 2>;
-using MmSmall2 = MmCfg<1, 2, 1, 1, 2, 4>;
-using MmSmall4 = MmCfg<1, 2, 1, 1, 4, 4>;
+using MmLarge = MmCfg<2, 2, 4, 2>;
+using MmSmall2 = MmCfg<1, 2, 2, 4>;
+using MmSmall4 = MmCfg<1, 2, 4, 4>;
 
 template <int EPI>
 hipError_t mm_attr() {

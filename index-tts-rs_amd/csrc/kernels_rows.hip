@@ -20,8 +20,6 @@
 #include "frag.h"
 #include "kernels.h"
 
-#include <algorithm>
-
 namespace itts {
 
 namespace {
@@ -213,12 +211,12 @@ __global__ __launch_bounds__(256) void rows_codes_kernel(const uint8_t *codes, i
 
 // ---- the product ------------------------------------------------------------------------
 // Block: one tile of BM = 32 TM rows x 64 columns by KS waves that split the K groups, their
-// partial tiles added through LDS (two halves of the waves at a time).  A wave keeps CH
-// groups of activation fragments, codes and scales in flight.
+// partial tiles added through LDS (two halves of the waves at a time).  A wave keeps a
+// group of activation fragments, codes and scales in flight.
 constexpr int kMaxSplit = 6;  // blocks that may share a tile's K
-template <int TM_, int KS_, int CH_>
+template <int TM_, int KS_>
 struct RmCfg {
-  static constexpr int TM = TM_, TN = 2, KS = KS_, CH = CH_;
+  static constexpr int TM = TM_, TN = 2, KS = KS_;
   static constexpr int BM = 32 * TM, BN = 64, LD = BN + 4, NT = 64 * KS, KL = KS > 2 ? KS / 2 : KS;
   static constexpr size_t LDS = sizeof(float) * (KL * BM * LD + 2 * BM);
   static_assert(LDS <= 65536, "dynamic LDS of a plain launch");
@@ -268,7 +266,7 @@ struct AttnPlanes<kRowsPairs> {
 template <int BITS, int EPI, int KVT, class C>
 __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(RowsMm a) {
   constexpr int TM = C::TM, TN = C::TN, KS = C::KS, KL = C::KL, BM = C::BM, BN = C::BN, LD = C::LD, NT = C::NT;
-  constexpr int CH = C::CH, CW = BITS == 8 ? 4 : 2;  // words of a lane's codes per 32 K values
+  constexpr int CW = BITS == 8 ? 4 : 2;  // words of a lane's codes per 32 K values
   extern __shared__ __attribute__((aligned(16))) float red[];
   float2 *row_stat = reinterpret_cast<float2 *>(red + KL * BM * LD);
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r31 = lane & 31;
@@ -299,8 +297,8 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
     uint32_t q[TN][2][CW];
     float s[TN];
   };
-  u32x4 fa[CH][4][TM][2];
-  Codes cq[CH];
+  u32x4 fa[4][TM][2];
+  Codes cq;
   auto load_a = [&](int g, int s4, u32x4(&f)[TM][2]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -329,15 +327,12 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       c.s[j] = (a.scale + (size_t)gc * a.ldn + n0 + j * 32)[r31];
     }
   };
-  auto load_rings = [&]() __attribute__((always_inline)) {
+  auto load_group = [&](int g) __attribute__((always_inline)) {
+    load_c(g, cq);
 #pragma unroll
-    for (int u = 0; u < CH; u++) {
-      load_c(g0 + u, cq[u]);
-#pragma unroll
-      for (int s4 = 0; s4 < 4; s4++) load_a(g0 + u, s4, fa[u][s4]);
-    }
+    for (int s4 = 0; s4 < 4; s4++) load_a(g, s4, fa[s4]);
   };
-  // the bias term's steps first (their loads go out ahead of the rings')
+  // the bias term's steps first (their loads go out ahead of the first group's)
   const int x0 = nx * kk / KT, x1 = nx * (kk + 1) / KT;
   for (int kx = x0; kx < x1; kx++) {
     u32x4 xa[TM][3], xb[TN][3];
@@ -354,7 +349,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       for (int q = 0; q < 3; q++) xb[j][q] = p[lane + 64 * q];
     }
     if (kx == x0 && g0 < g1) {
-      load_rings();
+      load_group(g0);
     }
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -362,7 +357,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       for (int j = 0; j < TN; j++) acc[i][j] = mma_planes<Bf16Triples, 3>(xa[i], xb[j], acc[i][j]);
   }
   if (x0 == x1 && g0 < g1) {
-    load_rings();
+    load_group(g0);
   }
   // What the epilogue needs, loaded here so that its latency passes under the K loop.  A
   // thread's items are the tile's rows tid / 8 + i NT / 8 at columns 8 (tid & 7) .. +7.
@@ -398,7 +393,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       old[i][1] = o[1];
     }
   }
-  auto group = [&](int g, u32x4(&f)[4][TM][2], Codes &c) __attribute__((always_inline)) {
+  auto group = [&](int g) __attribute__((always_inline)) {
     floatx16 P[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -411,7 +406,7 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       f16x8 b[TN];
 #pragma unroll
       for (int j = 0; j < TN; j++) {
-        const uint32_t *q = c.q[j][s4 >> 1];
+        const uint32_t *q = cq.q[j][s4 >> 1];
         b[j] = BITS == 8 ? codes_f16<BITS>(q[(s4 & 1) * 2], q[(s4 & 1) * 2 + (BITS == 8 ? 1 : 0)])
                          : codes_f16<BITS>(q[s4 & 1], 0);
       }
@@ -420,27 +415,20 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-          for (int j = 0; j < TN; j++) P[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, f[s4][i][p]), b[j], P[i][j], 0, 0, 0);
-      load_a(g + CH, s4, f[s4]);
+          for (int j = 0; j < TN; j++) P[i][j] = ITTS_MFMA16(__builtin_bit_cast(f16x8, fa[s4][i][p]), b[j], P[i][j], 0, 0, 0);
+      load_a(g + 1, s4, fa[s4]);
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      const float s = c.s[j];
+      const float s = cq.s[j];
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(s, P[i][j][e], acc[i][j][e]);
     }
-    load_c(g + CH, c);
+    load_c(g + 1, cq);
   };
-  int g = g0;
-  for (; g + CH <= g1; g += CH) {
-#pragma unroll
-    for (int u = 0; u < CH; u++) group(g + u, fa[u], cq[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < CH - 1; u++)
-    if (g + u < g1) group(g + u, fa[u], cq[u]);
+  for (int g = g0; g < g1; g++) group(g);
 
   if constexpr (kFold) {
     if (fin) {
@@ -463,47 +451,11 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
       if (tid % LPR == 0) row_stat[tid / LPR] = make_float2(mean, 1.0f / sqrtf(m2 / (float)a.K + 1e-5f));
     }
   }
-  // the tile to LDS: the upper half of the waves adds its partials to the lower half's
-  auto part = [&](int k) __attribute__((always_inline)) { return red + (size_t)k * BM * LD; };
-  auto place = [&](int i, int j, int e) __attribute__((always_inline)) {
-    return (i * 32 + (e >> 2) * 8 + h * 4 + (e & 3)) * LD + j * 32 + r31;
-  };
-  if constexpr (KS > KL) {
-    if (kq >= KL) {
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-          for (int e = 0; e < 16; e++) part(kq - KL)[place(i, j, e)] = acc[i][j][e];
-    }
-    __syncthreads();
-  }
-  if (kq < KL) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-          float *t = part(kq) + place(i, j, e);
-          *t = KS > KL ? acc[i][j][e] + *t : acc[i][j][e];
-        }
-  }
-  __syncthreads();
+  parts_to_lds<TM, TN, KS, KL, BM, LD>(red, acc, kq, h, r31);
 
   // eight columns of a tile row: the parts added, then the folded LayerNorm or the bias
   auto tile8 = [&](int row, int col, float v[8]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      float4 s = *reinterpret_cast<const float4 *>(red + (size_t)row * LD + col + 4 * q);
-#pragma unroll
-      for (int k = 1; k < KL; k++) {
-        const float4 p = *reinterpret_cast<const float4 *>(red + ((size_t)k * BM + row) * LD + col + 4 * q);
-        s.x += p.x, s.y += p.y, s.z += p.z, s.w += p.w;
-      }
-      v[4 * q] = s.x, v[4 * q + 1] = s.y, v[4 * q + 2] = s.z, v[4 * q + 3] = s.w;
-    }
+    parts_row8<KL, BM, LD>(red, row, col, v);
     if constexpr (kFold) {
       if (fin) {
         const float2 rs = row_stat[row];
@@ -830,20 +782,6 @@ __global__ __launch_bounds__(256, 2) void rows_attn_kernel(const u32x4 *qf, cons
   if (lane < 32) put_group_sum(out, t, head, nk, rb, gs);
 }
 
-// (row parts of the XCDs: the split with the fewest operand bytes read by each)
-int xcd_rows(int nM, int nN, double a_tile, double w_tile) {
-  int best = 1;
-  double least = 1e300;
-  for (int gm = 1; gm <= 8; gm *= 2) {
-    const int gn = 8 / gm, pm = (nM + gm - 1) / gm, pn = (nN + gn - 1) / gn;
-    double bytes = pm * a_tile + pn * w_tile;
-    if (bytes > 3e6)
-      bytes = std::max(bytes, pm * pn / 64.0 * (std::max(1.0, 64.0 / pn) * a_tile + std::min(pn, 64) * w_tile));
-    if (bytes < least) least = bytes, best = gm;
-  }
-  return best;
-}
-
 template <int BITS, int EPI, int KVT, class C>
 hipError_t run(RowsMm a, hipStream_t s) {
   a.nM = (a.M + C::BM - 1) / C::BM;
@@ -863,8 +801,8 @@ hipError_t run(RowsMm a, hipStream_t s) {
 // 5120 69.7 / 62.5 (459 TFLOP/s, 918 of fp16 products); 64 x 64 at K = 1280 too made prefills of 547
 // and 886 rows 2660 -> 2730 and 3590 -> 3735 us.  (Two groups in flight instead of one
 // gain nothing, eight waves on a tile lose wherever K is not split instead.)
-using RmSmall = RmCfg<1, 4, 1>;
-using RmLarge = RmCfg<2, 4, 1>;
+using RmSmall = RmCfg<1, 4>;
+using RmLarge = RmCfg<2, 4>;
 
 template <int BITS, int EPI, int KVT>
 hipError_t pick(RowsMm a, hipStream_t s) {
