@@ -65,9 +65,9 @@ def test_gemv_vs_fp64(gpt, bits, pd, N, K):
 
 
 # Shapes cover: the few-row kernel (M <= 8: one K split, several, a ragged last column
-# tile), the 64 x 64 tile with and without split-K, ragged N and M, the 128 x 128 tile
-# (M > 512) with and without split-K, the head's N = 8194, and the 4 x 547-row QKV product
-# (540 tiles, a ragged last M tile of 12 rows).
+# tile), the 64 x 64 LDS tile (up to 512 rows) with and without split-K, ragged N and M, the
+# products on fragment-order operands (M > 512), the head's N = 8194, and the 4 x 547-row QKV
+# product (a ragged last M tile).
 @pytest.mark.parametrize("bits,pd", [(8, H.ITTS_F16), (4, H.ITTS_F16), (8, H.ITTS_F32), (4, H.ITTS_F32)])
 @pytest.mark.parametrize("M,N,K", [(2, 37, 192), (8, 3840, 1280), (5, 1280, 5120), (7, 8194, 1280), (3, 96, 128),
                                    (99, 3840, 1280), (130, 1280, 5120), (64, 8194, 1280),
@@ -84,6 +84,20 @@ def test_mfma_gemm_vs_fp64(gpt, bits, pd, M, N, K):
     # split-K partials are added in split order: repeated calls are bit-identical
     again = gpt.qlinear_forward(q.codes, q.scales, q.biases, q.bias, x, N, K, bits, pd)
     assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+
+
+# The LDS tiles at the decoder's widths: K split over blocks for a batched step's rows (9-64), and
+# several row tiles.
+@pytest.mark.parametrize("bits,pd", [(8, H.ITTS_F16), (4, H.ITTS_F16), (8, H.ITTS_F32), (4, H.ITTS_F32)])
+@pytest.mark.parametrize("M,N,K", [(9, 1280, 1280), (10, 1280, 5120), (33, 3840, 1280), (63, 5120, 1280), (64, 1280, 5120),
+                                   (300, 1280, 5120)])
+def test_lds_tiles_vs_fp64(gpt, bits, pd, M, N, K):
+    say(f"[gpu] LDS tiles bits={bits} pd={pd} M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N + K)
+    q = _ql(rng, N, K, bits, pd)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = gpt.qlinear_forward(q.codes, q.scales, q.biases, q.bias, x, N, K, bits, pd)
+    _check_linear(got, q, bits, pd, x, 4e-6)  # (the bar above)
 
 
 def _logits_case(rng, n, kind):

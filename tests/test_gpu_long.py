@@ -283,7 +283,7 @@ def test_prefill_heavy_all_rows(full_model):
 
 def test_f32_group_params_full_size(full_f32_params):
     """The shipped checkpoint's dtype (F32 scales and biases, loader.rs:927-930) at the real
-    shape: a 535-row prefill (the 128 x 128 GEMM tiles), persistent decode steps, and a
+    shape: a 535-row prefill, persistent decode steps, and a
     long-context prefill_after with steps to 1734 keys, against the oracle."""
     W, g, M = full_f32_params
     say("[gpu] F32 group params, full size")
