@@ -73,14 +73,24 @@ struct Bf16Triples {
   static __device__ __forceinline__ void split(const float v[8], u32x4 (&p)[N]) { split8_bf16(v, p); }
 };
 // c + a b over operands of NA and T::N planes: the products of planes whose orders add up to
-// less than T::N (the others lie below the last plane's rounding).
+// less than T::N (the others lie below the last plane's rounding).  Of triples the small products
+// come first, so that a sum that starts at zero rounds them at their own magnitude.
 template <class T, int NA>
 __device__ __forceinline__ floatx16 mma_planes(const u32x4 (&a)[NA], const u32x4 (&b)[T::N], floatx16 c) {
+  auto mma = [&](int i, int j) __attribute__((always_inline)) {
+    c = T::mma(__builtin_bit_cast(typename T::V, a[i]), __builtin_bit_cast(typename T::V, b[j]), c);
+  };
+  if constexpr (T::N == 2) {
 #pragma unroll
-  for (int i = 0; i < NA; i++)
+    for (int i = 0; i < NA; i++)
 #pragma unroll
-    for (int j = 0; j < T::N - i; j++)
-      c = T::mma(__builtin_bit_cast(typename T::V, a[i]), __builtin_bit_cast(typename T::V, b[j]), c);
+      for (int j = 0; j < 2 - i; j++) mma(i, j);
+  } else {
+#pragma unroll
+    for (int o = T::N - 1; o >= 0; o--)
+#pragma unroll
+      for (int i = 0; i < NA && i <= o; i++) mma(i, o - i);
+  }
   return c;
 }
 
