@@ -72,6 +72,23 @@ def test_short_prompts_vs_fp64(T, bits, pd):
     assert rms(got) < 2 * rms(M.forward_rows(M.kv(128, kv_bf16=False), emb, 0)), rms(got)
 
 
+# either side of where fp32 rows' attention and the LayerNorms change their form
+@pytest.mark.parametrize("T", [384, 385, 512, 513])
+@pytest.mark.parametrize("kv", [H.ITTS_F32, H.ITTS_BF16])
+def test_prefill_route_edges(T, kv):
+    say(f"[gpu] rows prefill T={T} kv={kv}")
+    W, g, M = _model(8, H.ITTS_F32)
+    pr = synth.make_prompt(W.cfg, 3, 20, seed=T)
+    prior = (np.arange(T - 26, dtype=np.int32) * 13) % (W.cfg["mel_vocab"] - 2)
+    cache, okv = g.kv_cache(640, kv), M.kv(640, kv_bf16=kv == H.ITTS_BF16)
+    a = g.prefill_after(pr.text_tokens, pr.conds, pr.lang_id, prior, cache)
+    b = M.prefill_after(okv, pr.text_tokens, pr.conds, pr.lang_id, prior)
+    tol = 2e-5 if kv == H.ITTS_F32 else 2e-4  # (as in test_prefill_edges)
+    assert np.abs(a - b).max() < tol * max(1.0, np.abs(b).max())
+    s1, s2 = g.step(cache, 11, len(prior) + 2), M.step(okv, 11, len(prior) + 2)
+    assert np.abs(s1 - s2).max() < tol * max(1.0, np.abs(s2).max())
+
+
 def test_wide_model_without_folds():
     """d > 2048: the LayerNorms keep their row kernel."""
     over = (("n_layer", 2), ("d_model", 2112), ("n_head", 33), ("d_ffn", 128), ("text_vocab", 50), ("mel_vocab", 130))
