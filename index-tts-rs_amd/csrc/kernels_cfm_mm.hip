@@ -392,8 +392,9 @@ __global__ __launch_bounds__(C::NT, 2) void mm_kernel(CfmMm a) {
     }
   } else {
     // Q (rope, scaled by log2(e) / sqrt(64)) and K (rope) row fragments, V^T fragments with the
-    // attention's key order; a 64-column group is one head of one of q, k, v.  Rows past M (up
-    // to the tile of 64 keys) are zeros.
+    // attention's key order; a 64-column group is one head of one of q, k, v.  Rows past M are
+    // zeros to the end of the 32-row tile that holds row M - 1; a tile after it may stay unwritten
+    // (the attention's blocks of four query tiles load such a Q tile and drop what comes of it).
     const int d = a.N / 3, H = d / kHd, Tt = (a.M + 63) / 64 * 2;  // 32-key tiles
     const float2 *tab = reinterpret_cast<const float2 *>(a.g);
 #pragma unroll
@@ -505,9 +506,9 @@ __global__ __launch_bounds__(256) void qkv_frag_kernel(const float *qkv, const f
 }
 
 // ---- attention (cfm.rs:274-289): non-causal over T positions ----------------------------
-// Bound by the MFMA and VALU issue of its three fp16 products and exponentials: 22.8 us at
-// 2 x 1033 frames (575 TFLOP/s of fp16 products; 73 us before as LDS-staged tiles, a partial
-// buffer and a combine pass) and 81.7 us at 2 x 2325 (812; 224 us before).
+// Bound by the MFMA and VALU issue of its three fp16 products and exponentials: 24.2 us at
+// 2 x 1033 frames (541 TFLOP/s of fp16 products; 73 us before as LDS-staged tiles, a partial
+// buffer and a combine pass) and 81.4 us at 2 x 2325 (815; 224 us before).
 // Block: four waves, 32 WQ queries of one (batch, head), the key tiles split over WK = 4 / WQ
 // wave groups.  Output rows b T + t as fragment planes [B T][d].
 template <int WQ>

@@ -1,6 +1,6 @@
-// GEMM over row-major split activations for gfx950 (batched decode steps: 9 sequences and more on
-// the tiles, up to 8 on the few-row product), the activation splitter and the standalone
-// dequantiser.
+// GEMM over row-major split activations for gfx950 (batched decode steps and itts_qlinear_forward:
+// 9 rows and more on the tiles, up to 8 on the few-row product), the activation splitter and the
+// standalone dequantiser.
 //
 // The GEMM contracts M activation rows against the int8 (or int4) codes on the MFMA
 // units (v_mfma_f32_32x32x16_f16).  Codes are exact in fp16, so the matrix cores see the

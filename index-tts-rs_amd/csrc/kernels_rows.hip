@@ -624,7 +624,8 @@ __global__ __launch_bounds__(C::NT, C::NT <= 256 ? 2 : 1) void rows_mm_kernel(Ro
     }
   } else {
     // the 64 columns are one head of q, k or v: the attention's fragments (q scaled by
-    // log2(e) / 8; rows past M, up to whole tiles of 64 keys, zero), and the cache rows
+    // log2(e) / 8; rows past M zero to the end of the 32-row tile that holds row M - 1, a tile
+    // after it is not written and not read), and the cache rows
     using P = AttnPlanes<KVT>;
     constexpr int NQ = P::T::N, NP = P::NP;
     const int d = a.N / 3, which = n0 / d, head = (n0 - which * d) / 64, Tt = (a.M + 63) / 64 * 2;
