@@ -155,7 +155,7 @@ bool valid_config(const itts_config &c, std::string &why) {
 // Handles
 // ------------------------------------------------------------------------------------
 
-size_t round256(size_t n) { return (n + 255) / 256 * 256; }
+static size_t round256(size_t n) { return (n + 255) / 256 * 256; }
 
 struct QLHost {
   DevBuf codes, params, bias;
